@@ -128,12 +128,21 @@ int ssla_gla_chunk_fwd_noalloc(const void *q, const void *k, const void *v,
  * Forward: K <= 64, V <= 256 per call (wider K: groups of 64 keys whose o
  * add up).  Backward: K, V <= 64 per call (wider K or V: groups of 64 keys
  * or value columns, as for the bf16 backward); dh0 is required with h0.
- * Workspace of the backward: ssla_gla_chunk_f32_bwd_workspace_size bytes
- * (every chunk's entering state; no initialisation needed); cu_seqlens
- * must be non-decreasing. */
+ * ssla_gla_chunk_f32_fwd_ws is the forward with a workspace of
+ * ssla_gla_chunk_f32_fwd_workspace_size bytes (every chunk's entering state)
+ * that runs all chunks side by side; ssla_gla_chunk_f32_fwd needs none and
+ * walks each sequence's chunks in turn, many times slower.  Workspace of the
+ * backward: ssla_gla_chunk_f32_bwd_workspace_size bytes (every chunk's
+ * entering state and leaving-state gradient).  Neither needs initialisation;
+ * cu_seqlens must be non-decreasing. */
 int ssla_gla_chunk_f32_fwd(const float *q, const float *k, const float *v, const float *g,
                            const int64_t *cu_seqlens, int n_seq, int64_t T, int H, int K, int V,
                            float scale, const float *h0, float *o, float *ht, void *stream);
+size_t ssla_gla_chunk_f32_fwd_workspace_size(int n_seq, int64_t T, int H, int K, int V);
+int ssla_gla_chunk_f32_fwd_ws(const float *q, const float *k, const float *v, const float *g,
+                              const int64_t *cu_seqlens, int n_seq, int64_t T, int H, int K, int V,
+                              float scale, const float *h0, float *o, float *ht, void *workspace,
+                              size_t workspace_bytes, void *stream);
 size_t ssla_gla_chunk_f32_bwd_workspace_size(int n_seq, int64_t T, int H);
 int ssla_gla_chunk_f32_bwd(const float *q, const float *k, const float *v, const float *g,
                            const int64_t *cu_seqlens, int n_seq, int64_t T, int H, int K, int V,

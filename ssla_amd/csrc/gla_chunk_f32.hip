@@ -19,14 +19,15 @@
 //   2^(G_i - S_I) 2^(S_I - G_j) with S_I = G at the first row of block I:
 //   q~_i = q_i 2^(G_i - S_I) per row, and the k side per (row, I) -- dk;
 // * o, the state and dh use 2^G and 2^(gamma - G) (<= 1) directly.
-// All arithmetic is fp32 on the VALU: the matrix cores' fp32 rate is only
-// twice the VALU's, and these kernels serve the fp32 (training and
-// reference-precision) path, where the bf16 kernels do not apply.
+// All products are fp32: on the matrix cores' fp32 instruction in the
+// chunk-parallel kernels, on the VALU in the serial walk.
 //
-// Forward: one workgroup per (sequence, head, 16-column V tile) walks the
-// sequence's chunks with its state tile in LDS.  Backward: one workgroup per
-// (sequence, head) (K, V <= 64) first walks forward storing each chunk's
-// entering state in the workspace, then walks back: dv = A^T dO + k_d dh,
+// ssla_gla_chunk_f32_fwd_ws and ssla_gla_chunk_f32_bwd give every chunk its own
+// workgroup (below, with their workspace); ssla_gla_chunk_f32_fwd, for callers
+// that have no workspace, walks the chunks with one workgroup per (sequence,
+// head, 16-column V tile) and its state tile in LDS.  Backward of a chunk
+// (K, V <= 64), h its entering state and dh its leaving gradient:
+// dv = A^T dO + k_d dh,
 // dq, dk from dO h^T, v dh^T and dA = (dO v^T) masked, dg = reverse cumsum
 // of dG = q dq - k dk plus the chunk-total decay's term, dh <- 2^gamma dh +
 // s (q 2^G)^T dO.  dG is formed without the terms that cancel exactly (the
@@ -212,282 +213,713 @@ __global__ __launch_bounds__(kThreads) void f32_fwd_kernel(
   }
 }
 
-// --------------------------------------------------------------- backward --
-// Workspace slot of the chunk starting at row t0 of sequence n:
-// t0 / 64 + n is distinct for every chunk of every sequence when the
-// sequences do not overlap (at most T / 64 + n_seq + 1 slots).
-__device__ __forceinline__ int64_t state_slot(int64_t t0, int n) { return t0 / kC + n; }
+// ------------------------------------------------ chunk-parallel kernels --
+// Forward and backward with every chunk its own workgroup and all products
+// on v_mfma_f32_16x16x4_f32 (fp32 products, fp32 sums):
+//   f32_states_kernel   each chunk's own contribution to the state,
+//                       L = (k 2^(gamma - G))^T v, and (backward) to the state
+//                       gradient, R = s (q 2^G)^T dO, with its decay 2^gamma
+//   f32_prefix_kernel   S <- 2^gamma S + L over the chunks of a sequence (and
+//                       dh <- 2^gamma dh + R from its end), element by element,
+//                       leaving the entering value in each chunk's slot
+//   f32_out_kernel / f32_grad_kernel   o, or dq, dk, dv, dg, of a chunk from
+//                       its entering state (and leaving gradient)
+// The walks they replace ran one workgroup per (sequence, head), 48 of them
+// on 256 CUs at 12 ragged sequences of 8,209 rows in all, H = 4, K = V = 64:
+// 14.4 ms for forward and backward against 0.159 ms here (grad 74, states 37
+// in two launches, out 31, prefix 30 us of kernels under the profiler).  What
+// bounds them now is latency: each workgroup's load, cumsum, stage and product
+// phases follow one another with one or two workgroups per CU, and the prefix
+// is a serial chain over the longest sequence's chunks.
+//
+// A 64 x 64 fp32 tile in LDS holds row r's 16-byte segment s at s ^ (r & 15).
+// MFMA operands are read from it two ways, over the same order of the
+// contraction index (step 4t + e of lane group gq: index 16t + 4gq + e):
+//   row operand   lane r of the group holds row r's 4 columns 16t + 4gq ..
+//                 (one 16-byte read for 4 steps)
+//   col operand   lane r holds column c0 + r of row 16t + 4gq + e (4-byte
+//                 reads; the four groups fall on different banks)
+// A 16 x 16 result sits in the lanes as D[4gq + x][r]: as the second operand
+// of a product that contracts over its row index it needs no exchange, so
+// the blocks of A and dA feed the next product from registers.
+//
+// Decays inside a chunk: the gates are summed within each 16-row block, and
+// the decay between rows of two blocks is put together from their own sums
+// and the totals of the blocks between.  q~_i = q_i 2^(G_i - S_I) and
+// k~_j = k_j 2^(E_J - G_j) are staged once; a block pair takes the per-key factor 2^(S_I - E_J) on one
+// operand, or 2^(G_i - E_J) / 2^(S_I - G_j) on its result, all <= 1 for J < I.
+// For J = I the factor undoes at most the block's own decay: while |G - S_I|
+// stays within 40 (a factor of 2^80 between the extremes) every intermediate
+// is a normal number for inputs above 2^-46, and the block runs on the matrix
+// cores like the others; a chunk with a stronger decay (`slow`, uniform over
+// the workgroup) adds its diagonal blocks term by term, exponentials of
+// non-positive arguments only.
 
-__global__ __launch_bounds__(kThreads) void f32_bwd_kernel(
-    const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
-    const float *__restrict__ g, const int64_t *__restrict__ cu, int n_seq, int64_t T, int H, int K, int V,
-    float scale, const float *__restrict__ h0, const float *__restrict__ dO, const float *__restrict__ dht,
-    float *__restrict__ dq, float *__restrict__ dk, float *__restrict__ dv, float *__restrict__ dg,
-    float *__restrict__ dh0, float *__restrict__ hs, int64_t n_slots) {
-  // sHQ holds the chunk's entering state h until its products are done,
-  // then q~; sAD holds A until dv is done, then dA, then dG.
-  __shared__ float sQ[kC][kP], sK[kC][kP], sKt[kC][kP], sHQ[kC][kP], sG[kC][kP];
-  __shared__ float sV[kC][kP], sDO[kC][kP], sDH[64][kP], sAD[kC][kP];
-  __shared__ ChunkRefs R;
-  __shared__ float sDgH[64];   // 2^gamma sum_c dh h per key
-  const int tid = threadIdx.x;
-  const int h = static_cast<int>(blockIdx.x % H);
-  const int n = static_cast<int>(blockIdx.x / H);
-  int64_t bos, eos;
-  seq_bounds(cu, n, T, bos, eos);
-  const int64_t sb = (static_cast<int64_t>(n) * H + h) * K * V;
-  const int ri = tid >> 2, q4 = tid & 3, c16 = 16 * q4;   // row (or key), and its 16 columns
-  const int64_t nchunks = (eos - bos + kC - 1) / kC;
-  auto slot_ptr = [&](int64_t t0) { return hs + (min(state_slot(t0, n), n_slots - 1) * H + h) * 64 * 64; };
+constexpr float kDiagRange = 40.f;
 
-  // ---- forward: the state entering every chunk -> workspace ----------------
-  float S[16];
+__device__ __forceinline__ int tix(int r, int c) { return r * 64 + ((((c >> 2) ^ (r & 15)) << 2) | (c & 3)); }
+__device__ __forceinline__ f32x4 row4(const float *t, int r, int c) {
+  return *reinterpret_cast<const f32x4 *>(t + tix(r, c));
+}
+__device__ __forceinline__ void put4(float *t, int r, int c, const f32x4 &x) {
+  *reinterpret_cast<f32x4 *>(t + tix(r, c)) = x;
+}
+__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4 &c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 ref4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+
+// 4 columns from c of a row of C floats (zero where !ok or past C); VEC: C is
+// a multiple of 4 and the rows are 16-byte aligned.
+template <bool VEC>
+__device__ __forceinline__ f32x4 load4(const float *row, bool ok, int c, int C) {
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+  if (!ok) return x;
+  if (VEC) {
+    if (c < C) x = *reinterpret_cast<const f32x4 *>(row + c);
+  } else {
 #pragma unroll
-  for (int m = 0; m < 16; ++m) {
-    const int c = c16 + m;
-    S[m] = (h0 && ri < K && c < V) ? h0[sb + static_cast<int64_t>(ri) * V + c] : 0.f;
+    for (int m = 0; m < 4; ++m)
+      if (c + m < C) x[m] = row[c + m];
   }
-  for (int64_t ch = 0; ch < nchunks; ++ch) {
-    const int64_t t0 = bos + ch * kC;
-    const int nc = static_cast<int>(min(static_cast<int64_t>(kC), eos - t0));
-    float *slot = slot_ptr(t0);
+  return x;
+}
+template <bool VEC>
+__device__ __forceinline__ void store4(float *row, int c, int C, const f32x4 &x) {
+  if (VEC) {
+    if (c < C) *reinterpret_cast<f32x4 *>(row + c) = x;
+  } else {
 #pragma unroll
-    for (int m = 0; m < 16; ++m) slot[ri * 64 + c16 + m] = S[m];
-    __syncthreads();
-    for (int e = tid; e < kC * 64; e += kThreads) {
-      const int r = e >> 6, c = e & 63;
-      const int64_t row = (t0 + r) * H + h;
-      sK[r][c] = (r < nc && c < K) ? k[row * K + c] : 0.f;
-      sG[r][c] = (r < nc && c < K) ? g[row * K + c] * kLog2e : 0.f;
-      sV[r][c] = (r < nc && c < V) ? v[row * V + c] : 0.f;
-    }
-    __syncthreads();
-    chunk_cumsum(sG, R);
-    __syncthreads();
-    chunk_tilde(nullptr, sK, sG, R, sKt, nullptr);
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) S[m] *= R.DL[ri];
-    for (int j = 0; j < kC; ++j) {
-      const float kd = sKt[j][ri] * R.PE[j >> 4][ri];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) S[m] = fmaf(kd, sV[j][c16 + m], S[m]);
-    }
-  }
-  // ---- backward ----------------------------------------------------------------
-#pragma unroll
-  for (int m = 0; m < 16; ++m) {
-    const int c = c16 + m;
-    sDH[ri][c] = (dht && ri < K && c < V) ? dht[sb + static_cast<int64_t>(ri) * V + c] : 0.f;
-  }
-  for (int64_t ch = nchunks - 1; ch >= 0; --ch) {
-    const int64_t t0 = bos + ch * kC;
-    const int nc = static_cast<int>(min(static_cast<int64_t>(kC), eos - t0));
-    const float *slot = slot_ptr(t0);
-    __syncthreads();   // the previous (later) chunk is done with the tiles
-    for (int e = tid; e < kC * 64; e += kThreads) {
-      const int r = e >> 6, c = e & 63;
-      const int64_t row = (t0 + r) * H + h;
-      const bool okk = r < nc && c < K, okv = r < nc && c < V;
-      sQ[r][c] = okk ? q[row * K + c] : 0.f;
-      sK[r][c] = okk ? k[row * K + c] : 0.f;
-      sG[r][c] = okk ? g[row * K + c] * kLog2e : 0.f;
-      sV[r][c] = okv ? v[row * V + c] : 0.f;
-      sDO[r][c] = okv ? dO[row * V + c] : 0.f;
-      sHQ[r][c] = slot[e];   // the state entering this chunk (keys x values)
-    }
-    __syncthreads();
-    chunk_cumsum(sG, R);
-    __syncthreads();
-    chunk_tilde(nullptr, sK, sG, R, sKt, nullptr);
-    __syncthreads();
-    float da[16];   // dA_i,16J.. of thread (row ri, block q4), kept until A is read
-    {
-      float a[16];
-      a_row16(sQ, sK, sKt, sG, R, K, ri, q4, scale, a);
-#pragma unroll
-      for (int jj = 0; jj < 16; ++jj) da[jj] = 0.f;
-      if (q4 <= (ri >> 4)) {
-        for (int c = 0; c < V; ++c) {
-          const float d = sDO[ri][c];
-#pragma unroll
-          for (int jj = 0; jj < 16; ++jj) da[jj] = fmaf(d, sV[16 * q4 + jj][c], da[jj]);
-        }
-      }
-#pragma unroll
-      for (int jj = 0; jj < 16; ++jj) {
-        sAD[ri][16 * q4 + jj] = a[jj];
-        if (16 * q4 + jj > ri) da[jj] = 0.f;
-      }
-    }
-    __syncthreads();
-    {   // dv_j = sum_{i >= j} A_ij dO_i + k_d,j dh: thread (row ri, 16 columns)
-      float acc[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) acc[m] = 0.f;
-      for (int i = ri; i < kC; ++i) {
-        const float aij = sAD[i][ri];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) acc[m] = fmaf(aij, sDO[i][c16 + m], acc[m]);
-      }
-      const int J = ri >> 4;
-      for (int kk = 0; kk < K; ++kk) {
-        const float kd = sKt[ri][kk] * R.PE[J][kk];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) acc[m] = fmaf(kd, sDH[kk][c16 + m], acc[m]);
-      }
-      if (ri < nc) {
-#pragma unroll
-        for (int m = 0; m < 16; ++m)
-          if (c16 + m < V) dv[((t0 + ri) * H + h) * V + c16 + m] = acc[m];
-      }
-    }
-    __syncthreads();   // A is read: dA takes its place
-#pragma unroll
-    for (int jj = 0; jj < 16; ++jj) sAD[ri][16 * q4 + jj] = da[jj];
-    __syncthreads();
-    // dq and dk of row ri, keys c16 .. c16 + 15 (the same thread holds both, so
-    // dG = q dq - k dk needs no exchange)
-    float qdq[16], kdk[16], tdk[16];
-    {
-      const int I = ri >> 4;
-      float P[16], Ro[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) P[m] = Ro[m] = 0.f;
-      for (int c = 0; c < V; ++c) {   // P = dO_i . h_k
-        const float d = sDO[ri][c];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) P[m] = fmaf(d, sHQ[c16 + m][c], P[m]);
-      }
-      for (int J = 0; J < I; ++J) {   // blocks J < I: 2^(G_i - E_J) sum_j dA_ij k~_j
-        float r[16];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) r[m] = 0.f;
-        for (int j = 16 * J; j < 16 * J + 16; ++j) {
-          const float d = sAD[ri][j];
-#pragma unroll
-          for (int m = 0; m < 16; ++m) r[m] = fmaf(d, sKt[j][c16 + m], r[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < 16; ++m) Ro[m] = fmaf(ex2c(sG[ri][c16 + m] - R.E[J][c16 + m]), r[m], Ro[m]);
-      }
-      for (int j = 16 * I; j < ri; ++j) {   // the diagonal block, term by term
-        const float d = sAD[ri][j];
-#pragma unroll
-        for (int m = 0; m < 16; ++m)
-          Ro[m] = fmaf(d * sK[j][c16 + m], ex2c(sG[ri][c16 + m] - sG[j][c16 + m]), Ro[m]);
-      }
-      // j = i adds s dA_ii k_i to dq and s dA_ii q_i to dk: equal terms of
-      // q dq and k dk that cancel in dG, so dG is formed without them
-      const float dii = sAD[ri][ri];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        const int kk = c16 + m;
-        const float part = fmaf(ex2c(sG[ri][kk]), P[m], Ro[m]);
-        qdq[m] = sQ[ri][kk] * (scale * part);
-        const float dqv = scale * fmaf(dii, sK[ri][kk], part);
-        if (ri < nc && kk < K) dq[((t0 + ri) * H + h) * K + kk] = dqv;
-      }
-    }
-    if (tid < 64) {   // the state products are done with h: 2^gamma sum_c dh h
-      float s = 0.f;
-      for (int c = 0; c < V; ++c) s = fmaf(sDH[tid][c], sHQ[tid][c], s);
-      sDgH[tid] = s * R.DL[tid];
-    }
-    __syncthreads();
-    chunk_tilde(sQ, sK, sG, R, sKt, sHQ);   // q~ into sHQ (k~ again, unchanged)
-    __syncthreads();
-    {
-      const int J = ri >> 4;
-      float P[16], Ro[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) P[m] = Ro[m] = 0.f;
-      for (int c = 0; c < V; ++c) {   // P' = v_j . dh_k
-        const float d = sV[ri][c];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) P[m] = fmaf(d, sDH[c16 + m][c], P[m]);
-      }
-      for (int I = J + 1; I < 4; ++I) {   // blocks I > J: 2^(S_I - G_j) sum_i dA_ij q~_i
-        float r[16];
-#pragma unroll
-        for (int m = 0; m < 16; ++m) r[m] = 0.f;
-        for (int i = 16 * I; i < 16 * I + 16; ++i) {
-          const float d = sAD[i][ri];
-#pragma unroll
-          for (int m = 0; m < 16; ++m) r[m] = fmaf(d, sHQ[i][c16 + m], r[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < 16; ++m) Ro[m] = fmaf(ex2c(R.S[I][c16 + m] - sG[ri][c16 + m]), r[m], Ro[m]);
-      }
-      for (int i = ri + 1; i < 16 * J + 16; ++i) {   // the diagonal block, term by term
-        const float d = sAD[i][ri];
-#pragma unroll
-        for (int m = 0; m < 16; ++m)
-          Ro[m] = fmaf(d * sQ[i][c16 + m], ex2c(sG[i][c16 + m] - sG[ri][c16 + m]), Ro[m]);
-      }
-      const float dii = sAD[ri][ri];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        const int kk = c16 + m;
-        const float kd = sKt[ri][kk] * R.PE[J][kk];                                      // k 2^(gamma - G)
-        const float dkv = fmaf(ex2c(R.GAM[kk] - sG[ri][kk]), P[m], scale * fmaf(dii, sQ[ri][kk], Ro[m]));
-        // the state term k 2^(gamma - G) P' enters dG here and dgamma with the
-        // opposite sign: dG keeps the intra-chunk part, dg adds the state term
-        // of the rows before t as a forward prefix
-        kdk[m] = sK[ri][kk] * (scale * Ro[m]);
-        tdk[m] = kd * P[m];
-        if (ri < nc && kk < K) dk[((t0 + ri) * H + h) * K + kk] = dkv;
-      }
-    }
-    __syncthreads();   // dA and k~ are no longer read
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      sAD[ri][c16 + m] = qdq[m] - kdk[m];   // dG
-      sKt[ri][c16 + m] = tdk[m];
-    }
-    __syncthreads();
-    if (tid < 64) {
-      // dg_t = dgamma + sum_{r >= t} (q dq - k dk)_r with dgamma = 2^gamma
-      // sum dh h + sum_j tdk_j; the tdk_r of rows r >= t cancel, so
-      // dg_t = 2^gamma sum dh h + sum_{j < t} tdk_j + sum_{r >= t} dG_r
-      const int kk = tid;
-      float pre = 0.f;
-      for (int j = 0; j < nc; ++j) {   // exclusive prefix of tdk, in place
-        const float t = sKt[j][kk];
-        sKt[j][kk] = pre;
-        pre += t;
-      }
-      float acc = sDgH[kk];
-      for (int r = nc - 1; r >= 0; --r) {
-        acc += sAD[r][kk];
-        if (kk < K) dg[((t0 + r) * H + h) * K + kk] = acc + sKt[r][kk];
-      }
-    }
-    {   // dh <- 2^gamma dh + s sum_i (q 2^G)_i^T dO_i: thread (key ri, 16 columns);
-        // only this thread reads or writes its dh entries from here on
-      float acc[16];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) acc[m] = sDH[ri][c16 + m] * R.DL[ri];
-      for (int i = 0; i < kC; ++i) {
-        const float qg = scale * sQ[i][ri] * ex2c(sG[i][ri]);
-#pragma unroll
-        for (int m = 0; m < 16; ++m) acc[m] = fmaf(qg, sDO[i][c16 + m], acc[m]);
-      }
-#pragma unroll
-      for (int m = 0; m < 16; ++m) sDH[ri][c16 + m] = acc[m];
-    }
-  }
-  __syncthreads();
-  if (dh0) {
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int c = c16 + m;
-      if (ri < K && c < V) dh0[sb + static_cast<int64_t>(ri) * V + c] = sDH[ri][c];
-    }
+    for (int m = 0; m < 4; ++m)
+      if (c + m < C) row[c + m] = x[m];
   }
 }
 
-inline int64_t f32_bwd_slots(int n_seq, int64_t T) { return T / kC + n_seq + 1; }
+// Workspace slot of chunk c of sequence n: bos / 64 + n + c, distinct for
+// every chunk of non-overlapping sequences (at most T / 64 + n_seq + 1).
+struct ChunkAt {
+  int n, nc, c;     // sequence, rows, chunk of the sequence
+  int64_t t0;       // first row
+  bool first, last; // of its sequence
+};
+
+// The chunk of a slot (false: none).  Every wavefront searches the sequence
+// starts 64 probes per round trip.
+__device__ __forceinline__ bool chunk_of_slot(const int64_t *cu, int n_seq, int64_t T, int64_t slot, ChunkAt &at) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, hi = n_seq;
+  while (hi - lo > 1) {
+    const int step = (hi - lo + 63) >> 6;
+    const int64_t i = lo + static_cast<int64_t>(lane) * step;
+    const bool in = i < hi && min(max(cu[min(i, static_cast<int64_t>(hi - 1))], (int64_t)0), T) / kC + i <= slot;
+    const int cnt = __popcll(__ballot(in));
+    if (cnt == 0) return false;
+    lo += (cnt - 1) * step;
+    hi = min(hi, lo + step);
+  }
+  int64_t bos, eos;
+  seq_bounds(cu, lo, T, bos, eos);
+  const int64_t c = slot - (bos / kC + lo);
+  const int64_t t0 = bos + c * kC;
+  if (c < 0 || t0 >= eos) return false;
+  at.n = lo;
+  at.c = static_cast<int>(c);
+  at.t0 = t0;
+  at.nc = static_cast<int>(min(static_cast<int64_t>(kC), eos - t0));
+  at.first = c == 0;
+  at.last = t0 + kC >= eos;
+  return true;
+}
+
+// Cumsum of the gates (log2-scaled, in place) local to each 16-row block:
+// thread (quad, group) holds rows RPT group .. of keys 4 quad ..; a wavefront
+// holds 4 RPT rows.  Block-local sums keep the differences between rows exact
+// to the block's own decay (a chunk-wide sum loses two bits and more of them),
+// and every partial sum is formed in row order, so a row and the rows without
+// decay after it hold the same value.  wtot: each wavefront's total (a block's
+// when RPT is 4).  One barrier.
+template <int RPT>
+__device__ __forceinline__ void cumsum_rows(f32x4 (&g)[RPT], float (*wtot)[64]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, gq = lane >> 4, quad = lane & 15;
+#pragma unroll
+  for (int m = 0; m < RPT; ++m) {
+    g[m] *= kLog2e;
+    if (m) g[m] += g[m - 1];
+  }
+  f32x4 t[3];   // totals of groups 0 .. 2
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const float own = g[RPT - 1][x];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) t[i][x] = __shfl(own, 16 * i + quad);
+  }
+  if (gq == 3) *reinterpret_cast<f32x4 *>(&wtot[w][4 * quad]) = ((t[0] + t[1]) + t[2]) + g[RPT - 1];
+  __syncthreads();
+  f32x4 off = {0.f, 0.f, 0.f, 0.f};
+  if (RPT == 2 && (w & 1)) off = ref4(&wtot[w - 1][4 * quad]);   // the block's first eight rows
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (i < gq) off += t[i];
+#pragma unroll
+  for (int m = 0; m < RPT; ++m) g[m] += off;
+}
+
+// Decay of the whole blocks strictly between a and b at 4 keys: sE[B] = block
+// B's total (G at its last row).
+__device__ __forceinline__ f32x4 between(const float (*sE)[64], int a, int b, int col) {
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+  for (int B = a + 1; B < b; ++B) x += ref4(&sE[B][col]);
+  return x;
+}
+
+struct F32Args {
+  const float *q, *k, *v, *g, *dO, *h0, *dht;
+  const int64_t *cu;
+  float *o, *ht, *dq, *dk, *dv, *dg, *dh0;
+  float *sh, *sd;       // per (slot, head, value group): entering state / leaving gradient, [64][64]
+  float *eh, *ed;       // per (slot, head): 2^gamma of the keys, as each of them uses it
+  int64_t T, n_slots;
+  int n_seq, H, K, V, nvg;
+  float scale;
+};
+
+// L or R of one chunk (blockIdx.y: 0 = L, 1 = R); one workgroup per (slot,
+// head, value group), wavefront w the keys 16w ..
+template <bool VEC>
+__global__ __launch_bounds__(256) void f32_states_kernel(F32Args a, int need_last, int need_first) {
+  __shared__ __attribute__((aligned(16))) float sX[64 * 64], sY[64 * 64], wtot[4][64];
+  const bool rev = blockIdx.y;
+  const int vg = static_cast<int>(blockIdx.x % a.nvg);
+  const int h = static_cast<int>(blockIdx.x / a.nvg % a.H);
+  const int64_t slot = blockIdx.x / a.nvg / a.H;
+  ChunkAt at;
+  if (!chunk_of_slot(a.cu, a.n_seq, a.T, slot, at)) return;
+  if (rev ? (at.first && !need_first) : (at.last && !need_last)) return;   // nothing follows it
+  const int tid = threadIdx.x, quad = tid & 15, r0 = (tid >> 4) * 4, K = a.K, V = a.V, v0 = 64 * vg;
+  const float *X = rev ? a.q : a.k, *Y = rev ? a.dO : a.v;
+  f32x4 x[4], y[4], g[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const bool ok = r0 + m < at.nc;
+    const int64_t row = (at.t0 + r0 + m) * a.H + h;
+    g[m] = load4<VEC>(a.g + row * K, ok, 4 * quad, K);
+    x[m] = load4<VEC>(X + row * K, ok, 4 * quad, K);
+    y[m] = load4<VEC>(Y + row * V, ok, v0 + 4 * quad, V);
+  }
+  cumsum_rows<4>(g, wtot);
+  const int lane = tid & 63, w = tid >> 6, r = lane & 15, gq = lane >> 4;
+  const f32x4 tot = ref4(&wtot[w][4 * quad]);
+  const f32x4 far = rev ? between(wtot, -1, w, 4 * quad) : between(wtot, w, 4, 4 * quad);   // the other blocks' share
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      x[m][e] *= rev ? a.scale * ex2c(g[m][e] + far[e]) : ex2c((tot[e] - g[m][e]) + far[e]);
+    put4(sX, r0 + m, 4 * quad, x[m]);
+    put4(sY, r0 + m, 4 * quad, y[m]);
+  }
+  const int64_t sl = slot * a.H + h;
+  if (vg == 0 && tid < 64)
+    (rev ? a.ed : a.eh)[sl * 64 + tid] = ex2c(((wtot[0][tid] + wtot[1][tid]) + wtot[2][tid]) + wtot[3][tid]);
+  __syncthreads();
+  f32x4 acc[4] = {};
+#pragma unroll 4
+  for (int s = 0; s < 16; ++s) {
+    const int row = 16 * (s >> 2) + 4 * gq + (s & 3);
+    const float xv = sX[tix(row, 16 * w + r)];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = mfma4(sY[tix(row, 16 * c + r)], xv, acc[c]);
+  }
+  float *out = (rev ? a.sd : a.sh) + (sl * a.nvg + vg) * 4096 + (16 * w + r) * 64 + 4 * gq;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4 *>(out + 16 * c) = acc[c];
+}
+
+// Entering states (blockIdx.y 0) or leaving state gradients (1) from the
+// chunks' own contributions, in place; 4 values per thread, kPre chunks per
+// round trip.  Four workgroups per (sequence, head, value group).
+constexpr int kPre = 8;
+__global__ __launch_bounds__(256) void f32_prefix_kernel(F32Args a) {
+  const bool rev = blockIdx.y;
+  const int part = static_cast<int>(blockIdx.x & 3);
+  const int vg = static_cast<int>((blockIdx.x >> 2) % a.nvg);
+  const int h = static_cast<int>((blockIdx.x >> 2) / a.nvg % a.H);
+  const int n = static_cast<int>((blockIdx.x >> 2) / a.nvg / a.H);
+  int64_t bos, eos;
+  seq_bounds(a.cu, n, a.T, bos, eos);
+  const int64_t nch = (eos - bos + kC - 1) / kC;
+  const int e = part * 1024 + 4 * static_cast<int>(threadIdx.x), key = e >> 6, c = 64 * vg + (e & 63);
+  const int64_t sb = ((static_cast<int64_t>(n) * a.H + h) * a.K + key) * a.V + c;
+  const float *init = rev ? a.dht : a.h0;
+  float *fin = rev ? a.dh0 : a.ht;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (init && key < a.K) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      if (c + m < a.V) S[m] = init[sb + m];
+  }
+  const int64_t s0 = bos / kC + n;
+  float *st = rev ? a.sd : a.sh;
+  const float *dec = rev ? a.ed : a.eh;
+  for (int64_t i0 = 0; i0 < nch; i0 += kPre) {
+    f32x4 L[kPre];
+    float d[kPre];
+    float *p[kPre];
+#pragma unroll
+    for (int u = 0; u < kPre; ++u) {
+      const int64_t i = min(i0 + u, nch - 1);
+      const int64_t sl = min(s0 + (rev ? nch - 1 - i : i), a.n_slots - 1) * a.H + h;
+      p[u] = st + (sl * a.nvg + vg) * 4096 + e;
+      L[u] = *reinterpret_cast<const f32x4 *>(p[u]);
+      d[u] = dec[sl * 64 + key];
+    }
+#pragma unroll
+    for (int u = 0; u < kPre; ++u) {
+      if (i0 + u < nch) {
+        *reinterpret_cast<f32x4 *>(p[u]) = S;
+        S = d[u] * S + L[u];
+      }
+    }
+  }
+  if (fin && key < a.K) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      if (c + m < a.V) fin[sb + m] = S[m];
+  }
+}
+
+// q~ / k~ of the thread's rows into their tiles; sets *slow where a key's
+// decay over a 16-row block leaves the range of the matrix-core diagonal.
+template <int RPT>
+__device__ __forceinline__ void stage_tilde(const f32x4 (&q)[RPT], const f32x4 (&k)[RPT], const f32x4 (&g)[RPT],
+                                            const float (*sS)[64], const float (*sE)[64], int r0, int quad, float *tq,
+                                            float *tk, int *slow) {
+  const int B = r0 >> 4;
+  const f32x4 S = ref4(&sS[B][4 * quad]), E = ref4(&sE[B][4 * quad]);
+  bool out = false;
+#pragma unroll
+  for (int m = 0; m < RPT; ++m) {
+    f32x4 a, b;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = g[m][e] - S[e];
+      out |= !(fabsf(d) <= kDiagRange);
+      a[e] = q[m][e] * ex2c(d);
+      b[e] = k[m][e] * ex2c(E[e] - g[m][e]);
+    }
+    put4(tq, r0 + m, 4 * quad, a);
+    put4(tk, r0 + m, 4 * quad, b);
+  }
+  if (out) *slow = 1;
+}
+
+// The block references S (first row) and E (last row) of the thread's rows.
+template <int RPT>
+__device__ __forceinline__ void stage_refs(const f32x4 (&g)[RPT], int r0, int quad, float (*sS)[64], float (*sE)[64]) {
+  if ((r0 & 15) == 0) *reinterpret_cast<f32x4 *>(&sS[r0 >> 4][4 * quad]) = g[0];
+  if ((r0 & 15) == 16 - RPT) *reinterpret_cast<f32x4 *>(&sE[r0 >> 4][4 * quad]) = g[RPT - 1];
+}
+
+// 2^x of 4 keys.
+__device__ __forceinline__ f32x4 exp4(const f32x4 &x) {
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = ex2c(x[e]);
+  return y;
+}
+
+// One block pair's term-by-term sums sum_k q_ik k_jk 2^(G_i - G_j) as
+// D[4gq + x][r] with row index `row` of q (i) and column index of k (j) when
+// QROWS, or j and i when not; terms j > i are zero.
+template <bool QROWS>
+__device__ __forceinline__ f32x4 diag_terms(const float *tq, const float *tk, const float *tg, int B, int gq, int r,
+                                            int K) {
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int x = 0; x < 4; ++x) {
+    const int i = 16 * B + (QROWS ? 4 * gq + x : r), j = 16 * B + (QROWS ? r : 4 * gq + x);
+    float acc = 0.f;
+    if (j <= i) {
+#pragma unroll 1
+      for (int kk = 0; kk < K; kk += 4) {
+        const f32x4 qv = row4(tq, i, kk), kv = row4(tk, j, kk), gi = row4(tg, i, kk), gj = row4(tg, j, kk);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = fmaf(qv[e] * kv[e], ex2c(gi[e] - gj[e]), acc);
+      }
+    }
+    if (x == 0) s[0] = acc;
+    if (x == 1) s[1] = acc;
+    if (x == 2) s[2] = acc;
+    if (x == 3) s[3] = acc;
+  }
+  return s;
+}
+
+// o of one chunk: one workgroup per (slot, head, value group), wavefront I
+// the rows 16I ..; 66 KB of LDS, two workgroups per CU.
+template <bool VEC>
+__global__ __launch_bounds__(256, 2) void f32_out_kernel(F32Args a) {
+  __shared__ __attribute__((aligned(16))) float tQ[4096], tK[4096], tV[4096], tS[4096];
+  __shared__ __attribute__((aligned(16))) float wtot[4][64], sS[4][64], sE[4][64];
+  __shared__ int slow;
+  const int vg = static_cast<int>(blockIdx.x % a.nvg);
+  const int h = static_cast<int>(blockIdx.x / a.nvg % a.H);
+  const int64_t slot = blockIdx.x / a.nvg / a.H;
+  ChunkAt at;
+  if (!chunk_of_slot(a.cu, a.n_seq, a.T, slot, at)) return;
+  const int tid = threadIdx.x, quad = tid & 15, r0 = (tid >> 4) * 4, K = a.K, V = a.V, v0 = 64 * vg;
+  const float *st = a.sh + ((slot * a.H + h) * a.nvg + vg) * 4096;
+  f32x4 q[4], k[4], g[4], v[4], s[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const bool ok = r0 + m < at.nc;
+    const int64_t row = (at.t0 + r0 + m) * a.H + h;
+    g[m] = load4<VEC>(a.g + row * K, ok, 4 * quad, K);
+    q[m] = load4<VEC>(a.q + row * K, ok, 4 * quad, K);
+    k[m] = load4<VEC>(a.k + row * K, ok, 4 * quad, K);
+    v[m] = load4<VEC>(a.v + row * V, ok, v0 + 4 * quad, V);
+    s[m] = ref4(st + (r0 + m) * 64 + 4 * quad);
+  }
+  if (tid == 0) slow = 0;
+  cumsum_rows<4>(g, wtot);
+  stage_refs<4>(g, r0, quad, sS, sE);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    put4(tV, r0 + m, 4 * quad, v[m]);
+    put4(tS, r0 + m, 4 * quad, s[m]);
+  }
+  __syncthreads();
+  stage_tilde<4>(q, k, g, sS, sE, r0, quad, tQ, tK, &slow);
+  __syncthreads();
+  const int lane = tid & 63, I = tid >> 6, r = lane & 15, gq = lane >> 4;
+  const bool diag = !slow;
+  f32x4 acc[4] = {};
+  f32x4 qr[4];   // q~ of row 16 I + r, keys 16 t + 4 gq ..
+#pragma unroll
+  for (int t = 0; t < 4; ++t) qr[t] = row4(tQ, 16 * I + r, 16 * t + 4 * gq);
+  // q 2^G against the entering state
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const f32x4 S = ref4(&sS[I][16 * t + 4 * gq]) + between(sE, -1, I, 16 * t + 4 * gq);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float qg = qr[t][e] * ex2c(S[e]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = mfma4(tS[tix(16 * t + 4 * gq + e, 16 * c + r)], qg, acc[c]);
+    }
+  }
+  for (int J = 0; J <= I; ++J) {
+    if (J == I && !diag) break;
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};   // A[i = r][j = 4 gq + x]
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int kc = 16 * t + 4 * gq;
+      const f32x4 S = ref4(&sS[I][kc]);
+      const f32x4 f = qr[t] * exp4(J == I ? S - ref4(&sE[I][kc]) : S + between(sE, J, I, kc));   // 2^(S_I - E_J)
+      const f32x4 kr = row4(tK, 16 * J + r, 16 * t + 4 * gq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p = mfma4(kr[e], f[e], p);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const float pv = (J < I || 4 * gq + x <= r) ? p[x] : 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = mfma4(tV[tix(16 * J + 4 * gq + x, 16 * c + r)], pv, acc[c]);
+    }
+  }
+  if (!diag) {   // the diagonal blocks term by term, from raw q, k and G (in the state's tile)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const bool ok = r0 + m < at.nc;
+      const int64_t row = (at.t0 + r0 + m) * a.H + h;
+      q[m] = load4<VEC>(a.q + row * K, ok, 4 * quad, K);
+      k[m] = load4<VEC>(a.k + row * K, ok, 4 * quad, K);
+      g[m] = load4<VEC>(a.g + row * K, ok, 4 * quad, K);
+    }
+    cumsum_rows<4>(g, wtot);   // its barrier also ends the products above
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      put4(tQ, r0 + m, 4 * quad, q[m]);
+      put4(tK, r0 + m, 4 * quad, k[m]);
+      put4(tS, r0 + m, 4 * quad, g[m]);
+    }
+    __syncthreads();
+    const f32x4 p = diag_terms<false>(tQ, tK, tS, I, gq, r, K);
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = mfma4(tV[tix(16 * I + 4 * gq + x, 16 * c + r)], p[x], acc[c]);
+  }
+  if (16 * I + r < at.nc) {
+    float *o = a.o + ((at.t0 + 16 * I + r) * a.H + h) * V;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) store4<VEC>(o, v0 + 16 * c + 4 * gq, V, acc[c] * a.scale);
+  }
+}
+
+// Reverse inclusive scan over the 16 lanes of each DPP row.
+template <int N>
+__device__ __forceinline__ float row_shl(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+      0, __builtin_bit_cast(int, x), 0x100 + N, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_suffix_scan(float x) {
+  x += row_shl<1>(x);
+  x += row_shl<2>(x);
+  x += row_shl<4>(x);
+  x += row_shl<8>(x);
+  return x;
+}
+
+// dq, dk, dv, dg of one chunk: one workgroup of 8 wavefronts per (slot,
+// head); wavefront (I, P) the rows 16 I .. and the key / value tiles 2P,
+// 2P + 1.  Seven tiles: 128 KB of LDS, one workgroup per CU.  Results are
+// formed transposed (D[key][row]) so that a lane holds 4 consecutive keys of
+// one row, and the scans of dg over rows run across 16 lanes.
+constexpr int kGradThreads = 512;
+struct GradLds {
+  float tQ[4096], tK[4096], tV[4096], tO[4096], tH[4096], tD[4096], tG[4096];
+  float sDA[4][2][16][17];          // dA of the diagonal blocks (term by term), one copy per wavefront
+  float wtot[8][64], sS[4][64], sE[4][64], sDgH[64], totT[4][64], totG[4][64];
+  int slow;
+};
+template <bool VEC>
+__global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
+  __shared__ __attribute__((aligned(16))) GradLds L;
+  const int h = static_cast<int>(blockIdx.x % a.H);
+  const int64_t slot = blockIdx.x / a.H;
+  ChunkAt at;
+  if (!chunk_of_slot(a.cu, a.n_seq, a.T, slot, at)) return;
+  const int tid = threadIdx.x, quad = tid & 15, r0 = (tid >> 4) * 2, K = a.K, V = a.V;
+  const float *sh = a.sh + (slot * a.H + h) * 4096, *sd = a.sd + (slot * a.H + h) * 4096;
+  {
+    f32x4 q[2], k[2], g[2], v[2], d[2], hs[2], dh[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const bool ok = r0 + m < at.nc;
+      const int64_t row = (at.t0 + r0 + m) * a.H + h;
+      g[m] = load4<VEC>(a.g + row * K, ok, 4 * quad, K);
+      q[m] = load4<VEC>(a.q + row * K, ok, 4 * quad, K);
+      k[m] = load4<VEC>(a.k + row * K, ok, 4 * quad, K);
+      v[m] = load4<VEC>(a.v + row * V, ok, 4 * quad, V);
+      d[m] = load4<VEC>(a.dO + row * V, ok, 4 * quad, V);
+      hs[m] = ref4(sh + (r0 + m) * 64 + 4 * quad);
+      dh[m] = ref4(sd + (r0 + m) * 64 + 4 * quad);
+    }
+    if (tid == 0) L.slow = 0;
+    cumsum_rows<2>(g, L.wtot);
+    stage_refs<2>(g, r0, quad, L.sS, L.sE);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      put4(L.tV, r0 + m, 4 * quad, v[m]);
+      put4(L.tO, r0 + m, 4 * quad, d[m]);
+      put4(L.tH, r0 + m, 4 * quad, hs[m]);
+      put4(L.tD, r0 + m, 4 * quad, dh[m]);
+      put4(L.tG, r0 + m, 4 * quad, g[m]);
+      // sum over the values of dh h, per key (row of the state)
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = fmaf(hs[m][e], dh[m][e], s);
+      s = row_inclusive_scan(s);
+      if (quad == 15) L.sDgH[r0 + m] = s;
+    }
+    __syncthreads();
+    stage_tilde<2>(q, k, g, L.sS, L.sE, r0, quad, L.tQ, L.tK, &L.slow);
+  }
+  const int lane = tid & 63, w = tid >> 6, I = w >> 1, P = w & 1, r = lane & 15, gq = lane >> 4;
+  const int i0 = 16 * I + r;                       // this lane's row
+  const bool in = i0 < at.nc;
+  const int64_t grow = (at.t0 + i0) * a.H + h;
+  f32x4 qv[2], kv[2];                              // raw q, k of the row at this lane's keys
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    qv[c] = load4<VEC>(a.q + grow * K, in, 32 * P + 16 * c + 4 * gq, K);
+    kv[c] = load4<VEC>(a.k + grow * K, in, 32 * P + 16 * c + 4 * gq, K);
+  }
+  __syncthreads();
+  const bool diag = !L.slow;
+  f32x4 Gr[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) Gr[c] = row4(L.tG, i0, 32 * P + 16 * c + 4 * gq);
+  f32x4 dor[4], vr[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    dor[t] = row4(L.tO, i0, 16 * t + 4 * gq);
+    vr[t] = row4(L.tV, i0, 16 * t + 4 * gq);
+  }
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 pq[2] = {zero, zero}, pk[2] = {zero, zero}, ov[2] = {zero, zero};   // dO h^T, v dh^T, k_d dh
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const f32x4 kd = row4(L.tK, i0, 16 * t + 4 * gq) * exp4(between(L.sE, I, 4, 16 * t + 4 * gq));
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int c0 = 32 * P + 16 * c;
+      const f32x4 hr = row4(L.tH, c0 + r, 16 * t + 4 * gq), dr = row4(L.tD, c0 + r, 16 * t + 4 * gq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        pq[c] = mfma4(hr[e], dor[t][e], pq[c]);
+        pk[c] = mfma4(dr[e], vr[t][e], pk[c]);
+        ov[c] = mfma4(L.tD[tix(16 * t + 4 * gq + e, c0 + r)], kd[e], ov[c]);
+      }
+    }
+  }
+  float dii = 0.f;                                    // dA_ii of this lane's row
+  auto own_diag = [&](const f32x4 &da) {              // D[r][r] sits in lane 16 (r / 4) + r, element r % 4
+    const float x = (r & 2) ? ((r & 1) ? da[3] : da[2]) : ((r & 1) ? da[1] : da[0]);
+    return __shfl(x, 16 * (r >> 2) + r);
+  };
+  f32x4 rq[2] = {zero, zero}, rk[2] = {zero, zero};   // intra-chunk parts of dq, dk (no diagonal, no scale)
+  for (int J = 0; J <= I; ++J) {                      // dq: earlier rows j
+    if (J == I && !diag) break;
+    f32x4 da = zero;                                  // dA[i = r][j = 4 gq + x]
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const f32x4 vj = row4(L.tV, 16 * J + r, 16 * t + 4 * gq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) da = mfma4(vj[e], dor[t][e], da);
+    }
+    if (J == I) {
+      dii = own_diag(da);
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        if (4 * gq + x >= r) da[x] = 0.f;
+    }
+    f32x4 part[2] = {zero, zero};
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        part[c] = mfma4(L.tK[tix(16 * J + 4 * gq + x, 32 * P + 16 * c + r)], da[x], part[c]);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {   // 2^(G_i - E_J)
+      const int kc = 32 * P + 16 * c + 4 * gq;
+      rq[c] += exp4(J == I ? Gr[c] - ref4(&L.sE[I][kc]) : Gr[c] + between(L.sE, J, I, kc)) * part[c];
+    }
+  }
+  for (int B = I; B < 4; ++B) {                       // dk, dv: later rows i of block B
+    if (B == I && !diag) continue;
+    f32x4 da = zero, A = zero;                        // dA, A [i = 4 gq + x][j = r]
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const f32x4 oi = row4(L.tO, 16 * B + r, 16 * t + 4 * gq), qi = row4(L.tQ, 16 * B + r, 16 * t + 4 * gq);
+      const int kc = 16 * t + 4 * gq;
+      const f32x4 S = ref4(&L.sS[B][kc]);
+      const f32x4 kf =
+          row4(L.tK, i0, kc) * exp4(B == I ? S - ref4(&L.sE[I][kc]) : S + between(L.sE, I, B, kc));   // 2^(S_B - E_I)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        da = mfma4(oi[e], vr[t][e], da);
+        A = mfma4(qi[e], kf[e], A);
+      }
+    }
+    f32x4 part[2] = {zero, zero};
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const float d = (B > I || 4 * gq + x > r) ? da[x] : 0.f;
+      const float s = (B > I || 4 * gq + x >= r) ? A[x] * a.scale : 0.f;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int at_ = tix(16 * B + 4 * gq + x, 32 * P + 16 * c + r);
+        part[c] = mfma4(L.tQ[at_], d, part[c]);
+        ov[c] = mfma4(L.tO[at_], s, ov[c]);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {   // 2^(S_B - G_j)
+      const int kc = 32 * P + 16 * c + 4 * gq;
+      const f32x4 S = ref4(&L.sS[B][kc]);
+      rk[c] += exp4(B == I ? S - Gr[c] : (ref4(&L.sE[I][kc]) - Gr[c]) + (between(L.sE, I, B, kc) + S)) * part[c];
+    }
+  }
+  if (!diag) {
+    __syncthreads();   // q~ and k~ are read: raw q, k take their place
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const bool ok = r0 + m < at.nc;
+      const int64_t row = (at.t0 + r0 + m) * a.H + h;
+      put4(L.tQ, r0 + m, 4 * quad, load4<VEC>(a.q + row * K, ok, 4 * quad, K));
+      put4(L.tK, r0 + m, 4 * quad, load4<VEC>(a.k + row * K, ok, 4 * quad, K));
+    }
+    f32x4 da = zero;   // dA[i = 4 gq + x][j = r]
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) da = mfma4(dor[t][e], vr[t][e], da);
+    dii = own_diag(da);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) L.sDA[I][P][4 * gq + x][r] = da[x];
+    __syncthreads();
+    const f32x4 A = diag_terms<true>(L.tQ, L.tK, L.tG, I, gq, r, K);
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        ov[c] = mfma4(L.tO[tix(16 * I + 4 * gq + x, 32 * P + 16 * c + r)], A[x] * a.scale, ov[c]);
+#pragma unroll 1
+    for (int j = 0; j < 16; ++j) {
+      const int row = 16 * I + j;
+      const float dij = j < r ? L.sDA[I][P][r][j] : 0.f, dji = j > r ? L.sDA[I][P][j][r] : 0.f;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int kc = 32 * P + 16 * c + 4 * gq;
+        const f32x4 qj = row4(L.tQ, row, kc), kj = row4(L.tK, row, kc), gj = row4(L.tG, row, kc);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (j < r) rq[c][e] = fmaf(dij * kj[e], ex2c(Gr[c][e] - gj[e]), rq[c][e]);
+          if (j > r) rk[c][e] = fmaf(dji * qj[e], ex2c(gj[e] - Gr[c][e]), rk[c][e]);
+        }
+      }
+    }
+  }
+  // dv of the row: values 32 P + 16 c + 4 gq ..
+  if (in) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) store4<VEC>(a.dv + grow * V, 32 * P + 16 * c + 4 * gq, V, ov[c]);
+  }
+  // dq, dk; dG and the state term of dk with their scans over the rows
+  f32x4 pre[2], suf[2], eg[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int kc = 32 * P + 16 * c + 4 * gq;
+    // 2^G and 2^(gamma - G) of the row, from the start and to the end of the chunk
+    const f32x4 eG = exp4(Gr[c] + between(L.sE, -1, I, kc));
+    const f32x4 eE = exp4((ref4(&L.sE[I][kc]) - Gr[c]) + between(L.sE, I, 4, kc));
+    f32x4 dqv, dkv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float part = fmaf(eG[e], pq[c][e], rq[c][e]);
+      dqv[e] = a.scale * fmaf(dii, kv[c][e], part);
+      dkv[e] = fmaf(eE[e], pk[c][e], a.scale * fmaf(dii, qv[c][e], rk[c][e]));
+      const float dG = qv[c][e] * (a.scale * part) - kv[c][e] * (a.scale * rk[c][e]);
+      const float tdk = kv[c][e] * eE[e] * pk[c][e];
+      const float ps = row_inclusive_scan(tdk);
+      pre[c][e] = row_shr<1>(ps);
+      suf[c][e] = row_suffix_scan(dG);
+      eg[c][e] = ps;
+    }
+    if (r == 15) *reinterpret_cast<f32x4 *>(&L.totT[I][kc]) = eg[c];
+    if (r == 0) *reinterpret_cast<f32x4 *>(&L.totG[I][kc]) = suf[c];
+    if (in) {
+      store4<VEC>(a.dq + grow * K, kc, K, dqv);
+      store4<VEC>(a.dk + grow * K, kc, K, dkv);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int kc = 32 * P + 16 * c + 4 * gq;
+    f32x4 x = ref4(&L.sDgH[kc]) * exp4(between(L.sE, -1, 4, kc)) + (pre[c] + suf[c]);
+    for (int B = 0; B < 4; ++B) {
+      if (B < I) x += ref4(&L.totT[B][kc]);
+      if (B > I) x += ref4(&L.totG[B][kc]);
+    }
+    if (in) store4<VEC>(a.dg + grow * K, kc, K, x);
+  }
+}
+
+inline int64_t f32_slots(int n_seq, int64_t T) { return T / kC + n_seq + 1; }
+constexpr size_t kF32Align = 16;
 
 }  // namespace
 }  // namespace ssla
@@ -513,9 +945,62 @@ extern "C" int ssla_gla_chunk_f32_fwd(const float *q, const float *k, const floa
   return launch_status("gla_chunk_f32_fwd");
 }
 
+extern "C" size_t ssla_gla_chunk_f32_fwd_workspace_size(int n_seq, int64_t T, int H, int K, int V) {
+  if (n_seq < 0 || T < 0 || H <= 0 || K <= 0 || V <= 0) return 0;
+  const size_t items = static_cast<size_t>(ssla::f32_slots(n_seq, T)) * H;
+  return items * (64 + static_cast<size_t>((V + 63) / 64) * 4096) * sizeof(float) + ssla::kF32Align;
+}
+
+extern "C" int ssla_gla_chunk_f32_fwd_ws(const float *q, const float *k, const float *v, const float *g,
+                                         const int64_t *cu_seqlens, int n_seq, int64_t T, int H, int K, int V,
+                                         float scale, const float *h0, float *o, float *ht, void *workspace,
+                                         size_t workspace_bytes, void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(n_seq >= 0 && T >= 0 && H > 0 && K > 0 && V > 0,
+                 "gla_chunk_f32_fwd: bad sizes n_seq=%d T=%lld H=%d K=%d V=%d", n_seq, (long long)T, H, K, V);
+  if (K > 64 || V > 256) {
+    set_error("gla_chunk_f32_fwd: K=%d V=%d (K <= 64 and V <= 256 per call)", K, V);
+    return SSLA_ERR_UNSUPPORTED;
+  }
+  if (n_seq == 0) return SSLA_OK;
+  SSLA_CHECK_ARG(cu_seqlens && (T == 0 || (q && k && v && g && o)), "gla_chunk_f32_fwd: null pointer");
+  const size_t need = ssla_gla_chunk_f32_fwd_workspace_size(n_seq, T, H, K, V);
+  if (workspace == nullptr || workspace_bytes < need) {
+    set_error("gla_chunk_f32_fwd: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    return SSLA_ERR_WORKSPACE;
+  }
+  F32Args a = {};
+  a.q = q, a.k = k, a.v = v, a.g = g, a.h0 = h0, a.cu = cu_seqlens, a.o = o, a.ht = ht;
+  a.T = T, a.n_slots = f32_slots(n_seq, T), a.n_seq = n_seq, a.H = H, a.K = K, a.V = V, a.nvg = (V + 63) / 64;
+  a.scale = scale;
+  a.sh = reinterpret_cast<float *>((reinterpret_cast<uintptr_t>(workspace) + kF32Align - 1) / kF32Align * kF32Align);
+  a.eh = a.sh + static_cast<size_t>(a.n_slots) * H * a.nvg * 4096;
+  const int64_t chunks = a.n_slots * H * a.nvg, seqs = static_cast<int64_t>(n_seq) * H * a.nvg * 4;
+  SSLA_CHECK_ARG(chunks < 0x7fffffff && seqs < 0x7fffffff, "gla_chunk_f32_fwd: too many (chunk, head, tile) items");
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool vec = K % 4 == 0 && V % 4 == 0 && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(g, 16) &&
+                   aligned(o, 16);
+  const dim3 gc(static_cast<unsigned>(chunks));
+  if (T > 0) {
+    if (vec)
+      hipLaunchKernelGGL(f32_states_kernel<true>, gc, dim3(256), 0, s, a, ht != nullptr, 0);
+    else
+      hipLaunchKernelGGL(f32_states_kernel<false>, gc, dim3(256), 0, s, a, ht != nullptr, 0);
+  }
+  hipLaunchKernelGGL(f32_prefix_kernel, dim3(static_cast<unsigned>(seqs)), dim3(256), 0, s, a);
+  if (T > 0) {
+    if (vec)
+      hipLaunchKernelGGL(f32_out_kernel<true>, gc, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL(f32_out_kernel<false>, gc, dim3(256), 0, s, a);
+  }
+  return launch_status("gla_chunk_f32_fwd");
+}
+
 extern "C" size_t ssla_gla_chunk_f32_bwd_workspace_size(int n_seq, int64_t T, int H) {
   if (n_seq < 0 || T < 0 || H <= 0) return 0;
-  return static_cast<size_t>(ssla::f32_bwd_slots(n_seq, T)) * H * 64 * 64 * sizeof(float);
+  return static_cast<size_t>(ssla::f32_slots(n_seq, T)) * H * 2 * (64 + 4096) * sizeof(float) + ssla::kF32Align;
 }
 
 extern "C" int ssla_gla_chunk_f32_bwd(const float *q, const float *k, const float *v, const float *g,
@@ -540,10 +1025,33 @@ extern "C" int ssla_gla_chunk_f32_bwd(const float *q, const float *k, const floa
     set_error("gla_chunk_f32_bwd: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     return SSLA_ERR_WORKSPACE;
   }
-  const int64_t blocks = static_cast<int64_t>(n_seq) * H;
-  SSLA_CHECK_ARG(blocks < 0x7fffffff, "gla_chunk_f32_bwd: too many (sequence, head) items");
-  hipLaunchKernelGGL(f32_bwd_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0,
-                     static_cast<hipStream_t>(stream), q, k, v, g, cu_seqlens, n_seq, T, H, K, V, scale, h0, do_, dht,
-                     dq, dk, dv, dg, dh0, static_cast<float *>(workspace), f32_bwd_slots(n_seq, T));
+  F32Args a = {};
+  a.q = q, a.k = k, a.v = v, a.g = g, a.dO = do_, a.h0 = h0, a.dht = dht, a.cu = cu_seqlens;
+  a.dq = dq, a.dk = dk, a.dv = dv, a.dg = dg, a.dh0 = dh0;
+  a.T = T, a.n_slots = f32_slots(n_seq, T), a.n_seq = n_seq, a.H = H, a.K = K, a.V = V, a.nvg = 1, a.scale = scale;
+  const size_t items = static_cast<size_t>(a.n_slots) * H;
+  a.sh = reinterpret_cast<float *>((reinterpret_cast<uintptr_t>(workspace) + kF32Align - 1) / kF32Align * kF32Align);
+  a.sd = a.sh + items * 4096;
+  a.eh = a.sd + items * 4096;
+  a.ed = a.eh + items * 64;
+  const int64_t chunks = a.n_slots * H, seqs = static_cast<int64_t>(n_seq) * H * 4;
+  SSLA_CHECK_ARG(chunks < 0x7fffffff && seqs < 0x7fffffff, "gla_chunk_f32_bwd: too many (chunk, head) items");
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool vec = K % 4 == 0 && V % 4 == 0 && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(g, 16) &&
+                   aligned(do_, 16) && aligned(dq, 16) && aligned(dk, 16) && aligned(dv, 16) && aligned(dg, 16);
+  const dim3 gs(static_cast<unsigned>(chunks), 2), gc(static_cast<unsigned>(chunks));
+  if (T > 0) {
+    if (vec)
+      hipLaunchKernelGGL(f32_states_kernel<true>, gs, dim3(256), 0, s, a, 0, dh0 != nullptr);
+    else
+      hipLaunchKernelGGL(f32_states_kernel<false>, gs, dim3(256), 0, s, a, 0, dh0 != nullptr);
+  }
+  hipLaunchKernelGGL(f32_prefix_kernel, dim3(static_cast<unsigned>(seqs), 2), dim3(256), 0, s, a);
+  if (T > 0) {
+    if (vec)
+      hipLaunchKernelGGL(f32_grad_kernel<true>, gc, dim3(kGradThreads), 0, s, a);
+    else
+      hipLaunchKernelGGL(f32_grad_kernel<false>, gc, dim3(kGradThreads), 0, s, a);
+  }
   return launch_status("gla_chunk_f32_bwd");
 }

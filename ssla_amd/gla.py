@@ -172,7 +172,7 @@ def _chunk_fwd(q, k, v, g, cu, scale, h0, output_final_state):
 
 
 def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
-    """One ssla_gla_chunk_fwd call (K == KD), or one ssla_gla_chunk_f32_fwd
+    """One ssla_gla_chunk_fwd call (K == KD), or one ssla_gla_chunk_f32_fwd_ws
     call for fp32 inputs (K <= KD)."""
     T, H, K = q.shape
     V = v.shape[-1]
@@ -181,9 +181,12 @@ def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
     ht = torch.empty(N, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
     lib = _lib.load()
     if q.dtype == torch.float32:
-        st = lib.ssla_gla_chunk_f32_fwd(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.ptr(cu), N, T, H, K,
-                                        V, float(scale), _lib.ptr(h0), _lib.ptr(o), _lib.ptr(ht), _lib.stream_of(q))
-        _lib.check(st, "ssla_gla_chunk_f32_fwd")
+        ws_bytes = lib.ssla_gla_chunk_f32_fwd_workspace_size(N, T, H, K, V)
+        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+        st = lib.ssla_gla_chunk_f32_fwd_ws(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.ptr(cu), N, T, H,
+                                           K, V, float(scale), _lib.ptr(h0), _lib.ptr(o), _lib.ptr(ht), _lib.ptr(ws),
+                                           ws_bytes, _lib.stream_of(q))
+        _lib.check(st, "ssla_gla_chunk_f32_fwd_ws")
         return o, ht
     ws_bytes = lib.ssla_gla_chunk_workspace_size(N, T, H, K, V)
     ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None

@@ -1,0 +1,73 @@
+"""The chunk-parallel fp32 GLA kernels (ssla_gla_chunk_f32_fwd_ws and
+ssla_gla_chunk_f32_bwd) where their indexing can go wrong, against the fp64
+recurrence at the fp32 bar of the other chunk tests (rtol 1e-4, atol 1e-4 of
+the RMS): scalar loads (K or V not a multiple of 4), several value groups,
+sequence counts that take one, two and three rounds of the 64-way slot
+search, rows outside every sequence, and decays on both sides of the range
+the matrix-core diagonal blocks take (40 binary orders within 16 rows)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.conftest import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(lens, lead, tail, H, K, V, gate, seed):
+    gen = torch.Generator().manual_seed(seed)
+    T = lead + sum(lens) + tail
+    q, k, v = (torch.randn(T, H, d, generator=gen) for d in (K, K, V))
+    g = -gate * torch.rand(T, H, K, generator=gen) if gate > 0 else torch.randn(T, H, K, generator=gen) * -gate
+    cu = lead + np.concatenate([[0], np.cumsum(lens)])
+    h0 = torch.randn(len(lens), H, K, V, generator=gen) * 0.1
+    return q, k, v, g, torch.tensor(cu, dtype=torch.int64), h0
+
+
+@pytest.mark.parametrize("lens,lead,tail,H,K,V,gate", [
+    ([70, 64, 1], 3, 5, 2, 33, 30, 0.2),
+    ([129], 0, 0, 1, 5, 130, 1.0),
+    ([1] * 63 + [65] * 3, 2, 0, 1, 16, 16, 0.5),
+    ([2] * 70 + [0, 0, 66], 0, 9, 1, 64, 64, 3.4),      # 15 steps of up to 4.9 bits: both sides of 40
+    ([1] * 4100, 1, 1, 1, 4, 4, 0.1),
+    ([200, 63], 0, 0, 2, 64, 64, 30.0),                 # far past it: every diagonal block term by term
+    ([150], 0, 0, 2, 64, 48, -1.5),                     # growing gates: either sign
+])
+def test_f32_chunks(dev, lens, lead, tail, H, K, V, gate):
+    from ssla_amd.gla import chunk_gla
+    print(f"f32 chunks: {len(lens)} sequences K={K} V={V} gate={gate}", flush=True)
+    q, k, v, g, cu, h0 = _case(lens, lead, tail, H, K, V, gate, seed=len(lens) + K)
+    gen = torch.Generator().manual_seed(1)
+    do, dht = torch.randn(v.shape, generator=gen), torch.randn(h0.shape, generator=gen) * 0.1
+    lo, hi = int(cu[0]), int(cu[-1])
+    leaf = [t.to(dev).requires_grad_() for t in (q, k, v, g, h0)]
+    o, ht = chunk_gla(*leaf[:4], cu.to(dev), scale=0.3, initial_state=leaf[4], output_final_state=True)
+    seq = lambda t: t[lo:hi].numpy()   # noqa: E731
+    cz = cu.numpy() - lo
+    ro, rht = oracle.gla_recurrent(seq(q), seq(k), seq(v), seq(g), cz, 0.3, h0.numpy(), True)
+    assert_close(o.detach().cpu().numpy()[lo:hi], ro, 1e-4, "o")
+    assert_close(ht.detach().cpu().numpy(), rht, 1e-4, "ht")
+    if gate < 0:
+        return   # sums of growing terms: the forward only
+    # rows outside every sequence are unspecified: keep them out of the loss
+    ((o[lo:hi] * do[lo:hi].to(dev)).sum() + (ht * dht.to(dev)).sum()).backward()
+    ref = oracle.gla_recurrent_bwd(seq(q), seq(k), seq(v), seq(g), cz, seq(do), 0.3, h0.numpy(), dht.numpy())
+    for nm, t, r in zip(("dq", "dk", "dv", "dg", "dh0"), leaf, ref):
+        got = t.grad.cpu().numpy()
+        assert_close(got if nm == "dh0" else got[lo:hi], r, 1e-4, nm)
+
+
+def test_f32_chunk_forward_without_workspace(dev):
+    """ssla_gla_chunk_f32_fwd (no workspace) on the same inputs."""
+    from ssla_amd import _lib
+    lib = _lib.load()
+    q, k, v, g, cu, h0 = _case([70, 64, 1], 0, 0, 2, 32, 40, 0.3, seed=5)
+    ro, rht = oracle.gla_recurrent(q.numpy(), k.numpy(), v.numpy(), g.numpy(), cu.numpy(), 0.3, h0.numpy(), True)
+    d = [t.to(dev) for t in (q, k, v, g, cu, h0)]
+    o, ht = torch.empty_like(d[2]), torch.empty_like(d[5])
+    T, H, K = q.shape
+    _lib.check(lib.ssla_gla_chunk_f32_fwd(*(_lib.ptr(t) for t in d[:5]), 3, T, H, K, 40, 0.3, _lib.ptr(d[5]), _lib.ptr(o),
+                                          _lib.ptr(ht), _lib.stream_of(o)), "f32_fwd")
+    assert_close(o.cpu().numpy(), ro, 1e-4, "o")
+    assert_close(ht.cpu().numpy(), rht, 1e-4, "ht")
