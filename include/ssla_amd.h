@@ -491,6 +491,31 @@ int ssla_mos_attention_fwd(const float *events, int64_t n_events, int c_in, cons
                            const float *w_in, const float *ln_w, const float *ln_b, float eps, int hidden,
                            float *out, void *workspace, size_t workspace_bytes, void *stream);
 
+/* Training form of the same layer (up to the LayerNorm; reference
+ * layers/mos_attention.py:103-140): forward with what the backward needs
+ * kept, and the backward.  The matrices come folded per kernel position:
+ * Wa [A * 3H, c_in] (rows a * 3H + {q, v, g}: W_{q,v,g} W_scatter[a]), WbT
+ * [H, A * H] (columns a * H + m: W_gather[a] W_o), Win [H, c_in] or NULL.
+ * src, pos [n_rows]: event and kernel position of the patch rows (each
+ * (event, position) at most once), cu [n_patches + 1] the patch offsets.
+ * Writes qvh [E, A, 3H] (q, scan output h, sigmoid gate), y [E, A, H] = q h
+ * (zero for copies in no patch), valid [E, A] (zeroed by the caller; 1 for
+ * copies in a patch) and out [E, H] = sum_a Wb[a] y (+ Win x).  The backward
+ * takes dout [E, H], the saved tensors and the transposes WaT [c_in, A * 3H],
+ * Wbp = WbT^T [A * H, H], WinT [c_in, H] (or NULL), and writes those of devents
+ * [E, c_in], dWaT, dWbT (laid out as WaT, WbT) and dWinT [c_in, H] that are
+ * not NULL.  fp32; c_in, H <= 128, A <= 49; sums in a fixed order. */
+int ssla_mos_train_fwd(const float *events, int64_t E, int c_in, const int64_t *src, const int64_t *pos,
+                       int64_t n_rows, const int64_t *cu, int64_t n_patches, int A, const float *Wa,
+                       const float *WbT, const float *Win, int H, float *qvh, float *y, unsigned char *valid,
+                       float *out, void *stream);
+size_t ssla_mos_train_bwd_workspace_size(int64_t E, int c_in, int A, int H);
+int ssla_mos_train_bwd(const float *dout, const float *events, int64_t E, int c_in, const int64_t *src,
+                       const int64_t *pos, int64_t n_rows, const int64_t *cu, int64_t n_patches, int A,
+                       const float *WaT, const float *Wbp, const float *WinT, int H, const float *qvh,
+                       const float *y, const unsigned char *valid, float *devents, float *dWaT, float *dWbT,
+                       float *dWinT, void *workspace, size_t workspace_bytes, void *stream);
+
 /* Stable sort of (uint64 key, int32 value) pairs on the low end_bit key
  * bits; vals_in NULL means 0..n-1.  Used for the (batch, time) ordering of
  * LinearAttention.forward (layers/linear_attention.py:62-63) and the

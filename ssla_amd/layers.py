@@ -93,6 +93,59 @@ def _grouped_linear(x: torch.Tensor, pos: torch.Tensor, weights: torch.Tensor) -
 
 
 # ---------------------------------------------------------------- attention --
+def _plain_linear(m) -> bool:
+    """An nn.Linear without a bias, a parametrization or hooks: its map is
+    its weight alone."""
+    return (type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks
+            and not m._backward_hooks and not m._backward_pre_hooks)
+
+
+class MosTrainFunction(torch.autograd.Function):
+    """The part of MosAttention between the patch plan and the LayerNorm, with
+    its backward (ssla_mos_train_fwd / _bwd): out[e] = sum_a Wb[a] y[e, a]
+    (+ Win x[e]) with (q, v, g) = Wa[a] x[e], h = sigmoid(g) h_prev + v along
+    each patch and y = q h.  WaT ``[Cin, A * 3H]`` and WbT ``[H, A * H]`` are
+    the folded matrices, Win ``[H, Cin]`` or None; src, pos the patch rows'
+    event and kernel position, cu the patch offsets."""
+
+    @staticmethod
+    def forward(ctx, events, WaT, WbT, Win, src, pos, cu, A):
+        n, Cin = events.shape
+        H, dev = WbT.shape[0], events.device
+        new = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)   # noqa: E731
+        qvh, y, out = new(n, A * 3 * H), new(n, A * H), new(n, H)
+        valid = torch.zeros(n * A, dtype=torch.uint8, device=dev)
+        Wa, WbT = WaT.t().contiguous(), WbT.contiguous()
+        Win_c = None if Win is None else Win.contiguous()
+        P = _lib.ptr
+        _lib.check(_lib.load().ssla_mos_train_fwd(P(events), n, Cin, P(src), P(pos), src.numel(), P(cu),
+                                                  cu.numel() - 1, A, P(Wa), P(WbT), P(Win_c), H, P(qvh), P(y),
+                                                  P(valid), P(out), _lib.stream_of(events)), "mos_train_fwd")
+        ctx.A = A
+        ctx.save_for_backward(events, WaT, WbT, Win, src, pos, cu, qvh, y, valid)
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout):
+        events, WaT, WbT, Win, src, pos, cu, qvh, y, valid = ctx.saved_tensors
+        A, (n, Cin), H, dev = ctx.A, events.shape, WbT.shape[0], events.device
+        need = ctx.needs_input_grad
+        dout = dout.to(torch.float32).contiguous()
+        new = lambda on, *shape: torch.empty(*shape, dtype=torch.float32, device=dev) if on else None   # noqa: E731
+        dev_x, dWaT, dWbT = new(need[0], n, Cin), new(need[1], Cin, A * 3 * H), new(need[2], H, A * H)
+        dWinT = new(Win is not None and need[3], Cin, H)
+        WaT, Wbp = WaT.contiguous(), WbT.t().contiguous()
+        WinT = None if Win is None else Win.t().contiguous()
+        lib, P = _lib.load(), _lib.ptr
+        ws = E._ws(lib.ssla_mos_train_bwd_workspace_size(n, Cin, A, H), dev)
+        _lib.check(lib.ssla_mos_train_bwd(P(dout), P(events), n, Cin, P(src), P(pos), src.numel(), P(cu),
+                                          cu.numel() - 1, A, P(WaT), P(Wbp), P(WinT), H, P(qvh), P(y), P(valid),
+                                          P(dev_x), P(dWaT), P(dWbT), P(dWinT), P(ws), ws.numel(),
+                                          _lib.stream_of(dout)), "mos_train_bwd")
+        return dev_x, dWaT, dWbT, None if dWinT is None else dWinT.t(), None, None, None, None
+
+
 class MosAttention(nn.Module):
     """Mixture-of-sparse (patch) linear attention layer; reference
     layers/mos_attention.py:12-167.  forward(dict) -> dict with the keys of
@@ -169,10 +222,47 @@ class MosAttention(nn.Module):
             _lib.stream_of(events)), "mos_attention_fwd")
         return out
 
+    def _train_ok(self, events):
+        """The training kernels (MosTrainFunction) take the layer: fp32
+        throughout, sizes up to 128 and 49 positions, and projections that
+        are their weights alone (the composed path calls the modules)."""
+        A = self.kernel_size[0] * self.kernel_size[1]
+        ps = (self.scatter_conv_weights, self.gather_conv_weights, self.q_proj.weight, self.v_proj.weight,
+              self.g_proj.weight, self.o_proj.weight)
+        return (events.dim() == 2 and events.dtype == torch.float32 and events.shape[0] > 0
+                and events.shape[1] == self.input_size and not torch.is_autocast_enabled()
+                and self.input_size <= 128 and self.hidden_size <= 128 and A <= 49
+                and events.shape[0] * A < 0x7fffffff
+                and all(p.dtype == torch.float32 and p.device == events.device for p in ps)
+                and _plain_linear(self.o_proj)
+                and (self.input_proj is None or (_plain_linear(self.input_proj)
+                                                 and self.input_proj.weight.dtype == torch.float32)))
+
+    def _forward_train(self, inputs, events, rows):
+        """out + residual from the patch rows, differentiable (MosTrainFunction
+        on the folded matrices)."""
+        src, _tim, pos, _f_index, f_len, _n = rows
+        H, A = self.hidden_size, self.kernel_size[0] * self.kernel_size[1]
+        ws = self.scatter_conv_weights.reshape(-1, H, self.input_size)
+        wg = self.gather_conv_weights.reshape(-1, H, H)
+        wqvg = torch.cat([self.q_proj.weight, self.v_proj.weight, self.g_proj.weight], 0)
+        # folded in fp64: one rounding, where the products they stand for have one per step
+        Wa = torch.matmul(wqvg.double(), (ws if self.scatter_proj else ws[:1]).double()).float().expand(A, -1, -1)
+        Wb = torch.matmul((wg if self.gather_proj else wg[:1]).double(),
+                          self.o_proj.weight.double()).float().expand(A, -1, -1)
+        WaT = Wa.permute(2, 0, 1).reshape(self.input_size, A * 3 * H)
+        WbT = Wb.permute(1, 0, 2).reshape(H, A * H)
+        cu = F.pad(torch.cumsum(f_len, 0), (1, 0))
+        x = events.contiguous()
+        out = MosTrainFunction.apply(x, WaT, WbT, None if self.input_proj is None else self.input_proj.weight, src, pos,
+                                     cu, A)
+        return out if self.input_proj is not None else out + events
+
     def forward(self, inputs, fused=None):
-        """fused: None picks the fused forward whenever it applies; False
-        forces the composed (differentiable) path; True requires the fused
-        one (SslaError if it does not apply)."""
+        """fused: None picks the fused forward whenever it applies, else the
+        training kernels whenever they do; False forces the composed
+        (differentiable) path; True requires the fused one (SslaError if it
+        does not apply)."""
         events = inputs["events"]
         lengths = inputs["lengths"]
         dev = _lib.require_cuda(events, lengths)
@@ -185,8 +275,17 @@ class MosAttention(nn.Module):
             out = self._forward_fused(inputs, dev)
             return {"events": out, "time": inputs["time"], "w": inputs["w"], "h": inputs["h"],
                     "batch_id": inputs["batch_id"], "lengths": lengths, "batch_size": inputs["batch_size"]}
-        patch = E.scatter_group_events_to_patch(inputs, self.frame_size, self.patch2pixel_lut)
-        p_len, p_ev, p_pos = patch["lengths"], patch["events"], patch["pos_id"]
+        rows = E._rf_scatter(inputs, self.frame_size, self.patch2pixel_lut)
+        # The training kernels work on every (event, position) copy: with a
+        # stride most copies lie in no patch, and past half of them the
+        # composed path's fewer rows win.
+        n_copies = events.shape[0] * self.kernel_size[0] * self.kernel_size[1]
+        if (fused is None and 2 * rows[0].numel() >= n_copies and events.shape[0] == inputs["time"].shape[0]
+                and self._train_ok(events)):
+            out = self.norm(self._forward_train(inputs, events, rows))
+            return {"events": out, "time": inputs["time"], "w": inputs["w"], "h": inputs["h"],
+                    "batch_id": inputs["batch_id"], "lengths": lengths, "batch_size": inputs["batch_size"]}
+        p_ev, p_pos, p_len = E.gather_rows(events, rows[0]), rows[2], rows[4]
         x = self._project(p_ev, p_pos, self.scatter_conv_weights, self.scatter_proj, self.input_size)
         qvg = F.linear(x, torch.cat([self.q_proj.weight, self.v_proj.weight, self.g_proj.weight], 0))
         q, v, g = qvg.split(self.hidden_size, dim=1)
@@ -195,7 +294,7 @@ class MosAttention(nn.Module):
         h = scan(v.contiguous(), torch.sigmoid(g).contiguous(), cu)
         o = self.o_proj(q * h)
         o = self._project(o, p_pos, self.gather_conv_weights, self.gather_proj, self.hidden_size)
-        out = E.gather_patch_events_to_group(o, patch["orig_event_idx"], events.shape[0])
+        out = E.gather_patch_events_to_group(o, rows[0], events.shape[0])
         residual = self.input_proj(events) if self.input_proj is not None else events
         out = self.norm(out + residual)
         return {"events": out, "time": inputs["time"], "w": inputs["w"], "h": inputs["h"],
