@@ -78,8 +78,7 @@ int ssla_status_read(const int32_t *status, int *value_out, void *stream);
  * chunk_fwd_h (ops/common/chunk_h.py:242-294) and the intra-chunk /
  * output kernels (ops/gla/chunk.py:33-249, :644-743).  Supported: dtype
  * BF16 or F16, K == 64, V a multiple of 16 (<= 256) -- other key widths
- * run as groups of 64 keys (the last one zero-padded) whose o add up, since
- * each key's decay only touches its own state row; one sequence below
+ * go to ssla_gla_chunk_fwd_wide; one sequence below
  * 2^31 bytes per tensor (rows * H * max(K, V) * 4), SSLA_ERR_UNSUPPORTED
  * otherwise.  Only a batch with T * H * max(K, V) * 4 >= 2^31 can hold such
  * a sequence: then cu_seqlens is read back to check (one host
@@ -89,7 +88,9 @@ int ssla_status_read(const int32_t *status, int *value_out, void *stream);
  * initialisation needed) holds one bf16 hi / lo state pair (as the
  * reference stores its per-chunk states, ops/gla/chunk.py:933) and one
  * fp32 decay row per segment.  A size of 0
- * means no workspace is needed for this shape (pass NULL, 0). */
+ * means no workspace is needed for this shape (pass NULL, 0); a batch of so
+ * many sequences that one segment each fills the GPU is cut only to balance
+ * ragged lengths, and runs uncut when the workspace is not given. */
 size_t ssla_gla_chunk_workspace_size(int n_seq, int64_t T, int H, int K, int V);
 
 int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v,
@@ -98,6 +99,18 @@ int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v,
                        int H, int K, int V, float scale,
                        const float *h0, void *o, float *ht, int dtype,
                        void *workspace, size_t workspace_bytes, void *stream);
+
+/* ssla_gla_chunk_fwd for K a multiple of 16 up to 128 (wider keys: groups of
+ * 128 whose o add up, since each key's decay only touches its own state
+ * row), with its own workspace query. */
+size_t ssla_gla_chunk_wide_workspace_size(int n_seq, int64_t T, int H, int K, int V);
+
+int ssla_gla_chunk_fwd_wide(const void *q, const void *k, const void *v,
+                            const void *g, int g_dtype,
+                            const int64_t *cu_seqlens, int n_seq, int64_t T,
+                            int H, int K, int V, float scale,
+                            const float *h0, void *o, float *ht, int dtype,
+                            void *workspace, size_t workspace_bytes, void *stream);
 
 /* Allocation-free variant of ssla_gla_chunk_fwd (same arguments without
  * the workspace, same kernels, same results bit for bit).  It has no

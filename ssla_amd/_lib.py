@@ -50,6 +50,9 @@ SIGNATURES = {
     "ssla_gla_chunk_workspace_size": (_sz, [_i32, _i64, _i32, _i32, _i32]),
     "ssla_gla_chunk_fwd": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i32, _i32, _i32,
                                   _f32, _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
+    "ssla_gla_chunk_wide_workspace_size": (_sz, [_i32, _i64, _i32, _i32, _i32]),
+    "ssla_gla_chunk_fwd_wide": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i32, _i32, _i32,
+                                       _f32, _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
     "ssla_gla_chunk_fwd_noalloc": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i32, _i32, _i32,
                                           _f32, _vp, _vp, _vp, _i32, _vp]),
     "ssla_gla_chunk_f32_fwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _f32, _vp, _vp, _vp,

@@ -11,10 +11,12 @@
 // with S_0 = h0 (or 0) and ht = S after the last chunk.
 //
 // Schedule (two launches; the only intermediates are per-segment states):
-// * Each (sequence, head, V group) chain is cut into P segments of whole
-//   chunks (P chosen so that about two workgroups run per CU).
-// * state pass  : segments 0..P-2 run the state recurrence only (reads k, g,
-//   v) from h0 (segment 0) or zero, leaving the segment's final state and
+// * Each (sequence, head, V group) chain is cut into segments of `per` whole
+//   chunks (per chosen so that about two workgroups run per CU): longer
+//   sequences get more segments, so a ragged batch's longest sequence does
+//   not set the time alone.  A segment is found from its slot (seq_slots.h).
+// * state pass  : all but a sequence's last segment run the state recurrence
+//   only (reads k, g, v) from h0 (segment 0) or zero, leaving the segment's final state and
 //   total log2-decay D in a workspace slot.  The state is stored as a bf16
 //   pair: hi = bf16(S) and lo = bf16(S - hi), so hi + lo holds S to about
 //   2^-17.
@@ -29,7 +31,17 @@
 //   ht = S(fold(hi)) + decay * fold(lo)): ht carries fp32-level accuracy
 //   across segments without delaying the segment's first chunk.
 //
-// Inside a workgroup (256 threads, 4 wavefronts): wavefront I owns chunk
+// Keys: a wavefront works on 64 of them.  K <= 64 runs one such group (keys
+// past K read zeros), 64 < K <= 128 two groups side by side in a workgroup of
+// 8 wavefronts: the groups are independent GLAs (each key decays its own
+// state row) whose o tiles add up in fp32 through LDS before the one rounding.
+// 21 ragged sequences of 16,411 rows in all at H = 4, K = V = 128: 91 us a call
+// (state pass 23, segment pass 75 us under the profiler), against 288-333 us
+// as one call per 64 zero-padded keys, cut into equal counts of segments, with
+// the copies and the sum around them.  What bounds it is the segment pass's
+// chunk loop at two wavefronts per SIMD, as at K = 64.
+//
+// Inside a key group (256 threads, 4 wavefronts): wavefront I owns chunk
 // rows 16I..16I+15 ("block" I) and state rows (keys) 16I..16I+15 as MFMA
 // accumulators.  All products are v_mfma_f32_16x16x32_{bf16,f16}.  Within a
 // lane the 64 keys are held as k = 32*jj + 8*(lane/16) + e (jj = 0,1; e =
@@ -52,6 +64,7 @@
 // (states_in_fp32=False, ops/gla/chunk.py:933).  scale is applied to o at
 // the end.
 #include "lds_tile.h"
+#include "seq_slots.h"
 
 #include <atomic>
 #include <mutex>
@@ -226,25 +239,27 @@ struct LineOffs {
   uint32_t v;     // v: row 16w + lane/8, columns v0 + 8 (lane%8)
 };
 
-__device__ __forceinline__ LineOffs line_offs(int c, int wv, int lane, int H, int h, int V, int v0, int gsz) {
+__device__ __forceinline__ LineOffs line_offs(int c, int wv, int lane, int H, int h, int K, int k0, int V, int v0,
+                                              int gsz) {
   LineOffs o;
   const uint32_t r8 = static_cast<uint32_t>((c * BT + 16 * wv + (lane >> 3)) * H + h);
   const uint32_t r16 = static_cast<uint32_t>((c * BT + 16 * wv + (lane >> 4)) * H + h);
-  o.a16 = r8 * (KD * 2) + 16 * (lane & 7);
-  o.g = gsz == 4 ? r16 * (KD * 4) + 16 * (lane & 15) : o.a16;
+  o.a16 = (r8 * K + k0) * 2 + 16 * (lane & 7);
+  o.g = gsz == 4 ? (r16 * K + k0) * 4 + 16 * (lane & 15) : o.a16;
   o.v = r8 * static_cast<uint32_t>(V * 2) + static_cast<uint32_t>(v0 * 2) + 16 * (lane & 7);
   return o;
 }
 
 // Issue the whole-line loads of one chunk.  `valid` false (no next chunk)
 // turns every load into a zero read without memory traffic, so the
-// instruction stream is the same on every iteration; v pieces beyond the V
-// group (vcol_ok false) read zeros as well.
+// instruction stream is the same on every iteration; pieces beyond the keys
+// (k_ok, g_ok false) or the V group (vcol_ok false) read zeros as well.
 template <bool LOADQ, bool GF32>
 __device__ __forceinline__ void load_lines(LineRegs &L, const SeqRsrc &rs, bool valid, const LineOffs &o, int H,
-                                           int V, bool vcol_ok) {
-  const uint32_t a = valid ? o.a16 : kNoLoad, b = valid ? o.g : kNoLoad, c = (valid && vcol_ok) ? o.v : kNoLoad;
-  const uint32_t s16 = 8 * H * KD * 2, sg = 4 * H * KD * 4, sv = 8 * H * V * 2;
+                                           int K, int V, bool k_ok, bool g_ok, bool vcol_ok) {
+  const uint32_t a = (valid && k_ok) ? o.a16 : kNoLoad, c = (valid && vcol_ok) ? o.v : kNoLoad;
+  const uint32_t b = (valid && g_ok) ? o.g : kNoLoad;
+  const uint32_t s16 = 8 * H * K * 2, sg = 4 * H * K * 4, sv = 8 * H * V * 2;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     if (LOADQ) L.q[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs.q, a + i * s16, 0, 0));
@@ -321,10 +336,12 @@ __device__ __forceinline__ void store_v_lines(uint16_t *vs, const LineRegs &L, i
 // the instruction stream is the same on every iteration.
 template <bool LOADQ, bool GF32>
 __device__ __forceinline__ void load_chunk(SegRegs &R, const SeqRsrc &rs, bool valid, uint32_t oq,
-                                           uint32_t og, uint32_t ov, int kq, int vw) {
-  const uint32_t q0 = valid ? oq : kNoLoad, g0 = valid ? og : kNoLoad;
+                                           uint32_t og, uint32_t ov, int kq, int kw, int vw) {
 #pragma unroll
   for (int jj = 0; jj < 2; ++jj) {
+    // keys beyond the group's kw read zeros
+    const bool k_ok = valid && 32 * jj + kq < kw;
+    const uint32_t q0 = k_ok ? oq : kNoLoad, g0 = k_ok ? og : kNoLoad;
     if (LOADQ) R.q[jj] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs.q, q0 + 64 * jj, 0, 0));
     R.k[jj] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs.k, q0 + 64 * jj, 0, 0));
     if (GF32) {
@@ -387,21 +404,72 @@ struct ChunkArgs {
   const float *h0;
   uint16_t *o;
   float *ht;
-  const uint16_t *ws_state;  // [n_seq, H, P] slots of K*V bf16 in slot_index order: local end state of segment s (hi)
+  const uint16_t *ws_state;  // slots of 64 V bf16 in slot_index order: local end state of a segment (hi)
   const uint16_t *ws_lo;     // the same slots: bf16(S - hi)
-  const float *ws_decay;   // [n_seq, H, P, K] fp32: total log2 decay of segment s
+  const float *ws_decay;   // 64 fp32 per slot: total log2 decay of the segment
   int64_t bos;             // first row of the sequence
   int64_t len;             // rows of the sequence
+  int64_t store;           // workspace slot of the sequence's segment 0 (this head and key group)
+  int slot_step;           // workspace slots from one segment to the next
   int c_beg, c_end;        // chunk range of the segment
-  int H, V, h, n, v0, seg, P;
+  int H, K, V, h, n, v0, seg;
+  bool last;               // the sequence's last segment
   float scale;
 };
 
-// Chunk range of segment `seg` of a sequence with `nch` chunks cut in P parts.
-__device__ __forceinline__ void segment_range(int nch, int P, int seg, int &c0, int &c1) {
-  const int per = (nch + P - 1) / P;
-  c0 = min(seg * per, nch);
-  c1 = min(c0 + per, nch);
+// Where a workgroup works.  Blocks go to the 8 XCDs in turn: the `inner` blocks
+// that read the same rows (V groups, key groups of the state pass) are placed
+// 8 apart, so they run on one XCD close in time and share its L2.  Beyond that
+// heads vary fastest, so every XCD runs every segment index of a sequence in
+// equal shares (with a fixed segment index per XCD the one holding the last
+// segments, the longest folds, set the end: 54.8 against 48.1 us at 8 x 4096
+// rows, H = 8).  The state pass (STORES) runs over the storing segments' own
+// slots: over the segment pass's a quarter of its workgroups found nothing to
+// do, but had been dealt to CUs like the rest, and some CUs got three that
+// did and some one (37.1 against 29.5 us).
+struct SegPlace {
+  int n, seg, nseg, h, in;
+  int64_t bos, len, first;
+};
+template <bool STORES>
+__device__ __forceinline__ bool segment_place(const int64_t *cu, int n_seq, int64_t T, int H, int per, int inner,
+                                              int slots, int even, SegPlace &p) {
+  const unsigned t = blockIdx.x >> 3, item = t / inner * 8 + (blockIdx.x & 7);
+  p.in = static_cast<int>(t % inner);
+  p.h = static_cast<int>(item % H);
+  const int slot = static_cast<int>(item / H);
+  if (slot >= slots) return false;   // (the grid is rounded up)
+  const int64_t unit = static_cast<int64_t>(BT) * per;
+  int64_t eos;
+  if (even) {
+    // sequences of even * unit rows each, as far as the host can tell: if the
+    // one whose slot this would be is, its place is known without a search
+    // (a call of 8 x 4096 rows takes 77.5 us so, 79.1 with the search)
+    const int own = STORES ? even : even + 1;
+    p.n = static_cast<int>(static_cast<unsigned>(slot) / static_cast<unsigned>(own));
+    p.seg = slot - p.n * own;
+    if (p.n < n_seq) {
+      p.bos = cu[p.n];
+      eos = cu[p.n + 1];
+      if (p.bos == p.n * (even * unit) && eos == p.bos + even * unit) {
+        p.len = even * unit;
+        p.nseg = even;
+        p.first = static_cast<int64_t>(p.n) * own;
+        return p.seg < even;
+      }
+    }
+  }
+  if (!seq_of_slot<!STORES>(cu, n_seq, T, unit, slot, p.n, p.bos, eos, p.first)) return false;
+  p.len = eos - p.bos;
+  p.seg = static_cast<int>(slot - p.first);
+  // (an empty sequence has one empty segment: its final state is its initial one)
+  p.nseg = max(1, static_cast<int>((p.len + unit - 1) / unit));
+  return p.seg < p.nseg;
+}
+// Workspace slot of segment 0 of a sequence (first without n: only segments
+// with a successor store).
+__device__ __forceinline__ int64_t store_slot(int64_t first, const SegPlace &p, int H, int KG, int kg) {
+  return (first * H + p.h) * KG + kg;
 }
 
 // E = slot 0, E = 2^D(j) E + slot j for 0 < j < a.seg (in this order, so
@@ -417,8 +485,8 @@ __device__ __forceinline__ void fold_slots(const struct ChunkArgs &a, int64_t sl
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (j0 + u < a.seg) {
-        const int64_t so = sl0 + static_cast<int64_t>(j0 + u) * KD * a.V;
-        d[u] = *reinterpret_cast<const f32x4 *>(dk + static_cast<int64_t>(j0 + u) * KD);
+        const int64_t so = sl0 + static_cast<int64_t>(j0 + u) * a.slot_step * KD * a.V;
+        d[u] = *reinterpret_cast<const f32x4 *>(dk + static_cast<int64_t>(j0 + u) * a.slot_step * KD);
 #pragma unroll
         for (int t = 0; t < NVT; ++t) xb[u][t] = *reinterpret_cast<const uint2 *>(base + so + 4 * t);
       }
@@ -449,10 +517,16 @@ __device__ __forceinline__ void fold_slots(const struct ChunkArgs &a, int64_t sl
 }
 
 // --------------------------------------------------------- segment pass --
-template <int DT, bool GF32, int NVT>
-__device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, const int wv, int lane) {
+// KS: the key width when it is 64 (strides and guards are constants), else 0.
+// KG: key groups of the workgroup; this wavefront's is kg.  xch (KG = 2): the
+// o tiles each group hands to the other, [group][wavefront][tile][lane].
+template <int DT, bool GF32, int NVT, int KS, int KG>
+__device__ __forceinline__ void segment_loop(SmemA &sm, f32x4 *xch, const ChunkArgs &a, const int wv, const int kg,
+                                             int lane) {
   typedef Mfma<DT> M;
   typedef typename M::Vec MV;
+  const int K = KS ? KS : a.K;
+  const int kw = KS ? KD : min(KD, K - KD * kg);   // keys of this group
   const int r = lane & 15;        // row within block / MFMA column index
   const int gq = lane >> 4;       // lane group
   const int kq = 8 * gq;          // key offset of this lane inside each K=32 half
@@ -461,25 +535,26 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
   const int64_t len = a.len;
 
   // ---- entering state: keys 16wv + 4gq + i, columns v0 + 16t + r ---------
-  const int64_t sbase = (static_cast<int64_t>(a.n) * H + h) * KD;
+  const int64_t sbase = (static_cast<int64_t>(a.n) * H + h) * K + KD * kg;
   const int krow = 16 * wv + 4 * gq;
+  const bool rows_in = KS || 16 * wv < kw;   // this wavefront's state rows exist (K is a multiple of 16)
   // the first chunk's loads go out before the entering state is read
   const int row = 16 * wv + r;
   constexpr int gsz = GF32 ? 4 : 2;   // bytes per g element
   SeqRsrc rs;
-  rs.q = seq_rsrc(a.q + a.bos * H * KD, len * H * KD * 2);
-  rs.k = seq_rsrc(a.k + a.bos * H * KD, len * H * KD * 2);
-  rs.g = seq_rsrc(static_cast<const char *>(a.g) + a.bos * H * KD * gsz, len * H * KD * gsz);
+  rs.q = seq_rsrc(a.q + a.bos * H * K, len * H * K * 2);
+  rs.k = seq_rsrc(a.k + a.bos * H * K, len * H * K * 2);
+  rs.g = seq_rsrc(static_cast<const char *>(a.g) + a.bos * H * K * gsz, len * H * K * gsz);
   rs.v = seq_rsrc(a.v + a.bos * H * V, len * H * V * 2);
   rs.o = seq_rsrc(a.o + a.bos * H * V, len * H * V * 2);
   // byte offsets of this lane's row (chunk c_beg) inside the sequence, and
   // their per-chunk steps
   const uint32_t rowi = static_cast<uint32_t>((a.c_beg * BT + row) * H + h);
-  uint32_t oq = (rowi * KD + kq) * 2, og = (rowi * KD + kq) * gsz;
+  uint32_t oq = (rowi * K + KD * kg + kq) * 2, og = (rowi * K + KD * kg + kq) * gsz;
   uint32_t ov = (rowi * V + v0) * 2;   // row start of the V group (o uses it too)
-  const uint32_t sq = BT * H * KD * 2, sg = BT * H * KD * gsz, sv = BT * H * V * 2;
+  const uint32_t sq = BT * H * K * 2, sg = BT * H * K * gsz, sv = BT * H * V * 2;
   SegRegs buf;
-  load_chunk<true, GF32>(buf, rs, a.c_beg < a.c_end, oq, og, ov + 2 * kq, kq, vw);
+  load_chunk<true, GF32>(buf, rs, a.c_beg < a.c_end, oq, og, ov + 2 * kq, kq, kw, vw);
   f32x4 S[NVT];
   {
     // entering state: h0 for segment 0, else the fold of the earlier
@@ -487,17 +562,16 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
     // this order, so every segment gets the same bits); slots and decays are
     // loaded in batches (8, or 4 with the lo halves), so up to 8 segments
     // take one or two round trips
-    const int64_t chain = static_cast<int64_t>(a.n) * H + h;
     const int64_t eo = static_cast<int64_t>(krow) * V + v0 + r;   // this lane's element (i = 0, t = 0)
     if (a.seg == 0) {
-      const float *src = a.h0 ? a.h0 + sbase * V : nullptr;
+      const float *src = a.h0 && rows_in ? a.h0 + sbase * V : nullptr;
 #pragma unroll
       for (int t = 0; t < NVT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[t][i] = src ? src[eo + static_cast<int64_t>(i) * V + 16 * t] : 0.f;
     } else {
-      const int64_t sl0 = chain * a.P * KD * V + slot_index<NVT>(a.v0, wv, lane);
-      const float *dk = a.ws_decay + chain * a.P * KD + krow;
+      const int64_t sl0 = a.store * KD * V + slot_index<NVT>(a.v0, wv, lane);
+      const float *dk = a.ws_decay + a.store * KD + krow;
       fold_slots<NVT, false>(a, sl0, dk, S);
     }
   }
@@ -521,7 +595,7 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
     oq += sq;
     og += sg;
     ov += sv;
-    load_chunk<true, GF32>(nxt, rs, c + 1 < a.c_end, oq, og, ov + 2 * kq, kq, vw);
+    load_chunk<true, GF32>(nxt, rs, c + 1 < a.c_end, oq, og, ov + 2 * kq, kq, kw, vw);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- block-local inclusive cumsum over the 16 rows (DPP row scan) ------
@@ -642,6 +716,17 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
     }
 
     // ---- per V tile: o^T = S^T q0^T + V^T A^T, store ---------------------------
+    // With two key groups, each finishes half of the tiles: it hands the
+    // others' sums over and adds the other group's to its own.
+    constexpr int kHalfT = (NVT + 1) / 2;
+    f32x4 omine[KG == 2 ? kHalfT : 1];
+    auto store_o = [&](const f32x4 &x, int t) __attribute__((always_inline)) {
+      // rows past the sequence end fall outside rs.o and are dropped
+      const f32x8 o8 = {x[0] * a.scale, x[1] * a.scale, x[2] * a.scale, x[3] * a.scale, 0.f, 0.f, 0.f, 0.f};
+      const uint4 ob = to_bits(M::cvt(o8));
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      __builtin_amdgcn_raw_buffer_store_b64((u32x2){ob.x, ob.y}, rs.o, orow + 2 * (16 * t + 4 * gq), 0, 0);
+    };
 #pragma unroll
     for (int t = 0; t < NVT; ++t) {
       f32x4 oacc = {0.f, 0.f, 0.f, 0.f};
@@ -655,15 +740,24 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
           oacc = M::mma(va, ab[pr], oacc);
         }
       }
-      {
-        // rows past the sequence end fall outside rs.o and are dropped
-        const f32x8 o8 = {oacc[0] * a.scale, oacc[1] * a.scale, oacc[2] * a.scale, oacc[3] * a.scale,
-                          0.f, 0.f, 0.f, 0.f};
-        const uint4 ob = to_bits(M::cvt(o8));
-        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-        __builtin_amdgcn_raw_buffer_store_b64((u32x2){ob.x, ob.y}, rs.o, orow + 2 * (16 * t + 4 * gq), 0, 0);
+      if (KG == 1) {
+        store_o(oacc, t);
+      } else if ((t < kHalfT) == (kg == 0)) {
+        omine[kg == 0 ? t : t - kHalfT] = oacc;
+      } else {
+        xch[((kg * 4 + wv) * kHalfT + (kg == 0 ? t - kHalfT : t)) * 64 + lane] = oacc;
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (KG == 2) {
+      lds_barrier();  // ----------------------------------- both groups' tiles
+      // (rewritten after the next chunk's barriers 1 and 2)
+#pragma unroll
+      for (int t = 0; t < NVT; ++t)
+        if ((t < kHalfT) == (kg == 0)) {
+          const int m = kg == 0 ? t : t - kHalfT;
+          store_o(omine[m] + xch[(((1 - kg) * 4 + wv) * kHalfT + m) * 64 + lane], t);
+        }
     }
 
     // ---- S <- 2^(G_last) S + k^^T V for the state rows of this wavefront ------
@@ -688,14 +782,13 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
   if (c < a.c_end) chunk_step(buf, buf2, c);
 
   // ---- final state of the sequence -----------------------------------------
-  if (a.seg == a.P - 1 && a.ht) {
+  if (a.last && a.ht && rows_in) {
     if (a.seg > 0) {
       // the lo halves of the earlier segments' states, folded as the hi
       // halves were and carried through this segment's decay
-      const int64_t chain = static_cast<int64_t>(a.n) * H + h;
       f32x4 lo[NVT];
-      fold_slots<NVT, true>(a, chain * a.P * KD * V + slot_index<NVT>(a.v0, wv, lane),
-                            a.ws_decay + chain * a.P * KD + krow, lo);
+      fold_slots<NVT, true>(a, a.store * KD * V + slot_index<NVT>(a.v0, wv, lane), a.ws_decay + a.store * KD + krow,
+                            lo);
 #pragma unroll
       for (int t = 0; t < NVT; ++t)
 #pragma unroll
@@ -708,41 +801,36 @@ __device__ __forceinline__ void segment_loop(SmemA &sm, const ChunkArgs &a, cons
   }
 }
 
-template <int DT, bool GF32, int NVT>
-__global__ __launch_bounds__(256, SSLA_GC_SEG_WAVES) void gla_chunk_segment_kernel(
+template <int DT, bool GF32, int NVT, int KS, int KG>
+__global__ __launch_bounds__(256 * KG, SSLA_GC_SEG_WAVES) void gla_chunk_segment_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
     const uint16_t *__restrict__ v, const void *__restrict__ g,
-    const int64_t *__restrict__ cu_seqlens, int n_seq, int64_t T, int H, int V, float scale,
-    const float *__restrict__ h0, uint16_t *__restrict__ o, float *__restrict__ ht, int P,
+    const int64_t *__restrict__ cu_seqlens, int n_seq, int64_t T, int H, int K, int V, float scale,
+    const float *__restrict__ h0, uint16_t *__restrict__ o, float *__restrict__ ht, int per, int slots, int even,
     const uint16_t *__restrict__ ws_state, const uint16_t *__restrict__ ws_lo, const float *__restrict__ ws_decay) {
-  __shared__ SmemA sm;
-  const int nvg = V / (16 * NVT);
-  // block -> (segment, sequence, head, V group), segment-major: consecutive
-  // blocks go to different XCDs, so each XCD runs every segment index in
-  // equal shares (with the segment fastest, XCD s would run all of segment
-  // s, and the one holding the last segments -- the longest folds -- would
-  // carry all of their slot traffic alone: 54.8 against 48.1 us at C2)
-  const int64_t chains = static_cast<int64_t>(n_seq) * H * nvg;
-  int64_t b = blockIdx.x;
+  __shared__ SmemA sm[KG];
+  __shared__ f32x4 xch[KG == 2 ? 8 * ((NVT + 1) / 2) * 64 : 1];
+  SegPlace p;
+  if (!segment_place<false>(cu_seqlens, n_seq, T, H, per, V / (16 * NVT), slots, even, p)) return;   // workgroup-uniform
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = KG == 2 ? wid >> 2 : 0;
   ChunkArgs a;
-  a.P = P;
-  a.seg = static_cast<int>(b / chains);
-  b %= chains;
-  const int vg = static_cast<int>(b % nvg);
-  b /= nvg;
-  a.h = static_cast<int>(b % H);
-  a.n = static_cast<int>(b / H);
+  a.n = p.n;
+  a.h = p.h;
+  a.seg = p.seg;
+  a.last = p.seg == p.nseg - 1;
   a.q = q; a.k = k; a.v = v; a.g = g; a.h0 = h0; a.o = o; a.ht = ht;
   a.ws_state = ws_state;
   a.ws_lo = ws_lo;
   a.ws_decay = ws_decay;
-  a.H = H; a.V = V; a.scale = scale;
-  a.v0 = vg * 16 * NVT;
-  a.bos = min(max(cu_seqlens[a.n], (int64_t)0), T);
-  const int64_t eos = min(max(cu_seqlens[a.n + 1], a.bos), T);
-  a.len = eos - a.bos;
-  segment_range(static_cast<int>((a.len + BT - 1) / BT), P, a.seg, a.c_beg, a.c_end);
-  segment_loop<DT, GF32, NVT>(sm, a, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+  a.store = store_slot(p.first - p.n, p, H, KG, kg);
+  a.slot_step = H * KG;
+  a.H = H; a.K = K; a.V = V; a.scale = scale;
+  a.v0 = p.in * 16 * NVT;
+  a.bos = p.bos;
+  a.len = p.len;
+  a.c_beg = p.seg * per;
+  a.c_end = static_cast<int>(min(static_cast<int64_t>(a.c_beg) + per, (p.len + BT - 1) / BT));
+  segment_loop<DT, GF32, NVT, KS, KG>(sm[kg], xch, a, wid & 3, kg, threadIdx.x & 63);
 }
 
 // ----------------------------------------------------------- state pass --
@@ -754,62 +842,60 @@ struct __align__(16) SmemS {
   float fac[4][2][KD];     // per-wavefront per-key: G_last - E_I-1, 2^G_last
 };
 
-// State-only walk over segment seg (< P - 1) of one (sequence, head, V
-// group):  S <- 2^(G_last) S + (k 2^(G_last - G))^T v  per chunk, from h0
-// for segment 0 and from zero otherwise.  Writes the workspace slot and,
-// for seg >= 1, the segment's total log2 decay.
-template <int DT, bool GF32, int NVT>
+// State-only walk over one segment, not its sequence's last, of one
+// (sequence, head, key group, V group):  S <- 2^(G_last) S + (k 2^(G_last -
+// G))^T v  per chunk, from h0 for segment 0 and from zero otherwise.  Writes
+// the workspace slot and, for seg >= 1, the segment's total log2 decay.
+template <int DT, bool GF32, int NVT, int KS>
 __global__ __launch_bounds__(256, SSLA_GC_STATE_WAVES) void gla_chunk_state_kernel(
     const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, const void *__restrict__ g,
-    const int64_t *__restrict__ cu_seqlens, int n_seq, int64_t T, int H, int V,
-    const float *__restrict__ h0, int P, uint16_t *__restrict__ ws_state, uint16_t *__restrict__ ws_lo,
+    const int64_t *__restrict__ cu_seqlens, int n_seq, int64_t T, int H, int K_, int V,
+    const float *__restrict__ h0, int per, int slots, int even, int KG, uint16_t *__restrict__ ws_state, uint16_t *__restrict__ ws_lo,
     float *__restrict__ ws_decay) {
   typedef Mfma<DT> M;
   typedef typename M::Vec MV;
   __shared__ SmemS sm;
+  const int K = KS ? KS : K_;
   const int nvg = V / (16 * NVT);
-  int64_t b = blockIdx.x;
-  const int seg = static_cast<int>(b % (P - 1));
-  b /= (P - 1);
-  const int vg = static_cast<int>(b % nvg);
-  b /= nvg;
-  const int h = static_cast<int>(b % H);
-  const int n = static_cast<int>(b / H);
-  const int v0 = vg * 16 * NVT;
+  SegPlace p;
+  if (!segment_place<true>(cu_seqlens, n_seq, T, H, per, nvg * KG, slots, even, p)) return;   // workgroup-uniform
+  if (p.seg == p.nseg - 1) return;
+  const int seg = p.seg, h = p.h, n = p.n;
+  const int kg = p.in / nvg;
+  const int v0 = p.in % nvg * 16 * NVT;
   const int vw = 16 * NVT;
+  const int kw = KS ? KD : min(KD, K - KD * kg);   // keys of this group
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, gq = lane >> 4, kq = 8 * gq;
   const int krow = 16 * wv + 4 * gq;
   const int row = 16 * wv + r;
 
-  const int64_t sbase = (static_cast<int64_t>(n) * H + h) * KD;
+  const int64_t sbase = (static_cast<int64_t>(n) * H + h) * K + KD * kg;
   f32x4 S[NVT];
 #pragma unroll
   for (int t = 0; t < NVT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      S[t][i] = (seg == 0 && h0) ? h0[(sbase + krow + i) * V + v0 + 16 * t + r] : 0.f;
+      S[t][i] = (seg == 0 && h0 && (KS || 16 * wv < kw)) ? h0[(sbase + krow + i) * V + v0 + 16 * t + r] : 0.f;
 
-  const int64_t bos = min(max(cu_seqlens[n], (int64_t)0), T);
-  const int64_t eos = min(max(cu_seqlens[n + 1], bos), T);
-  const int64_t len = eos - bos;
-  int c_beg, c_end;
-  segment_range(static_cast<int>((len + BT - 1) / BT), P, seg, c_beg, c_end);
+  const int64_t bos = p.bos, len = p.len;
+  const int c_beg = seg * per, c_end = c_beg + per;   // whole: a segment follows
   float dsum = 0.f;   // lane = key
 
   constexpr int gsz = GF32 ? 4 : 2;
   SeqRsrc rs;
-  rs.k = seq_rsrc(k + bos * H * KD, len * H * KD * 2);
-  rs.g = seq_rsrc(static_cast<const char *>(g) + bos * H * KD * gsz, len * H * KD * gsz);
+  rs.k = seq_rsrc(k + bos * H * K, len * H * K * 2);
+  rs.g = seq_rsrc(static_cast<const char *>(g) + bos * H * K * gsz, len * H * K * gsz);
   rs.v = seq_rsrc(v + bos * H * V, len * H * V * 2);
-  LineOffs lo = line_offs(c_beg, wv, lane, H, h, V, v0, gsz);
-  const uint32_t sq = BT * H * KD * 2, sg = BT * H * KD * gsz, sv = BT * H * V * 2;
+  LineOffs lo = line_offs(c_beg, wv, lane, H, h, K, KD * kg, V, v0, gsz);
+  const uint32_t sq = BT * H * K * 2, sg = BT * H * K * gsz, sv = BT * H * V * 2;
+  const bool k_ok = KS || 8 * (lane & 7) < kw, g_ok = KS || (GF32 ? 4 * (lane & 15) : 8 * (lane & 7)) < kw;
   const bool vcol_ok = 8 * (lane & 7) < vw;
   // Loads run one chunk ahead over two register sets used in turn (the loop
   // is unrolled by two, so no copies).
   LineRegs buf, buf2;
-  load_lines<false, GF32>(buf, rs, c_beg < c_end, lo, H, V, vcol_ok);
+  load_lines<false, GF32>(buf, rs, c_beg < c_end, lo, H, K, V, k_ok, g_ok, vcol_ok);
   auto chunk_step = [&](LineRegs &cl, LineRegs &nxt, const int c) __attribute__((always_inline)) {
     const int par = (c - c_beg) & 1;
     ChunkRegs cur;
@@ -819,7 +905,7 @@ __global__ __launch_bounds__(256, SSLA_GC_STATE_WAVES) void gla_chunk_state_kern
     lo.a16 += sq;
     lo.g += sg;
     lo.v += sv;
-    load_lines<false, GF32>(nxt, rs, c + 1 < c_end, lo, H, V, vcol_ok);
+    load_lines<false, GF32>(nxt, rs, c + 1 < c_end, lo, H, K, V, k_ok, g_ok, vcol_ok);
     __builtin_amdgcn_sched_barrier(0);
     f32x8 gs[2];
     unpack_gates<DT, GF32>(cur, gs);
@@ -874,7 +960,7 @@ __global__ __launch_bounds__(256, SSLA_GC_STATE_WAVES) void gla_chunk_state_kern
   }
   if (c < c_end) chunk_step(buf, buf2, c);
 
-  const int64_t slot = (static_cast<int64_t>(n) * H + h) * P + seg;
+  const int64_t slot = store_slot(p.first + seg, p, H, KG, kg);
   const int64_t so = slot * KD * V + slot_index<NVT>(v0, wv, lane);
 #pragma unroll
   for (int t = 0; t < NVT; ++t) {
@@ -924,98 +1010,113 @@ inline int pick_nvt(int V) {
   return 1;
 }
 
-// Segments per sequence: about two workgroups per CU (256 CUs), at least
-// two chunks per segment on average, at most 64 segments, and a count that
-// leaves no segment empty (P = ceil(chunks / ceil(chunks / P))).
-inline int pick_segments(int n_seq, int64_t T, int H, int V) {
+// Segments: about two workgroups per CU (256 CUs), at least two chunks per
+// segment, at most 64 segments per average sequence, and for sequences of
+// equal length a count that leaves no segment empty.  `per` chunks each; a
+// batch whose average sequence is one segment of fewer than 16 chunks is not
+// cut at all (per = 0): the state pass's launch would cost about what its
+// longer sequences' walks do.
+struct Segments {
+  int P, per;      // segments of an average sequence, chunks of a segment (0: uncut)
+  int64_t stores;  // workspace slots per (head, key group)
+};
+inline Segments pick_segments(int n_seq, int64_t T, int H, int V) {
   const int nvg = V / (16 * pick_nvt(V));
   const int64_t chains = static_cast<int64_t>(n_seq) * H * nvg;
-  if (chains <= 0) return 1;
+  if (chains <= 0) return {1, 0, 0};
   int64_t p = (512 + chains - 1) / chains;
   const int64_t avg_chunks = (T / std::max<int64_t>(n_seq, 1) + BT - 1) / BT;
   p = std::min<int64_t>(p, std::max<int64_t>(1, avg_chunks / 2));
   p = std::min<int64_t>(p, 64);
   p = std::max<int64_t>(p, 1);
+  int64_t per = std::max<int64_t>(avg_chunks, 1);
   if (avg_chunks > 0) {
-    const int64_t per = (avg_chunks + p - 1) / p;
+    per = (avg_chunks + p - 1) / p;
     p = (avg_chunks + per - 1) / per;
   }
-  return static_cast<int>(p);
+  // one sequence of T rows is exactly T / n_seq long: nothing to balance
+  if (p == 1 && (per < 16 || n_seq == 1)) return {1, 0, 0};
+  // every stored segment is whole and has a successor: at most (T - 1) / unit
+  const int64_t stores = std::max<int64_t>(p > 1 ? n_seq * p : 0, (T - 1) / (BT * per));
+  return {static_cast<int>(p), static_cast<int>(per), stores};
 }
 
-inline size_t workspace_bytes_for(int n_seq, int H, int V, int P) {
-  if (P <= 1) return 0;
-  const size_t slots = static_cast<size_t>(n_seq) * H * P;
+inline size_t workspace_bytes_for(const Segments &sg, int H, int KG, int V) {
+  const size_t slots = static_cast<size_t>(sg.stores) * H * KG;
   return 2 * slots * KD * V * sizeof(uint16_t) + slots * KD * sizeof(float);   // hi, lo, decays
 }
 
-template <int DT, bool GF32, int NVT>
-int launch_nvt(const void *q, const void *k, const void *v, const void *g, const int64_t *cu, int n_seq,
-               int64_t T, int H, int V, float scale, const float *h0, void *o, float *ht, int P,
-               uint16_t *ws_state, uint16_t *ws_lo, float *ws_decay, hipStream_t st) {
-  const int nvg = V / (16 * NVT);
-  const int64_t blocks_a = static_cast<int64_t>(n_seq) * H * nvg * P;
-  if (blocks_a > 0x7fffffff) {
+struct FwdArgs {
+  const void *q, *k, *v, *g;
+  const int64_t *cu;
+  int n_seq;
+  int64_t T;
+  int H, K, V;
+  float scale;
+  const float *h0;
+  void *o;
+  float *ht;
+  Segments sg;
+  uint16_t *ws_state, *ws_lo;
+  float *ws_decay;
+  hipStream_t st;
+};
+
+template <int DT, bool GF32, int NVT, int KS, int KG>
+int launch_kg(const FwdArgs &f) {
+  const int nvg = f.V / (16 * NVT);
+  // an uncut batch: a segment longer than any sequence
+  const int per = f.sg.per ? f.sg.per : static_cast<int>(std::min<int64_t>(f.T / BT + 1, int64_t{1} << 24));
+  const int64_t slots = f.T / (static_cast<int64_t>(BT) * per) + f.n_seq + 1;
+  const int64_t items = (slots * f.H + 7) / 8 * 8;   // (segment_place deals them in eights)
+  const int64_t stores = f.sg.per ? (f.T - 1) / (static_cast<int64_t>(BT) * per) : 0;
+  const int64_t unit = static_cast<int64_t>(BT) * per;
+  const int even = f.sg.per && f.T % (f.n_seq * unit) == 0 ? static_cast<int>(f.T / (f.n_seq * unit)) : 0;
+  if (items * nvg * KG > 0x7fffffff) {
     set_error("gla_chunk_fwd: too many workgroups");
     return SSLA_ERR_UNSUPPORTED;
   }
-  const uint16_t *q16 = static_cast<const uint16_t *>(q);
-  uint16_t *o16 = static_cast<uint16_t *>(o);
-  if (P > 1) {
-    const int64_t blocks_s = static_cast<int64_t>(n_seq) * H * nvg * (P - 1);
-    hipLaunchKernelGGL((gla_chunk_state_kernel<DT, GF32, NVT>), dim3(static_cast<unsigned>(blocks_s)),
-                       dim3(256), 0, st, static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
-                       g, cu, n_seq, T, H, V, h0, P, ws_state, ws_lo, ws_decay);
-  }
-  hipLaunchKernelGGL((gla_chunk_segment_kernel<DT, GF32, NVT>), dim3(static_cast<unsigned>(blocks_a)),
-                     dim3(256), 0, st, q16, static_cast<const uint16_t *>(k),
-                     static_cast<const uint16_t *>(v), g, cu, n_seq, T, H, V, scale, h0, o16, ht, P,
-                     ws_state, ws_lo, ws_decay);
+  const uint16_t *k16 = static_cast<const uint16_t *>(f.k), *v16 = static_cast<const uint16_t *>(f.v);
+  if (stores > 0)
+    hipLaunchKernelGGL((gla_chunk_state_kernel<DT, GF32, NVT, KS>),
+                       dim3(static_cast<unsigned>((stores * f.H + 7) / 8 * 8 * nvg * KG)), dim3(256), 0, f.st, k16, v16,
+                       f.g, f.cu, f.n_seq, f.T, f.H, f.K, f.V, f.h0, per, static_cast<int>(stores), even, KG, f.ws_state,
+                       f.ws_lo, f.ws_decay);
+  hipLaunchKernelGGL((gla_chunk_segment_kernel<DT, GF32, NVT, KS, KG>), dim3(static_cast<unsigned>(items * nvg)),
+                     dim3(256 * KG), 0, f.st, static_cast<const uint16_t *>(f.q), k16, v16, f.g, f.cu, f.n_seq, f.T,
+                     f.H, f.K, f.V, f.scale, f.h0, static_cast<uint16_t *>(f.o), f.ht, per, static_cast<int>(slots),
+                     even, f.ws_state, f.ws_lo, f.ws_decay);
   return launch_status("gla_chunk_fwd");
 }
 
+template <int DT, bool GF32, int NVT>
+int launch_nvt(const FwdArgs &f) {
+  if (f.K == KD) return launch_kg<DT, GF32, NVT, KD, 1>(f);
+  return f.K < KD ? launch_kg<DT, GF32, NVT, 0, 1>(f) : launch_kg<DT, GF32, NVT, 0, 2>(f);
+}
+
 template <int DT, bool GF32>
-int launch_chunk(const void *q, const void *k, const void *v, const void *g, const int64_t *cu, int n_seq,
-                 int64_t T, int H, int V, float scale, const float *h0, void *o, float *ht, int P,
-                 uint16_t *ws_state, uint16_t *ws_lo, float *ws_decay, hipStream_t st) {
-  switch (pick_nvt(V)) {
-    case 4: return launch_nvt<DT, GF32, 4>(q, k, v, g, cu, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
-    case 3: return launch_nvt<DT, GF32, 3>(q, k, v, g, cu, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
-    case 2: return launch_nvt<DT, GF32, 2>(q, k, v, g, cu, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
-    default: return launch_nvt<DT, GF32, 1>(q, k, v, g, cu, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
+int launch_chunk(const FwdArgs &f) {
+  switch (pick_nvt(f.V)) {
+    case 4: return launch_nvt<DT, GF32, 4>(f);
+    case 3: return launch_nvt<DT, GF32, 3>(f);
+    case 2: return launch_nvt<DT, GF32, 2>(f);
+    default: return launch_nvt<DT, GF32, 1>(f);
   }
 }
 
-}  // namespace
-}  // namespace ssla
-
-extern "C" size_t ssla_gla_chunk_workspace_size(int n_seq, int64_t T, int H, int K, int V) {
-  if (n_seq <= 0 || T < 0 || H <= 0 || K != ssla::KD || V <= 0 || V % 16 != 0) return 0;
-  return ssla::workspace_bytes_for(n_seq, H, V, ssla::pick_segments(n_seq, T, H, V));
-}
-
-extern "C" int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v, const void *g,
-                                  int g_dtype, const int64_t *cu_seqlens, int n_seq, int64_t T,
-                                  int H, int K, int V, float scale, const float *h0, void *o,
-                                  float *ht, int dtype, void *workspace, size_t workspace_bytes,
-                                  void *stream) {
-  using namespace ssla;
-  clear_error();
-  SSLA_CHECK_ARG(n_seq >= 0 && T >= 0 && H > 0 && K > 0 && V > 0,
-                 "gla_chunk_fwd: bad sizes n_seq=%d T=%lld H=%d K=%d V=%d", n_seq, (long long)T, H, K, V);
-  if (K != KD || V % 16 != 0 || V > 256) {
-    set_error("gla_chunk_fwd: needs K == 64 and V a multiple of 16 up to 256 (K=%d V=%d)", K, V);
-    return SSLA_ERR_UNSUPPORTED;
-  }
+// The forward for K a multiple of 16 up to 128 (arguments checked but for K).
+int chunk_fwd(const void *q, const void *k, const void *v, const void *g, int g_dtype, const int64_t *cu_seqlens,
+              int n_seq, int64_t T, int H, int K, int V, float scale, const float *h0, void *o, float *ht, int dtype,
+              void *workspace, size_t workspace_bytes, void *stream) {
   if (n_seq == 0) return SSLA_OK;
   SSLA_CHECK_ARG(cu_seqlens != nullptr, "gla_chunk_fwd: cu_seqlens is NULL");
-  // kernels address a sequence with 32-bit byte offsets
   {
     // Each sequence's rows are addressed through buffer resources with
     // 32-bit byte offsets: a sequence must stay below 2^31 bytes per tensor.
     // Only a batch whose whole tensor reaches that size can hold such a
     // sequence; then the lengths are read back (one host synchronisation).
-    const int64_t row_bytes = static_cast<int64_t>(H) * std::max(K, V) * 4;
+    const int64_t row_bytes = static_cast<int64_t>(H) * std::max({K, V, KD}) * 4;
     const int64_t max_rows = ((int64_t{1} << 31) - 1) / row_bytes;
     if (T > max_rows) {
       const int st = check_seq_lengths(cu_seqlens, n_seq, T, max_rows, static_cast<hipStream_t>(stream));
@@ -1033,26 +1134,77 @@ extern "C" int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v, c
     set_error("gla_chunk_fwd: g dtype %d must be fp32 or the dtype of q", g_dtype);
     return SSLA_ERR_DTYPE;
   }
-  const int P = pick_segments(n_seq, T, H, V);
-  const size_t need = workspace_bytes_for(n_seq, H, V, P);
+  const int KG = K > KD ? 2 : 1;
+  FwdArgs f = {q, k, v, g, cu_seqlens, n_seq, T, H, K, V, scale, h0, o, ht, pick_segments(n_seq, T, H, V), nullptr,
+               nullptr, nullptr, static_cast<hipStream_t>(stream)};
+  size_t need = workspace_bytes_for(f.sg, H, KG, V);
+  if (f.sg.P == 1 && (workspace == nullptr || workspace_bytes < need)) {
+    f.sg = {1, 0, 0};   // cut only to balance a ragged batch: runs uncut without its workspace
+    need = 0;
+  }
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_error("gla_chunk_fwd: workspace of %zu bytes needed (ssla_gla_chunk_workspace_size), %zu given",
               need, workspace_bytes);
     return SSLA_ERR_WORKSPACE;
   }
   SSLA_CHECK_ARG(need == 0 || aligned(workspace, 16), "gla_chunk_fwd: workspace must be 16-byte aligned");
-  uint16_t *ws_state = static_cast<uint16_t *>(workspace);
-  // slots are K*V*2 bytes (a multiple of 2048), so lo and the decays stay 16-byte aligned
-  const size_t slot_elems = static_cast<size_t>(n_seq) * H * P * KD * V;
-  uint16_t *ws_lo = need ? ws_state + slot_elems : nullptr;
-  float *ws_decay = need ? reinterpret_cast<float *>(ws_state + 2 * slot_elems) : nullptr;
-  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (need) {
+    // slots are 64 V 2 bytes (a multiple of 2048), so lo and the decays stay 16-byte aligned
+    const size_t slot_elems = static_cast<size_t>(f.sg.stores) * H * KG * KD * V;
+    f.ws_state = static_cast<uint16_t *>(workspace);
+    f.ws_lo = f.ws_state + slot_elems;
+    f.ws_decay = reinterpret_cast<float *>(f.ws_state + 2 * slot_elems);
+  }
   const bool gf32 = g_dtype == SSLA_F32;
-  if (dtype == SSLA_BF16)
-    return gf32 ? launch_chunk<SSLA_BF16, true>(q, k, v, g, cu_seqlens, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st)
-                : launch_chunk<SSLA_BF16, false>(q, k, v, g, cu_seqlens, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
-  return gf32 ? launch_chunk<SSLA_F16, true>(q, k, v, g, cu_seqlens, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st)
-              : launch_chunk<SSLA_F16, false>(q, k, v, g, cu_seqlens, n_seq, T, H, V, scale, h0, o, ht, P, ws_state, ws_lo, ws_decay, st);
+  if (dtype == SSLA_BF16) return gf32 ? launch_chunk<SSLA_BF16, true>(f) : launch_chunk<SSLA_BF16, false>(f);
+  return gf32 ? launch_chunk<SSLA_F16, true>(f) : launch_chunk<SSLA_F16, false>(f);
+}
+
+}  // namespace
+}  // namespace ssla
+
+extern "C" size_t ssla_gla_chunk_workspace_size(int n_seq, int64_t T, int H, int K, int V) {
+  if (n_seq <= 0 || T < 0 || H <= 0 || K != ssla::KD || V <= 0 || V % 16 != 0) return 0;
+  return ssla::workspace_bytes_for(ssla::pick_segments(n_seq, T, H, V), H, 1, V);
+}
+
+extern "C" size_t ssla_gla_chunk_wide_workspace_size(int n_seq, int64_t T, int H, int K, int V) {
+  if (n_seq <= 0 || T < 0 || H <= 0 || K <= 0 || K % 16 != 0 || K > 2 * ssla::KD || V <= 0 || V % 16 != 0) return 0;
+  return ssla::workspace_bytes_for(ssla::pick_segments(n_seq, T, H, V), H, K > ssla::KD ? 2 : 1, V);
+}
+
+extern "C" int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v, const void *g,
+                                  int g_dtype, const int64_t *cu_seqlens, int n_seq, int64_t T,
+                                  int H, int K, int V, float scale, const float *h0, void *o,
+                                  float *ht, int dtype, void *workspace, size_t workspace_bytes,
+                                  void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(n_seq >= 0 && T >= 0 && H > 0 && K > 0 && V > 0,
+                 "gla_chunk_fwd: bad sizes n_seq=%d T=%lld H=%d K=%d V=%d", n_seq, (long long)T, H, K, V);
+  if (K != KD || V % 16 != 0 || V > 256) {
+    set_error("gla_chunk_fwd: needs K == 64 and V a multiple of 16 up to 256 (K=%d V=%d)", K, V);
+    return SSLA_ERR_UNSUPPORTED;
+  }
+  return chunk_fwd(q, k, v, g, g_dtype, cu_seqlens, n_seq, T, H, K, V, scale, h0, o, ht, dtype, workspace,
+                   workspace_bytes, stream);
+}
+
+extern "C" int ssla_gla_chunk_fwd_wide(const void *q, const void *k, const void *v, const void *g,
+                                       int g_dtype, const int64_t *cu_seqlens, int n_seq, int64_t T,
+                                       int H, int K, int V, float scale, const float *h0, void *o,
+                                       float *ht, int dtype, void *workspace, size_t workspace_bytes,
+                                       void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(n_seq >= 0 && T >= 0 && H > 0 && K > 0 && V > 0,
+                 "gla_chunk_fwd_wide: bad sizes n_seq=%d T=%lld H=%d K=%d V=%d", n_seq, (long long)T, H, K, V);
+  if (K % 16 != 0 || K > 2 * KD || V % 16 != 0 || V > 256) {
+    set_error("gla_chunk_fwd_wide: needs K a multiple of 16 up to 128 and V up to 256 (K=%d V=%d)", K, V);
+    return SSLA_ERR_UNSUPPORTED;
+  }
+  return chunk_fwd(q, k, v, g, g_dtype, cu_seqlens, n_seq, T, H, K, V, scale, h0, o, ht, dtype, workspace,
+                   workspace_bytes, stream);
 }
 
 namespace ssla {
@@ -1112,7 +1264,8 @@ extern "C" int ssla_gla_chunk_fwd_noalloc(const void *q, const void *k, const vo
                                           float *ht, int dtype, void *stream) {
   using namespace ssla;
   clear_error();
-  const size_t need = ssla_gla_chunk_workspace_size(n_seq, T, H, K, V);
+  size_t need = ssla_gla_chunk_workspace_size(n_seq, T, H, K, V);
+  if (need > kNoallocScratchBytes && pick_segments(n_seq, T, H, V).P == 1) need = 0;   // runs uncut
   if (need > kNoallocScratchBytes) {
     set_error("gla_chunk_fwd_noalloc: this shape needs %zu bytes of workspace, the static scratch holds %zu "
               "(call ssla_gla_chunk_fwd with a workspace)", need, kNoallocScratchBytes);

@@ -34,7 +34,7 @@
 // j = i term of A, and the state term of dk against the same term of the
 // chunk-total decay's gradient): with strongly decaying gates dg is small
 // next to q dq and k dk, and those terms would leave only their rounding.
-#include "common.h"
+#include "seq_slots.h"
 
 namespace ssla {
 namespace {
@@ -295,39 +295,23 @@ __device__ __forceinline__ void store4(float *row, int c, int C, const f32x4 &x)
   }
 }
 
-// Workspace slot of chunk c of sequence n: bos / 64 + n + c, distinct for
-// every chunk of non-overlapping sequences (at most T / 64 + n_seq + 1).
+// A chunk's workspace slot is its slot in units of 64 rows (seq_slots.h).
 struct ChunkAt {
-  int n, nc, c;     // sequence, rows, chunk of the sequence
+  int nc;           // rows
   int64_t t0;       // first row
   bool first, last; // of its sequence
 };
 
-// The chunk of a slot (false: none).  Every wavefront searches the sequence
-// starts 64 probes per round trip.
+// The chunk of a slot (false: none).
 __device__ __forceinline__ bool chunk_of_slot(const int64_t *cu, int n_seq, int64_t T, int64_t slot, ChunkAt &at) {
-  const int lane = threadIdx.x & 63;
-  int lo = 0, hi = n_seq;
-  while (hi - lo > 1) {
-    const int step = (hi - lo + 63) >> 6;
-    const int64_t i = lo + static_cast<int64_t>(lane) * step;
-    const bool in = i < hi && min(max(cu[min(i, static_cast<int64_t>(hi - 1))], (int64_t)0), T) / kC + i <= slot;
-    const int cnt = __popcll(__ballot(in));
-    if (cnt == 0) return false;
-    lo += (cnt - 1) * step;
-    hi = min(hi, lo + step);
-  }
-  int64_t bos, eos;
-  seq_bounds(cu, lo, T, bos, eos);
-  const int64_t c = slot - (bos / kC + lo);
-  const int64_t t0 = bos + c * kC;
-  if (c < 0 || t0 >= eos) return false;
-  at.n = lo;
-  at.c = static_cast<int>(c);
-  at.t0 = t0;
-  at.nc = static_cast<int>(min(static_cast<int64_t>(kC), eos - t0));
-  at.first = c == 0;
-  at.last = t0 + kC >= eos;
+  int n;
+  int64_t bos, eos, first;
+  if (!seq_of_slot(cu, n_seq, T, kC, slot, n, bos, eos, first)) return false;
+  at.t0 = bos + (slot - first) * kC;
+  if (at.t0 >= eos) return false;
+  at.nc = static_cast<int>(min(static_cast<int64_t>(kC), eos - at.t0));
+  at.first = slot == first;
+  at.last = at.t0 + kC >= eos;
   return true;
 }
 

@@ -10,10 +10,11 @@ Drop-in for the reference's GLA API (haohq19/ssla ``ops/gla``):
   (reference ops/gla/naive.py:50-111).
 
 They run hand-written gfx950 kernels through libssla_amd.so; there is no
-CPU or Triton fallback.  The chunk kernels work on 64 keys: other key
-widths (multiples of 16 up to 256) run as groups of 64 keys, the last one
-zero-padded -- the decay is per key, so each key group is an independent
-GLA whose outputs add up (o = sum of the groups' o, ht = the groups' rows).
+CPU or Triton fallback.  The 16-bit forward takes key widths up to 128 (in
+multiples of 16), the fp32 forward and both backwards 64 keys: wider keys (up
+to 256) run as groups -- the decay is per key, so each key group is an
+independent GLA whose outputs add up (o = sum of the groups' o, ht = the
+groups' rows).
 ``chunk_gla`` is differentiable (:class:`ChunkGLAFunction`, backward
 ``ssla_gla_chunk_bwd`` / ``ssla_gla_chunk_f32_bwd``, run in groups of 64
 keys by 64 value columns) for the shapes the chunk kernels take; fp32
@@ -34,12 +35,13 @@ __all__ = ["chunk_gla", "ChunkGLAFunction", "fused_recurrent_gla", "fused_recurr
            "chunk_kernel_supports", "chunk_backward_supports"]
 
 
-KD = 64   # keys of one chunk-kernel call
+KD = 64    # keys of one fp32 forward or one backward call
+KF = 128   # keys of one 16-bit forward call
 
 
 def chunk_kernel_supports(q: torch.Tensor, v: torch.Tensor) -> bool:
     """True when the chunk kernels handle this dtype/shape: bf16/fp16 with K
-    a multiple of 16 up to 256 (run in groups of 64 keys) and V a multiple
+    a multiple of 16 up to 256 (run in groups of 128 keys) and V a multiple
     of 16 up to 256 (the fused MFMA kernels), or fp32 with K and V up to
     256 (the fp32 chunk kernels, ``ssla_gla_chunk_f32_*``)."""
     K, V = q.shape[-1], v.shape[-1]
@@ -123,7 +125,7 @@ def chunk_gla(
     reference (``torch.empty_like``).
 
     bf16/fp16 inputs with K a multiple of 16 up to 256 run the fused MFMA
-    chunk kernels (in groups of 64 keys); fp32 inputs run the fp32 chunk
+    chunk kernels (in groups of 128 keys); fp32 inputs run the fp32 chunk
     kernels (chunks of 64 rows, fp32 products); other shapes run the fused
     recurrent kernel (same math, fp32 state, serial over time).
     """
@@ -156,24 +158,28 @@ def _chunk_fwd(q, k, v, g, cu, scale, h0, output_final_state):
         o = torch.empty_like(v)
         ht = torch.empty(N, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
         return _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
-    if K == KD or (q.dtype == torch.float32 and K <= KD):
+    step = KD if q.dtype == torch.float32 else KF
+    if K <= step:
         return _chunk_call(q, k, v, g, cu, scale, h0, output_final_state)
     # key groups: o adds up over the groups (in fp32, rounded once more for
     # 16-bit inputs), ht stacks their key rows
     os, hts = [], []
-    for s, w in _key_groups(K):
-        o_i, ht_i = _chunk_call(_keys_of(q, s, w, 2), _keys_of(k, s, w, 2), v, _keys_of(g, s, w, 2), cu, scale,
-                                _keys_of(h0, s, w, 2), output_final_state)
+    for s in range(0, K, step):
+        w = min(step, K - s)
+        q_i, k_i, g_i = (t.narrow(2, s, w).contiguous() for t in (q, k, g))
+        h0_i = None if h0 is None else h0.narrow(2, s, w).contiguous()
+        o_i, ht_i = _chunk_call(q_i, k_i, v, g_i, cu, scale, h0_i, output_final_state)
         os.append(o_i)
         if ht_i is not None:
-            hts.append(ht_i[:, :, :w])
+            hts.append(ht_i)
     o = os[0] if len(os) == 1 else torch.stack(os).float().sum(0).to(v.dtype)
     return o, (torch.cat(hts, dim=2) if output_final_state else None)
 
 
 def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
-    """One ssla_gla_chunk_fwd call (K == KD), or one ssla_gla_chunk_f32_fwd_ws
-    call for fp32 inputs (K <= KD)."""
+    """One ssla_gla_chunk_fwd (K == 64) or ssla_gla_chunk_fwd_wide call (other
+    K up to 128), or one ssla_gla_chunk_f32_fwd_ws call for fp32 inputs (K up
+    to 64)."""
     T, H, K = q.shape
     V = v.shape[-1]
     N = cu.numel() - 1
@@ -188,9 +194,11 @@ def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
                                            ws_bytes, _lib.stream_of(q))
         _lib.check(st, "ssla_gla_chunk_f32_fwd_ws")
         return o, ht
-    ws_bytes = lib.ssla_gla_chunk_workspace_size(N, T, H, K, V)
+    size, fwd = ((lib.ssla_gla_chunk_workspace_size, lib.ssla_gla_chunk_fwd) if K == KD else
+                 (lib.ssla_gla_chunk_wide_workspace_size, lib.ssla_gla_chunk_fwd_wide))
+    ws_bytes = size(N, T, H, K, V)
     ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
-    st = lib.ssla_gla_chunk_fwd(
+    st = fwd(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.DTYPE_CODE[g.dtype],
         _lib.ptr(cu), N, T, H, K, V, float(scale), _lib.ptr(h0), _lib.ptr(o), _lib.ptr(ht),
         _lib.DTYPE_CODE[q.dtype], _lib.ptr(ws), ws_bytes, _lib.stream_of(q))

@@ -1,0 +1,73 @@
+"""The 16-bit chunk forward's segments and key widths where their indexing
+can go wrong, against the fp64 recurrence in the bands of test_gpu_gla.py
+(twice the errors measured there; bf16 for both types): one long sequence
+among short and empty ones (many segments of one chain, whose states fold
+over more than one batch of 8), leading rows outside every sequence, more
+sequences than one probe round of the slot search takes, key widths of one
+partial group, two groups and two calls, the cut that only balances ragged
+lengths (and the same call without its workspace, uncut)."""
+import numpy as np
+import pytest
+import torch
+
+from tests.conftest import assert_close
+from tests.test_gpu_gla import HT_BANDS, O_BANDS, _inputs, _oracle, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens,H,K,V,dtype,g16", [
+    ([5, 0, 2000, 64, 1, 0, 130], 2, 64, 64, torch.bfloat16, False),
+    ([3000, 1, 63], 1, 64, 32, torch.float16, False),
+    ([1] * 70 + [900] + [65] * 3, 2, 64, 48, torch.bfloat16, False),
+    ([700, 0, 65, 7], 2, 16, 16, torch.bfloat16, False),
+    ([700, 0, 65, 7], 3, 48, 64, torch.float16, True),
+    ([1500, 64, 1], 2, 128, 128, torch.bfloat16, False),
+    ([129, 700, 0], 3, 80, 16, torch.bfloat16, True),
+    ([300, 65], 2, 112, 48, torch.float16, False),
+    ([300, 65], 2, 144, 80, torch.bfloat16, False),
+    ([200, 30], 1, 256, 64, torch.bfloat16, False),
+])
+def test_segments(dev, lens, H, K, V, dtype, g16):
+    from ssla_amd.gla import chunk_gla
+    print(f"segments lens={lens[:4]}.. H={H} K={K} V={V} {dtype} g16={g16}", flush=True)
+    q, k, v, g, cu, s0 = _inputs(lens, H, K, V, dtype, seed=K + V)
+    if g16:
+        g = g.to(dtype)
+    o, ht = _run(chunk_gla, q, k, v, g, cu, s0, K ** -0.5, dev)
+    ro, rht = _oracle(q, k, v, g, cu, s0, K ** -0.5)
+    assert_close(o, ro, 0.0, "o", band=O_BANDS["logsig"][0], ratio_max=O_BANDS["logsig"][1])
+    assert_close(ht, rht, 0.0, "ht", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
+    # the same sequences after rows that belong to none
+    pad = lambda t: torch.cat([torch.zeros(3, *t.shape[1:], dtype=t.dtype), t])   # noqa: E731
+    o2, ht2 = _run(chunk_gla, pad(q), pad(k), pad(v), pad(g), cu + 3, s0, K ** -0.5, dev)
+    assert_close(o2[3:], ro, 0.0, "o, led", band=O_BANDS["logsig"][0], ratio_max=O_BANDS["logsig"][1])
+    assert_close(ht2, rht, 0.0, "ht, led", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
+
+
+def test_many_ragged_sequences(dev):
+    """64 sequences x 8 heads of 1,024 rows on average (one segment each
+    fills the GPU), one of them 9,000 rows: cut to balance, and uncut when
+    the caller has no workspace."""
+    from ssla_amd import _lib
+    from ssla_amd.gla import chunk_gla
+    rng = np.random.default_rng(0)
+    lens = rng.integers(600, 1150, 63).tolist()
+    lens = lens + [64 * 1024 - sum(lens)]
+    q, k, v, g, cu, s0 = _inputs(lens, 8, 64, 16, torch.bfloat16, seed=9)
+    T = sum(lens)
+    lib = _lib.load()
+    assert lib.ssla_gla_chunk_workspace_size(64, T, 8, 64, 16) > 0
+    print("many ragged sequences", flush=True)
+    o, ht = _run(chunk_gla, q, k, v, g, cu, s0, 0.125, dev)
+    ro, rht = _oracle(q, k, v, g, cu, s0, 0.125)
+    for nm, a, b, bands in (("o", o, ro, O_BANDS), ("ht", ht, rht, HT_BANDS)):
+        assert_close(a, b, 0.0, nm, band=bands["logsig"][0], ratio_max=bands["logsig"][1])
+    d = [t.to(dev) for t in (q, k, v, g, cu, s0)]
+    o2, ht2 = torch.empty_like(d[2]), torch.empty_like(d[5])
+    P = _lib.ptr
+    _lib.check(lib.ssla_gla_chunk_fwd(P(d[0]), P(d[1]), P(d[2]), P(d[3]), _lib.SSLA_F32, P(d[4]), 64, T, 8, 64, 16, 0.125,
+                                      P(d[5]), P(o2), P(ht2), _lib.SSLA_BF16, None, 0, _lib.stream_of(o2)), "fwd")
+    assert_close(o2.float().cpu().numpy(), ro, 0.0, "o, uncut", band=O_BANDS["logsig"][0],
+                 ratio_max=O_BANDS["logsig"][1])
+    assert_close(ht2.cpu().numpy(), rht, 0.0, "ht, uncut", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
