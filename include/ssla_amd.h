@@ -212,6 +212,11 @@ int ssla_gla_chunk_bwd(const void *q, const void *k, const void *v,
  * walking the whole sequence.  The size query returns 0 for shapes where
  * the single pass is faster (sequences shorter than 64 steps on average)
  * or not available (K not a multiple of 16 up to 64); then pass NULL, 0. */
+/* cu_seqlens[0] and cu_seqlens[n_seq] into host_out[0..1] (pinned host
+ * memory) in stream order, then `event` (hipEvent_t) recorded: the rows the
+ * sequences cover, known without waiting for work queued after. */
+int ssla_seq_bounds_async(const int64_t *cu_seqlens, int n_seq, int64_t *host_out, void *event, void *stream);
+
 size_t ssla_gla_recurrent_workspace_size(int n_seq, int64_t T, int H, int K, int V);
 int ssla_gla_recurrent_fwd(const void *q, const void *k, const void *v,
                            const void *g, int g_dtype,
@@ -375,6 +380,18 @@ int ssla_scatter_mean(const float *src, const int64_t *index, int64_t E,
 /* Copies the device status word written by the last scatter call that used
  * `workspace` into *status_out (host), synchronising `stream`.  Returns
  * SSLA_OK; *status_out is SSLA_ERR_ARG if any index was out of range. */
+/* ssla_scatter_max / _mean that settle the index's validity first: *host_bad
+ * (pinned host memory, set to SSLA_OK by the caller) receives SSLA_ERR_ARG
+ * for an index out of [0, n_out) or, with index_sorted, below the one before
+ * it, and `event` (hipEvent_t) is recorded on the stream after that and
+ * before the reduction, so a caller can wait for the answer while the
+ * reduction runs. */
+int ssla_scatter_max_checked(const float *src, const int64_t *index, int64_t E, int C, int64_t n_out,
+                             int index_sorted, float *out, int64_t *argmax, void *workspace,
+                             size_t workspace_bytes, int32_t *host_bad, void *event, void *stream);
+int ssla_scatter_mean_checked(const float *src, const int64_t *index, int64_t E, int C, int64_t n_out,
+                              int index_sorted, float *out, void *workspace, size_t workspace_bytes,
+                              int32_t *host_bad, void *event, void *stream);
 int ssla_scatter_check(const void *workspace, int *status_out, void *stream);
 
 

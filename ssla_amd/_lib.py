@@ -83,6 +83,9 @@ SIGNATURES = {
     "ssla_scatter_workspace_size": (_sz, [_i64, _i32, _i64]),
     "ssla_scatter_max": (_i32, [_vp, _vp, _i64, _i32, _i64, _i32, _vp, _vp, _vp, _sz, _vp]),
     "ssla_scatter_mean": (_i32, [_vp, _vp, _i64, _i32, _i64, _i32, _vp, _vp, _sz, _vp]),
+    "ssla_scatter_max_checked": (_i32, [_vp, _vp, _i64, _i32, _i64, _i32, _vp, _vp, _vp, _sz, _vp, _vp, _vp]),
+    "ssla_scatter_mean_checked": (_i32, [_vp, _vp, _i64, _i32, _i64, _i32, _vp, _vp, _sz, _vp, _vp, _vp]),
+    "ssla_seq_bounds_async": (_i32, [_vp, _i32, _vp, _vp, _vp]),
     "ssla_scatter_check": (_i32, [_vp, C.POINTER(_i32), _vp]),
     "ssla_rf_lut_shape": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, C.POINTER(_i64)]),
     "ssla_rf_lut": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
@@ -198,6 +201,41 @@ def ptr(t: torch.Tensor | None) -> int | None:
 def stream_of(t: torch.Tensor) -> int:
     """The raw handle of the current stream of t's device."""
     return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+class HostWords:
+    """Two int64 words of pinned host memory that a kernel writes, and the
+    event recorded behind it.  ``take`` hands one out, ``read`` waits for the
+    event (not for work queued after it), returns the words and puts the
+    object back; at most 16 per device are kept.  One caller owns an object
+    between the two, so threads and streams never share one."""
+    __slots__ = ("words", "event", "dev", "ptr", "handle")
+    _free: dict = {}
+
+    def __init__(self, dev: int):
+        with torch.cuda.device(dev):
+            self.words = torch.zeros(2, dtype=torch.int64, pin_memory=True).numpy()
+            self.event = torch.cuda.Event()
+            self.event.record()   # creates it on this device
+        self.dev, self.ptr, self.handle = dev, self.words.ctypes.data, self.event.cuda_event
+
+    @classmethod
+    def take(cls, t: torch.Tensor) -> "HostWords":
+        dev = t.get_device()
+        try:
+            w = cls._free[dev].pop()   # (one bytecode-level call: safe between threads)
+        except (KeyError, IndexError):
+            w = cls(dev)
+        w.words[:] = 0
+        return w
+
+    def read(self):
+        self.event.synchronize()
+        out = int(self.words[0]), int(self.words[1])
+        free = self._free.setdefault(self.dev, [])
+        if len(free) < 16:
+            free.append(self)
+        return out
 
 
 class ParamWatch:

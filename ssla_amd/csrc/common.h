@@ -105,6 +105,13 @@ template <> struct Elem<SSLA_F16> {
 // ~1 ulp over the normal range, flushes results below 2^-126 to 0).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// A word of pinned (coherent) host memory, visible to the host once an event
+// recorded after the kernel has passed.
+template <typename T>
+__device__ __forceinline__ void store_host(T *p, T x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------------------- DPP --
 // Shift right by N lanes inside each 16-lane DPP row; lanes whose source
 // lies outside the row read 0 (bound_ctrl), so an add of the result folds

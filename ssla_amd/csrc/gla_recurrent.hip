@@ -785,6 +785,29 @@ extern "C" int ssla_gla_recurrent_fwd(const void *q, const void *k, const void *
   return SSLA_ERR_DTYPE;
 }
 
+namespace ssla {
+namespace {
+__global__ void seq_bounds_kernel(const int64_t *__restrict__ cu, int n_seq, int64_t *host) {
+  if (threadIdx.x < 2) store_host(host + threadIdx.x, cu[threadIdx.x ? n_seq : 0]);
+}
+}  // namespace
+}  // namespace ssla
+
+extern "C" int ssla_seq_bounds_async(const int64_t *cu_seqlens, int n_seq, int64_t *host_out, void *event,
+                                     void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(cu_seqlens && host_out && event && n_seq >= 0, "seq_bounds_async: bad arguments");
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(seq_bounds_kernel, dim3(1), dim3(64), 0, st, cu_seqlens, n_seq, host_out);
+  const hipError_t e = hipEventRecord(static_cast<hipEvent_t>(event), st);
+  if (e != hipSuccess) {
+    set_error("seq_bounds_async: event record failed: %s", hipGetErrorString(e));
+    return SSLA_ERR_LAUNCH;
+  }
+  return launch_status("seq_bounds_async");
+}
+
 extern "C" size_t ssla_gla_recurrent_workspace_size(int n_seq, int64_t T, int H, int K, int V) {
   if (H <= 0) return 0;
   return ssla::seg_layout(n_seq, T, H, K, V).total;

@@ -176,7 +176,7 @@ template <bool LDS>
 __global__ __launch_bounds__(kEvThreads) void hist_kernel(
     const int64_t *__restrict__ index, int64_t E, int64_t n_out, int64_t NB, int n_hist,
     int32_t *__restrict__ hist, int32_t *__restrict__ errs, int32_t *ticket, uint64_t *flags,
-    int64_t n_flags, int32_t *arrive, int64_t n_arrive) {
+    int64_t n_flags, int32_t *arrive, int64_t n_arrive, int32_t *host_bad) {
   clear_scan_state(ticket, flags, n_flags, arrive, n_arrive);
   bool bad = false;
   if constexpr (LDS) {
@@ -211,6 +211,7 @@ __global__ __launch_bounds__(kEvThreads) void hist_kernel(
   }
   const int any_bad = __syncthreads_or(bad ? 1 : 0);
   if (threadIdx.x == 0) errs[blockIdx.x] = any_bad ? SSLA_ERR_ARG : SSLA_OK;
+  if (threadIdx.x == 0 && any_bad && host_bad) store_host(host_bad, static_cast<int32_t>(SSLA_ERR_ARG));
 }
 
 // ---------------------------------------------------------------- scan --
@@ -978,9 +979,36 @@ __global__ __launch_bounds__(256) void fill_i32(int32_t *__restrict__ p, int64_t
     p[i] = val;
 }
 
+// The sorted path's check on its own (its range kernel finds a bad index only
+// while it reduces): reads the index alone, 3-4 us for 300,000 events against
+// the 38 us of the reduction a caller would otherwise wait for.
+__global__ __launch_bounds__(256) void sorted_check_kernel(const int64_t *__restrict__ index, int64_t E, int64_t n_out,
+                                                           int32_t *host_bad) {
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  bool bad = false;
+  for (int64_t i0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i0 < E; i0 += 4 * stride) {
+    int64_t r[4], p[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = i0 + u * stride;
+      r[u] = i < E ? index[i] : 0;
+      p[u] = i < E && i > 0 ? index[i - 1] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) bad |= i0 + u * stride < E && (bad_row(r[u], n_out) || r[u] < p[u]);
+  }
+  if (__syncthreads_or(bad ? 1 : 0) && threadIdx.x == 0) store_host(host_bad, static_cast<int32_t>(SSLA_ERR_ARG));
+}
+
+// host_bad (pinned host memory holding SSLA_OK, or NULL): receives
+// SSLA_ERR_ARG for a bad index; `checked` is recorded on the stream once that
+// is settled, ahead of the reduction's launches.
 template <bool MEAN>
 int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_t n_out,
-                int sorted, float *out, int64_t *argmax, void *ws, size_t ws_bytes, hipStream_t st) {
+                int sorted, float *out, int64_t *argmax, void *ws, size_t ws_bytes, hipStream_t st,
+                int32_t *host_bad = nullptr, hipEvent_t checked = nullptr) {
+  auto settled = [&]() { return host_bad ? hipEventRecord(checked, st) : hipSuccess; };
+  hipError_t ee = hipSuccess;
   const char *name = MEAN ? "scatter_mean" : "scatter_max";
   SSLA_CHECK_ARG(E >= 0 && n_out >= 0 && C > 0, "%s: bad sizes E=%lld C=%d n_out=%lld", name,
                  (long long)E, C, (long long)n_out);
@@ -995,7 +1023,9 @@ int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_
   int32_t *status = reinterpret_cast<int32_t *>(base + L.status);
   int32_t *ticket = status + 1;
   if (n_out == 0) {
+    // (an index has no row to name: the status stays OK, as before)
     hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, status, (int64_t)1, (int32_t)SSLA_OK);
+    if (settled() != hipSuccess) set_error("%s: event record failed", name);
     return launch_status(name);
   }
   SSLA_CHECK_ARG(out && (MEAN || argmax), "%s: null output pointer", name);
@@ -1011,6 +1041,12 @@ int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_
     uint64_t *rpieces = reinterpret_cast<uint64_t *>(base + L.rpieces);
     SSLA_CHECK_ARG(L.n_rseg < 0x7fffffff, "%s: too many events x channel blocks", name);
     const int32_t E32 = static_cast<int32_t>(E), n32 = static_cast<int32_t>(n_out), r32 = static_cast<int32_t>(L.n_rseg);
+    if (host_bad) {
+      if (E > 0)
+        hipLaunchKernelGGL(sorted_check_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(1024, (E + 1023) / 1024))),
+                           dim3(256), 0, st, index, E, n_out, host_bad);
+      ee = settled();
+    }
     if (C == 64)
       hipLaunchKernelGGL((seg_range_kernel<MEAN, 64>), dim3(static_cast<unsigned>(L.n_rseg)), dim3(64 * kRangeWaves),
                          0, st, src, index, E32, C, n32, out, argmax, rflags, rpieces, r32, status);
@@ -1019,6 +1055,10 @@ int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_
                          0, st, src, index, E32, C, n32, out, argmax, rflags, rpieces, r32, status);
     hipLaunchKernelGGL(seg_link_kernel<MEAN>, dim3(static_cast<unsigned>((L.n_rseg + kLinkWaves - 1) / kLinkWaves)),
                        dim3(64 * kLinkWaves), 0, st, E, C, n_out, out, argmax, rflags, rpieces, n_rng, status);
+    if (ee != hipSuccess) {
+      set_error("%s: event record failed: %s", name, hipGetErrorString(ee));
+      return SSLA_ERR_LAUNCH;
+    }
     return launch_status(name);
   }
   // unsorted: bucketing by 64-row buckets, then the LDS reduce per chunk
@@ -1040,16 +1080,17 @@ int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_
   int n_err = 0;
   if (lds) {
     hipLaunchKernelGGL((hist_kernel<true>), dim3(L.n_hist), dim3(kEvThreads), 0, st, index, E, n_out, NB, L.n_hist,
-                       hist, errs, ticket, flags, n_scan + 1, arrive, NB * ncb);
+                       hist, errs, ticket, flags, n_scan + 1, arrive, NB * ncb, host_bad);
     n_err = L.n_hist;
   } else {
     hipLaunchKernelGGL(fill_i32, dim3(static_cast<unsigned>(std::min<int64_t>(1024, (NB + 256) / 256))), dim3(256),
                        0, st, hist, NB + 1, 0);
     const int nb = global_hist_blocks(E);
     hipLaunchKernelGGL((hist_kernel<false>), dim3(nb), dim3(kEvThreads), 0, st, index, E, n_out, NB, 1, hist, errs,
-                       ticket, flags, n_scan + 1, arrive, NB * ncb);
+                       ticket, flags, n_scan + 1, arrive, NB * ncb, host_bad);
     n_err = nb;
   }
+  ee = settled();
   hipLaunchKernelGGL(scan_kernel, dim3(static_cast<unsigned>(n_scan)), dim3(kScanCells * kScanTpc), 0, st, hist,
                      L.n_hist, NB, off, coff, cdesc, L.n_chunks, ticket, flags, errs, n_err, status);
   if (lds) {
@@ -1070,6 +1111,10 @@ int run_scatter(const float *src, const int64_t *index, int64_t E, int C, int64_
       hipLaunchKernelGGL((bucket_reduce_kernel<MEAN, 0>), dim3(static_cast<unsigned>(L.n_chunks * ncb)),
                          dim3(64 * kRedWaves), 0, st, src, perm, cdesc, coff, NB32, E32, C, n32, out, argmax, parts,
                          pcnt, arrive, static_cast<int32_t>(L.n_chunks));
+  }
+  if (ee != hipSuccess) {
+    set_error("%s: event record failed: %s", name, hipGetErrorString(ee));
+    return SSLA_ERR_LAUNCH;
   }
   return launch_status(name);
 }
@@ -1096,6 +1141,25 @@ extern "C" int ssla_scatter_mean(const float *src, const int64_t *index, int64_t
   ssla::clear_error();
   return ssla::run_scatter<true>(src, index, E, C, n_out, index_sorted, out, nullptr, workspace,
                                  workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int ssla_scatter_max_checked(const float *src, const int64_t *index, int64_t E, int C,
+                                        int64_t n_out, int index_sorted, float *out, int64_t *argmax,
+                                        void *workspace, size_t workspace_bytes, int32_t *host_bad, void *event,
+                                        void *stream) {
+  ssla::clear_error();
+  SSLA_CHECK_ARG(host_bad && event, "scatter_max_checked: null pointer");
+  return ssla::run_scatter<false>(src, index, E, C, n_out, index_sorted, out, argmax, workspace, workspace_bytes,
+                                  static_cast<hipStream_t>(stream), host_bad, static_cast<hipEvent_t>(event));
+}
+
+extern "C" int ssla_scatter_mean_checked(const float *src, const int64_t *index, int64_t E, int C,
+                                         int64_t n_out, int index_sorted, float *out, void *workspace,
+                                         size_t workspace_bytes, int32_t *host_bad, void *event, void *stream) {
+  ssla::clear_error();
+  SSLA_CHECK_ARG(host_bad && event, "scatter_mean_checked: null pointer");
+  return ssla::run_scatter<true>(src, index, E, C, n_out, index_sorted, out, nullptr, workspace, workspace_bytes,
+                                 static_cast<hipStream_t>(stream), host_bad, static_cast<hipEvent_t>(event));
 }
 
 extern "C" int ssla_scatter_check(const void *workspace, int *status_out, void *stream) {

@@ -329,8 +329,9 @@ def fused_recurrent_gla(
     o has q's dtype, the final state is fp32.  As the reference concatenates
     the outputs of its sequences (naive.py:106), o holds the rows
     ``cu_seqlens[0]:cu_seqlens[-1]``.  Finding them reads the two bounds
-    back, one host sync per call (as the reference's ``.item()`` calls do),
-    unless ``cu_seqlens`` is a CPU tensor; :func:`fused_recurrent_gla_rows`
+    back, one host wait per call (as the reference's ``.item()`` calls do; for
+    the work queued before, not for the recurrence), unless ``cu_seqlens`` is
+    a CPU tensor; :func:`fused_recurrent_gla_rows`
     makes no sync and returns all T rows (for callers whose sequences cover
     the batch, e.g. under HIP graph capture)."""
     if scale is None:
@@ -344,8 +345,17 @@ def fused_recurrent_gla(
                          f"got {tuple(h0.shape)}")
     o = torch.empty(T, H, V, device=q.device, dtype=q.dtype)
     ht = torch.empty(N, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
+    # the bounds are queued ahead of the recurrence and read while it runs
+    bounds = None
+    if N > 0 and cu_seqlens.is_cuda:
+        bounds = _lib.HostWords.take(cu)
+        _lib.check(_lib.load().ssla_seq_bounds_async(_lib.ptr(cu), N, bounds.ptr, bounds.handle, _lib.stream_of(cu)),
+                   "ssla_seq_bounds_async")
     o, ht = _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
-    lo, hi = (int(x) for x in cu_seqlens[[0, -1]].tolist()) if N > 0 else (0, 0)
+    if bounds is not None:
+        lo, hi = bounds.read()
+    else:
+        lo, hi = (int(x) for x in cu_seqlens[[0, -1]].tolist()) if N > 0 else (0, 0)
     if (lo, hi) != (0, T):
         o = o[lo:hi]
     return o, ht

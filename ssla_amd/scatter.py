@@ -58,24 +58,27 @@ def _prep(name, src, index, dim, dim_size):
     return src.contiguous(), index, int(dim_size), Cc, squeeze
 
 
-def _run(name, fn, src, index, n_out, sorted_index, out, argmax, check):
+def _run(name, src, index, n_out, sorted_index, out, argmax, check):
     E, Cp = src.shape
     lib = _lib.load()
+    fn = getattr(lib, f"ssla_{name}_checked" if check else f"ssla_{name}")
     ws_bytes = lib.ssla_scatter_workspace_size(E, Cp, n_out)
     ws = torch.empty(ws_bytes, device=src.device, dtype=torch.uint8)
     args = [_lib.ptr(src), _lib.ptr(index), E, Cp, n_out, 1 if sorted_index else 0, _lib.ptr(out)]
     if argmax is not None:
         args.append(_lib.ptr(argmax))
-    args += [_lib.ptr(ws), ws_bytes, _lib.stream_of(src)]
-    _lib.check(fn(*args), name)
-    if check:
-        import ctypes
-        status = ctypes.c_int(0)
-        _lib.check(lib.ssla_scatter_check(_lib.ptr(ws), ctypes.byref(status), _lib.stream_of(src)),
-                   "ssla_scatter_check")
-        if status.value != 0:
-            raise ValueError(f"{name}: index out of range [0, {n_out})"
-                             + (" or not sorted" if sorted_index else ""))
+    args += [_lib.ptr(ws), ws_bytes]
+    if not check:
+        _lib.check(fn(*args, _lib.stream_of(src)), name)
+        return
+    # The index is checked ahead of the reduction: this waits for the answer
+    # while the reduction runs (waiting for the whole call left the device
+    # idle through the next call's host work).
+    bad = _lib.HostWords.take(src)
+    _lib.check(fn(*args, bad.ptr, bad.handle, _lib.stream_of(src)), name)
+    if bad.read()[0] != 0:
+        raise ValueError(f"{name}: index out of range [0, {n_out})"
+                         + (" or not sorted" if sorted_index else ""))
 
 
 def _no_out(name, out):
@@ -91,7 +94,7 @@ class _ScatterMax(torch.autograd.Function):
         E, Cc = src.shape
         res = torch.empty(n_out, Cc, device=src.device, dtype=torch.float32)
         arg = torch.empty(n_out, Cc, device=src.device, dtype=torch.int64)
-        _run("scatter_max", _lib.load().ssla_scatter_max, src, idx, n_out, sorted_index, res, arg, check)
+        _run("scatter_max", src, idx, n_out, sorted_index, res, arg, check)
         ctx.save_for_backward(arg)
         ctx.n_src = E
         ctx.mark_non_differentiable(arg)
@@ -110,7 +113,7 @@ class _ScatterMean(torch.autograd.Function):
     def forward(ctx, src, idx, n_out, sorted_index, check):
         Cc = src.shape[1]
         res = torch.empty(n_out, Cc, device=src.device, dtype=torch.float32)
-        _run("scatter_mean", _lib.load().ssla_scatter_mean, src, idx, n_out, sorted_index, res, None, check)
+        _run("scatter_mean", src, idx, n_out, sorted_index, res, None, check)
         ctx.save_for_backward(idx)
         ctx.n_out = n_out
         return res
