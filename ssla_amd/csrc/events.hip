@@ -720,6 +720,42 @@ __global__ void rf_count_lanes(const int64_t *__restrict__ lut, int64_t n_rf, in
   }
 }
 
+// rf_count for other A up to 16, 16 lanes per field, four fields at a time:
+// one chain of lookups per lane and coalesced table rows, where rf_count makes
+// A chains after one another in a thread (583,680 3 x 3 fields: 56 us, here 31).
+constexpr int kCountU = 4;
+__global__ __launch_bounds__(256) void rf_count16(const int64_t *__restrict__ lut, int64_t n_rf, int A, int64_t n_f,
+                                                  int64_t HW, const int32_t *__restrict__ pixmap,
+                                                  const int64_t *__restrict__ glen, int64_t *__restrict__ nev,
+                                                  int64_t *__restrict__ act, int64_t *__restrict__ pk) {
+  const int j = threadIdx.x & 15;
+  const int64_t f0 = static_cast<int64_t>(blockIdx.x) * kCountU * 16 + (threadIdx.x >> 4);
+  int64_t p[kCountU], b[kCountU], n[kCountU];
+  int32_t g[kCountU];
+#pragma unroll
+  for (int u = 0; u < kCountU; ++u) {
+    const int64_t f = f0 + u * 16;
+    b[u] = static_cast<uint32_t>(f) / static_cast<uint32_t>(n_rf);   // n_f < 2^31
+    p[u] = f < n_f && j < A ? lut[(f - b[u] * n_rf) * A + j] : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < kCountU; ++u) g[u] = p[u] >= 0 ? pixmap[b[u] * HW + p[u]] : -1;
+#pragma unroll
+  for (int u = 0; u < kCountU; ++u) n[u] = g[u] >= 0 ? glen[g[u]] : 0;
+#pragma unroll
+  for (int u = 0; u < kCountU; ++u) {
+    const int64_t f = f0 + u * 16;
+    const uint64_t any = __builtin_amdgcn_ballot_w64(g[u] >= 0) >> (threadIdx.x & 48) & 0xffff;
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2) n[u] += __shfl_xor(static_cast<long long>(n[u]), d, 16);
+    if (f < n_f && j == 0) {
+      nev[f] = n[u];
+      act[f] = any ? 1 : 0;
+      if (pk) pk[f] = (n[u] << kPackBits) | (any ? 1 : 0);
+    }
+  }
+}
+
 // From the prefix sum of the packed pairs, in one launch: act_pre / ev_pre
 // of every field, the flat index and event count of every active field
 // (f_index / f_len at its active index, as rf_fields writes them) and the
@@ -1596,6 +1632,118 @@ __global__ void rf_merge(const int32_t *__restrict__ ev2g, const int64_t *__rest
     if (o_fidx) o_fidx[row] = static_cast<int32_t>(act_pre[b * n_rf + rf]);
   }
 }
+
+// The same fill with 16 lanes per active field (at most 16 positions): lane
+// a looks up position a's run once, the field's rows (event, position, time)
+// are laid side by side in LDS, position by position, and a row's place is
+// the number of rows before it by (time, place) -- compared against all of
+// them, where rf_merge makes every (event, position) pair look the other
+// positions' runs up again and search each.  A 3 x 3 field holds 7 rows on
+// average (400,000 events, 3.6 M rows): rf_merge 212 us, here 124.  Fields of
+// more than kFieldRows rows search the runs.
+// Bound by its instructions (some 300 per wavefront of four fields), so a row
+// carries one 64-bit key (time << 7 | place) and a place is one compare per
+// other row.
+constexpr int kFieldRows = 96;
+constexpr int64_t kFieldTime = (int64_t{1} << 56) - 1;   // the latest time a key holds
+template <int N>
+__device__ __forceinline__ int row_shr_i(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x110 + N, 0xf, 0xf, true);
+}
+// Orders LDS between the lanes of a field, which share a wavefront.
+__device__ __forceinline__ void field_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__global__ __launch_bounds__(256) void rf_merge_fields(
+    const int64_t *__restrict__ f_index, int64_t n_act, const int32_t *__restrict__ pixmap,
+    const int64_t *__restrict__ gstart, const int64_t *__restrict__ glen, const int64_t *__restrict__ lut, int64_t n_rf,
+    int A, int64_t n_f, int64_t HW, const int64_t *__restrict__ ev_pre, const int64_t *__restrict__ time, int64_t E_in,
+    int64_t E_out, int64_t *__restrict__ o_src, int64_t *__restrict__ o_time, int64_t *__restrict__ o_pos,
+    int32_t *__restrict__ dst_map) {
+  // (odd pitches: the four fields of a wavefront read different banks)
+  __shared__ uint64_t s_t[16][kFieldRows + 1];   // time (clamped at 0) << 7 | row
+  __shared__ uint32_t s_e[16][kFieldRows + 1];   // event << 4 | position
+  const int j = threadIdx.x & 15, fl = threadIdx.x >> 4;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 16 + fl;
+  const int64_t f = i < n_act ? f_index[i] : -1;
+  const bool valid = f >= 0 && f < n_f;
+  const int64_t base = valid ? ev_pre[f] : 0;
+  int s = 0, n = 0;   // E_in < 2^28
+  if (valid && j < A) {
+    const uint32_t b = static_cast<uint32_t>(f) / static_cast<uint32_t>(n_rf);
+    const int64_t p = lut[(f - static_cast<int64_t>(b) * n_rf) * A + j];
+    const int32_t g = p >= 0 ? pixmap[b * HW + p] : -1;
+    if (g >= 0) {
+      s = static_cast<int>(min(max(gstart[g], (int64_t)0), E_in));
+      n = static_cast<int>(min(max(glen[g], (int64_t)0), E_in - s));
+    }
+  }
+  const int nc = min(n, kFieldRows + 1);   // (no sum of a field's runs overflows)
+  int off = nc;   // inclusive, then exclusive over the field's positions
+  off += row_shr_i<1>(off);
+  off += row_shr_i<2>(off);
+  off += row_shr_i<4>(off);
+  off += row_shr_i<8>(off);
+  const int total = __shfl(off, 15, 16);
+  off -= nc;
+  auto emit = [&](int64_t e, int64_t t, int a, int rank) {
+    const int64_t row = base + rank;
+    if (row < 0 || row >= E_out) return;   // inconsistent inputs: drop, never write out of range
+    o_src[row] = e;
+    if (o_time) o_time[row] = t;
+    o_pos[row] = a;
+    if (dst_map) dst_map[e * A + a] = static_cast<int32_t>(row);
+  };
+  bool late = total > kFieldRows;
+  if (!late) {
+    for (int k = 0; k < n; ++k) s_e[fl][off + k] = static_cast<uint32_t>(s + k) << 4 | static_cast<uint32_t>(j);
+    field_sync();
+    for (int r = j; r < total; r += 16) {
+      const int64_t t = time[s_e[fl][r] >> 4];
+      late |= t >= kFieldTime;
+      s_t[fl][r] = static_cast<uint64_t>(min(max(t, (int64_t)0), kFieldTime)) << 7 | static_cast<uint64_t>(r);
+    }
+    field_sync();
+  }
+  // A field with more rows, or later times, than its keys hold goes by search.
+  if ((__builtin_amdgcn_ballot_w64(late) >> (threadIdx.x & 48) & 0xffff) == 0) {
+    for (int r = j; r < total; r += 16) {
+      const uint64_t key = s_t[fl][r];
+      int rank = 0;
+#pragma unroll 4
+      for (int q = 0; q < total; ++q) rank += s_t[fl][q] < key ? 1 : 0;
+      const int64_t e = s_e[fl][r] >> 4, t = static_cast<int64_t>(key >> 7);
+      emit(e, o_time && t == 0 ? time[e] : t, static_cast<int>(s_e[fl][r] & 15), rank);
+    }
+    return;
+  }
+  for (int a = 0; a < A; ++a) {
+    const int sa = __shfl(s, a, 16), na = __shfl(n, a, 16);
+    for (int k0 = 0; k0 < na; k0 += 16) {
+      const bool in = k0 + j < na;
+      const int64_t e = sa + k0 + j;
+      const int64_t t = in ? time[e] : 0, tc = max(t, (int64_t)0);
+      int rank = k0 + j;
+      for (int a2 = 0; a2 < A; ++a2) {
+        const int s2 = __shfl(s, a2, 16);
+        int lo = 0, hi = __shfl(n, a2, 16);
+        if (a2 == a || !in) continue;
+        while (lo < hi) {   // elements < tc (<= tc for earlier positions)
+          const int mid = (lo + hi) >> 1;
+          const int64_t v = max(time[s2 + mid], (int64_t)0);
+          if (a2 < a ? v <= tc : v < tc)
+            lo = mid + 1;
+          else
+            hi = mid;
+        }
+        rank += lo;
+      }
+      if (in) emit(e, t, a, rank);
+    }
+  }
+}
 }  // namespace
 
 // ---- receptive-field / patch scatter ---------------------------------------------
@@ -1705,6 +1853,10 @@ int rf_plan_impl(const int64_t *gr_batch, const int64_t *gr_h, const int64_t *gr
   } else if (lanes)
     hipLaunchKernelGGL(rf_count_lanes, dim3(static_cast<unsigned>((n_f * A + kThreads - 1) / kThreads)),
                        dim3(kThreads), 0, st, lut, n_rf, A, B, H, W, L.pixmap, gr_len, L.nev, L.act,
+                       packed ? L.pk : nullptr);
+  else if (A <= 16 && n_f < 0x7fffffff && n_f > 0)
+    hipLaunchKernelGGL(rf_count16, dim3(static_cast<unsigned>((n_f + 16 * kCountU - 1) / (16 * kCountU))), dim3(256),
+                       0, st, lut, n_rf, A, n_f, static_cast<int64_t>(H) * W, L.pixmap, gr_len, L.nev, L.act,
                        packed ? L.pk : nullptr);
   else
     hipLaunchKernelGGL(rf_count, dim3(grid_for(n_f)), dim3(kThreads), 0, st, lut, n_rf, A, B, H, W, L.pixmap, gr_len,
@@ -1821,8 +1973,19 @@ extern "C" int ssla_rf_scatter_fill_sorted(const int64_t *gr_batch, const int64_
   const int64_t HW = static_cast<int64_t>(H) * W;
   const int64_t n_dst = dst_map ? E_in * A : 0;
   const int64_t n_act = std::max<int64_t>(n_active, 0);
-  hipLaunchKernelGGL(rf_sorted_setup, dim3(grid_for(std::max(std::max(HW * A, n_dst), n_act))), dim3(kThreads), 0, st,
-                     inv, HW * A, dst_map, n_dst, f_index, L.f_index, f_len, L.f_len, n_act);
+  // one position has nothing to merge; past 16 a field's lanes would take several lookups each
+  // (rf_merge needs the inverse table, rf_merge_fields none)
+  const bool fields = A > 1 && A <= 16 && n_f < 0x7fffffff && E_in < (int64_t{1} << 28);
+  hipLaunchKernelGGL(rf_sorted_setup, dim3(grid_for(std::max(std::max(fields ? 0 : HW * A, n_dst), n_act))),
+                     dim3(kThreads), 0, st, inv, fields ? 0 : HW * A, dst_map, n_dst, f_index, L.f_index, f_len, L.f_len,
+                     n_act);
+  if (fields) {
+    if (n_act > 0 && E_out > 0)
+      hipLaunchKernelGGL(rf_merge_fields, dim3(static_cast<unsigned>((n_act + 15) / 16)), dim3(256), 0, st, L.f_index,
+                         n_act, L.pixmap, L.gstart, gr_len, lut, n_rf, A, n_f, HW, L.ev_pre, time, E_in, E_out, out_src,
+                         out_time, out_pos, dst_map);
+    return launch_status("rf_scatter_fill_sorted");
+  }
   hipLaunchKernelGGL(rf_inv_lut, dim3(grid_for(n_rf * A)), dim3(kThreads), 0, st, lut, n_rf, A, HW, inv);
   if (E_in > 0) {
     if (E_out > 0)
