@@ -546,6 +546,17 @@ int ssla_mos_train_bwd(const float *dout, const float *events, int64_t E, int c_
                        const float *y, const unsigned char *valid, float *devents, float *dWaT, float *dWbT,
                        float *dWinT, void *workspace, size_t workspace_bytes, void *stream);
 
+/* LayerNorm of n > 0 rows of H <= 128 fp32 channels (the norm of
+ * layers/mos_attention.py:101) and its backward.  stats [n, 2] receives mean and
+ * 1 / sqrt(var + eps).  The backward writes those of dx [n, H], dw, db [H]
+ * that are not NULL; the workspace is needed for dw and db.  Sums in a fixed
+ * order. */
+int ssla_row_norm_fwd(const float *x, int64_t n, int H, const float *w, const float *b, float eps, float *y,
+                      float *stats, void *stream);
+size_t ssla_row_norm_bwd_workspace_size(int64_t n, int H);
+int ssla_row_norm_bwd(const float *dy, const float *x, const float *stats, int64_t n, int H, const float *w,
+                      float *dx, float *dw, float *db, void *workspace, size_t workspace_bytes, void *stream);
+
 /* Stable sort of (uint64 key, int32 value) pairs on the low end_bit key
  * bits; vals_in NULL means 0..n-1.  Used for the (batch, time) ordering of
  * LinearAttention.forward (layers/linear_attention.py:62-63) and the

@@ -112,6 +112,9 @@ SIGNATURES = {
                                       _vp, _vp, _i32, _vp, _vp, _vp, _f32, _i32, _vp, _vp, _sz, _vp]),
     "ssla_mos_train_fwd": (_i32, [_vp, _i64, _i32, _vp, _vp, _i64, _vp, _i64, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp,
                                   _vp, _vp]),
+    "ssla_row_norm_fwd": (_i32, [_vp, _i64, _i32, _vp, _vp, _f32, _vp, _vp, _vp]),
+    "ssla_row_norm_bwd_workspace_size": (_sz, [_i64, _i32]),
+    "ssla_row_norm_bwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "ssla_mos_train_bwd_workspace_size": (_sz, [_i64, _i32, _i32, _i32]),
     "ssla_mos_train_bwd": (_i32, [_vp, _vp, _i64, _i32, _vp, _vp, _i64, _vp, _i64, _i32, _vp, _vp, _vp, _i32, _vp, _vp,
                                   _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),

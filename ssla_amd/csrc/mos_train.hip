@@ -15,7 +15,7 @@
 // composed forward and backward ran some 475 launches, with library products
 // of 52k-long reductions into 48 x 48 results at 135-425 us each and 440 us
 // per row sum: 11.6 ms for a training step of a 24 -> 48 layer on 52,000
-// events (9 positions), 1.26 ms here.  The kernels are bound by their row
+// events (9 positions), 1.16 ms here.  The kernels are bound by their row
 // traffic (468,000 rows of 48 channels): scans 113 and 153 us at 4 TB/s,
 // projection 70, the wide weight gradient 95, d events 65 us.
 //
@@ -441,6 +441,144 @@ dim3 scan_grid(const ScanArgs &a) {
 
 size_t up16(size_t x) { return (x + 15) / 16 * 16; }
 
+// ------------------------------------------------------------ layer norm --
+// LayerNorm over the H <= 128 channels of a row and its backward, 16 lanes per
+// row: lane j holds channels j, j + 16, ..., the row sums are lane rotations.
+// A row is read once (the centred second moment is taken in registers), so
+// both passes are bound by their rows: 52,000 x 48 forward 6 us and backward
+// 8 + 7 us, where the library's took 53 us (a workgroup of one wavefront per row)
+// and 81 us (the weight gradients alone 50).  A workgroup's rows are summed
+// per lane for the weight gradients, then over its 16 row groups, then over
+// the workgroups (norm_grad_sum): no atomics, the same bits every run.
+constexpr int kNormBlocks = 1024;
+template <int N>
+__device__ __forceinline__ float ror16(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + N, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float sum16(float x) {
+  x += ror16<8>(x);
+  x += ror16<4>(x);
+  x += ror16<2>(x);
+  return x + ror16<1>(x);
+}
+
+template <int CPL>
+__device__ __forceinline__ void row_ld(const float *p, int j, int H, float (&x)[CPL]) {
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) x[i] = j + 16 * i < H ? p[j + 16 * i] : 0.f;
+}
+
+template <int CPL>
+__global__ __launch_bounds__(256) void row_norm_fwd(const float *__restrict__ x, int64_t n, int H,
+                                                    const float *__restrict__ w, const float *__restrict__ b, float eps,
+                                                    float *__restrict__ y, float2 *__restrict__ stats) {
+  const int j = threadIdx.x & 15;
+  float wj[CPL], bj[CPL];
+  row_ld(w, j, H, wj);
+  row_ld(b, j, H, bj);
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4); r < n;
+       r += static_cast<int64_t>(gridDim.x) * 16) {
+    float v[CPL], s = 0.f, m2 = 0.f;
+    row_ld(x + r * H, j, H, v);
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) s += v[i];
+    const float mean = sum16(s) / H;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      v[i] -= mean;
+      if (j + 16 * i < H) m2 = fmaf(v[i], v[i], m2);
+    }
+    const float rstd = 1.f / sqrtf(sum16(m2) / H + eps);
+#pragma unroll
+    for (int i = 0; i < CPL; ++i)
+      if (j + 16 * i < H) y[r * H + j + 16 * i] = fmaf(v[i] * rstd, wj[i], bj[i]);
+    if (j == 0) stats[r] = make_float2(mean, rstd);
+  }
+}
+
+// part (nullable): [gridDim.x, 2, H], this workgroup's sums of dy xhat and dy.
+template <int CPL>
+__global__ __launch_bounds__(256) void row_norm_bwd(const float *__restrict__ dy, const float *__restrict__ x,
+                                                    const float2 *__restrict__ stats, int64_t n, int H,
+                                                    const float *__restrict__ w, float *__restrict__ dx,
+                                                    float *__restrict__ part) {
+  __shared__ float s_g[16][2][16 * CPL + 1];
+  const int j = threadIdx.x & 15, gr = threadIdx.x >> 4;
+  float wj[CPL], dw[CPL], db[CPL];
+  row_ld(w, j, H, wj);
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) dw[i] = db[i] = 0.f;
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * 16 + gr; r < n; r += static_cast<int64_t>(gridDim.x) * 16) {
+    float g[CPL], h[CPL], s1 = 0.f, s2 = 0.f;
+    row_ld(dy + r * H, j, H, g);
+    row_ld(x + r * H, j, H, h);
+    const float2 st = stats[r];
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      h[i] = (h[i] - st.x) * st.y;
+      dw[i] = fmaf(g[i], h[i], dw[i]);
+      db[i] += g[i];
+      g[i] *= wj[i];
+      if (j + 16 * i < H) {
+        s1 += g[i];
+        s2 = fmaf(g[i], h[i], s2);
+      }
+    }
+    const float m1 = sum16(s1) / H, m2 = sum16(s2) / H;
+    if (dx) {
+#pragma unroll
+      for (int i = 0; i < CPL; ++i)
+        if (j + 16 * i < H) dx[r * H + j + 16 * i] = st.y * (g[i] - m1 - h[i] * m2);
+    }
+  }
+  if (part == nullptr) return;
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) {
+    s_g[gr][0][j + 16 * i] = dw[i];
+    s_g[gr][1][j + 16 * i] = db[i];
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < 2 * H; c += 256) {
+    const int m = c / H, ch = c - m * H;
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += s_g[k][m][ch];
+    part[static_cast<int64_t>(blockIdx.x) * 2 * H + c] = s;
+  }
+}
+
+// out[c] = sum over the workgroups of part[., c], 64 threads per 4 channels.
+__global__ __launch_bounds__(256) void norm_grad_sum(const float *__restrict__ part, int blocks, int H,
+                                                     float *__restrict__ dw, float *__restrict__ db) {
+  __shared__ float s_p[4][65];
+  const int c = blockIdx.x * 4 + (threadIdx.x & 3), p = threadIdx.x >> 2;
+  float s = 0.f;
+  if (c < 2 * H)
+    for (int k = p; k < blocks; k += 64) s += part[static_cast<int64_t>(k) * 2 * H + c];
+  s_p[threadIdx.x & 3][p] = s;
+  for (int d = 32; d > 0; d >>= 1) {
+    __syncthreads();
+    if (p < d) s_p[threadIdx.x & 3][p] += s_p[threadIdx.x & 3][p + d];
+  }
+  if (p == 0 && c < 2 * H) {
+    float *out = c < H ? dw : db;
+    if (out) out[c < H ? c : c - H] = s_p[threadIdx.x & 3][0];
+  }
+}
+
+int norm_blocks(int64_t n) { return static_cast<int>(std::min<int64_t>((n + 15) / 16, kNormBlocks)); }
+
+template <typename F>
+void for_lane_channels(int H, F f) {   // f(channels per lane): 1, 2, 3, 4, 6 or 8
+  const int c = (H + 15) / 16;
+  if (c <= 1) f(std::integral_constant<int, 1>{});
+  else if (c <= 2) f(std::integral_constant<int, 2>{});
+  else if (c <= 3) f(std::integral_constant<int, 3>{});
+  else if (c <= 4) f(std::integral_constant<int, 4>{});
+  else if (c <= 6) f(std::integral_constant<int, 6>{});
+  else f(std::integral_constant<int, 8>{});
+}
+
 int train_check(const char *what, int64_t E, int Cin, int64_t R, int64_t P, int A, int H) {
   SSLA_CHECK_ARG(E > 0 && Cin > 0 && R >= 0 && P >= 0 && A > 0 && H > 0, "%s: bad sizes E=%lld Cin=%d R=%lld P=%lld "
                  "A=%d H=%d", what, (long long)E, Cin, (long long)R, (long long)P, A, H);
@@ -527,4 +665,52 @@ extern "C" int ssla_mos_train_bwd(const float *dout, const float *events, int64_
     }
   }
   return launch_status("mos_train_bwd");
+}
+
+extern "C" int ssla_row_norm_fwd(const float *x, int64_t n, int H, const float *w, const float *b, float eps, float *y,
+                                 float *stats, void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(n > 0 && H > 0 && x && w && b && y && stats, "row_norm_fwd: bad arguments");
+  SSLA_CHECK_ARG((reinterpret_cast<uintptr_t>(stats) & 7) == 0, "row_norm_fwd: stats must be 8-byte aligned");
+  if (H > 128) {
+    set_error("row_norm_fwd: H=%d exceeds 128", H);
+    return SSLA_ERR_UNSUPPORTED;
+  }
+  for_lane_channels(H, [&](auto c) {
+    hipLaunchKernelGGL(row_norm_fwd<decltype(c)::value>, dim3(norm_blocks(n)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), x, n, H, w, b, eps, y, reinterpret_cast<float2 *>(stats));
+  });
+  return launch_status("row_norm_fwd");
+}
+
+extern "C" size_t ssla_row_norm_bwd_workspace_size(int64_t n, int H) {
+  return n > 0 && H > 0 ? sizeof(float) * 2 * H * ssla::norm_blocks(n) : 0;
+}
+
+extern "C" int ssla_row_norm_bwd(const float *dy, const float *x, const float *stats, int64_t n, int H, const float *w,
+                                 float *dx, float *dw, float *db, void *workspace, size_t workspace_bytes,
+                                 void *stream) {
+  using namespace ssla;
+  clear_error();
+  SSLA_CHECK_ARG(n > 0 && H > 0 && dy && x && stats && w, "row_norm_bwd: bad arguments");
+  SSLA_CHECK_ARG((reinterpret_cast<uintptr_t>(stats) & 7) == 0, "row_norm_bwd: stats must be 8-byte aligned");
+  if (H > 128) {
+    set_error("row_norm_bwd: H=%d exceeds 128", H);
+    return SSLA_ERR_UNSUPPORTED;
+  }
+  const size_t need = ssla_row_norm_bwd_workspace_size(n, H);
+  if ((dw || db) && (workspace == nullptr || workspace_bytes < need)) {
+    set_error("row_norm_bwd: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    return SSLA_ERR_WORKSPACE;
+  }
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  float *part = dw || db ? static_cast<float *>(workspace) : nullptr;
+  const int blocks = norm_blocks(n);
+  for_lane_channels(H, [&](auto c) {
+    hipLaunchKernelGGL(row_norm_bwd<decltype(c)::value>, dim3(blocks), dim3(256), 0, st, dy, x,
+                       reinterpret_cast<const float2 *>(stats), n, H, w, dx, part);
+  });
+  if (part) hipLaunchKernelGGL(norm_grad_sum, dim3((2 * H + 3) / 4), dim3(256), 0, st, part, blocks, H, dw, db);
+  return launch_status("row_norm_bwd");
 }

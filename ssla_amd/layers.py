@@ -100,6 +100,44 @@ def _plain_linear(m) -> bool:
             and not m._backward_hooks and not m._backward_pre_hooks)
 
 
+def _plain_norm(m, H, dev) -> bool:
+    """An nn.LayerNorm over H fp32 channels with weight and bias, without
+    hooks: the map of RowNormFunction."""
+    return (type(m) is nn.LayerNorm and tuple(m.normalized_shape) == (H,) and H <= 128
+            and all(p is not None and p.dtype == torch.float32 and p.device == dev for p in (m.weight, m.bias))
+            and not m._forward_hooks and not m._forward_pre_hooks and not m._backward_hooks
+            and not m._backward_pre_hooks)
+
+
+class RowNormFunction(torch.autograd.Function):
+    """LayerNorm of fp32 rows ``[n, H]``, n > 0 and H <= 128, with its
+    backward (ssla_row_norm_fwd / _bwd)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps):
+        x, w, b = x.contiguous(), weight.contiguous(), bias.contiguous()
+        y, stats = torch.empty_like(x), torch.empty(x.shape[0], 2, dtype=torch.float32, device=x.device)
+        P = _lib.ptr
+        _lib.check(_lib.load().ssla_row_norm_fwd(P(x), x.shape[0], x.shape[1], P(w), P(b), float(eps), P(y), P(stats),
+                                                 _lib.stream_of(x)), "row_norm_fwd")
+        ctx.save_for_backward(x, weight, stats)
+        return y
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy):
+        x, weight, stats = ctx.saved_tensors
+        need, (n, H) = ctx.needs_input_grad, x.shape
+        dy, w = dy.to(torch.float32).contiguous(), weight.contiguous()
+        new = lambda on, *shape: torch.empty(*shape, dtype=torch.float32, device=x.device) if on else None   # noqa: E731
+        dx, dw, db = new(need[0], n, H), new(need[1], H), new(need[2], H)
+        lib, P = _lib.load(), _lib.ptr
+        ws = E._ws(lib.ssla_row_norm_bwd_workspace_size(n, H), x.device)
+        _lib.check(lib.ssla_row_norm_bwd(P(dy), P(x), P(stats), n, H, P(w), P(dx), P(dw), P(db), P(ws), ws.numel(),
+                                         _lib.stream_of(dy)), "row_norm_bwd")
+        return dx, dw, db, None
+
+
 class MosTrainFunction(torch.autograd.Function):
     """The part of MosAttention between the patch plan and the LayerNorm, with
     its backward (ssla_mos_train_fwd / _bwd): out[e] = sum_a Wb[a] y[e, a]
@@ -282,7 +320,9 @@ class MosAttention(nn.Module):
         n_copies = events.shape[0] * self.kernel_size[0] * self.kernel_size[1]
         if (fused is None and 2 * rows[0].numel() >= n_copies and events.shape[0] == inputs["time"].shape[0]
                 and self._train_ok(events)):
-            out = self.norm(self._forward_train(inputs, events, rows))
+            out = self._forward_train(inputs, events, rows)
+            out = (RowNormFunction.apply(out, self.norm.weight, self.norm.bias, self.norm.eps)
+                   if _plain_norm(self.norm, self.hidden_size, out.device) else self.norm(out))
             return {"events": out, "time": inputs["time"], "w": inputs["w"], "h": inputs["h"],
                     "batch_id": inputs["batch_id"], "lengths": lengths, "batch_size": inputs["batch_size"]}
         p_ev, p_pos, p_len = E.gather_rows(events, rows[0]), rows[2], rows[4]

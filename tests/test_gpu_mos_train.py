@@ -113,3 +113,47 @@ def test_mos_train_keeps_the_composed_path(dev):
         assert not _uses_train(layer(gr)["events"])
     layer.o_proj.register_forward_hook(lambda m, i, o: 2 * o)
     assert not _uses_train(layer(gr)["events"])
+
+
+@pytest.mark.parametrize("H", [1, 3, 15, 16, 17, 33, 48, 70, 96, 128])
+@pytest.mark.parametrize("n", [1, 17, 16 * 1024 + 1, 40000])
+def test_row_norm(dev, H, n):
+    """The LayerNorm kernels against float64, row counts about a workgroup's 16
+    and the 16,384 of a full grid.  u = 2^-24: a row's mean and moment are sums
+    of at most 8 + 4 terms in sequence, so y is within 16 u (|x| + |mean|) rstd
+    |w| + 2 u |b| and dx within 32 u of its terms; a weight gradient sums at
+    most 3 rows, 16 groups, 16 workgroups and 6 levels in sequence."""
+    from ssla_amd.layers import RowNormFunction
+    u, eps = 2.0 ** -24, 1e-5
+    gen = torch.Generator().manual_seed(H * 7 + n)
+    x = (torch.randn(n, H, generator=gen) * 2 + 1).to(dev).requires_grad_()
+    w, b = (torch.randn(H, generator=gen).to(dev).requires_grad_() for _ in range(2))
+    dy = torch.randn(n, H, generator=gen).to(dev)
+    y = RowNormFunction.apply(x, w, b, eps)
+    got = torch.autograd.grad(y, [x, w, b], dy, retain_graph=True)
+    assert all(torch.equal(p, q) for p, q in zip(got, torch.autograd.grad(y, [x, w, b], dy)))
+    X, W, Bi, D = (t.detach().double() for t in (x, w, b, dy))
+    mean = X.mean(1, keepdim=True)
+    rstd = ((X - mean).square().mean(1, keepdim=True) + eps).rsqrt()
+    h, g = (X - mean) * rstd, D * W
+    dh = 16 * u * (X.abs().amax(1, keepdim=True) + mean.abs()) * rstd * (1 + h.abs())   # bound on xhat's error
+    assert ((y.double() - (h * W + Bi)).abs() <= dh * W.abs() + 2 * u * Bi.abs() + 1e-30).all()
+    m1, m2 = g.mean(1, keepdim=True), (g * h).mean(1, keepdim=True)
+    ga, gh = g.abs().mean(1, keepdim=True), (g * h).abs().mean(1, keepdim=True)
+    bound = rstd * (32 * u * (g.abs() + ga + h.abs() * gh) + dh * gh + h.abs() * (g.abs() * dh).mean(1, keepdim=True))
+    assert ((got[0].double() - rstd * (g - m1 - h * m2)).abs() <= bound + dh * rstd * (g.abs() + ga)).all()
+    assert ((got[1].double() - (D * h).sum(0)).abs() <= 44 * u * (D * h).abs().sum(0) + (D.abs() * dh).sum(0)).all()
+    assert ((got[2].double() - D.sum(0)).abs() <= 44 * u * D.abs().sum(0)).all()
+
+
+def test_mos_train_hooked_norm(dev):
+    """A norm with a hook or of another type is called as a module."""
+    gr = _random_grouped(dev, C=8, seed=5)
+    gr["events"].requires_grad_()
+    layer = _layer(dev, 8, 12, 3)
+    y = layer(gr)["events"]
+    layer.norm.register_forward_hook(lambda m, i, o: 2 * o)
+    assert torch.allclose(layer(gr)["events"], 2 * y, rtol=1e-5, atol=1e-5)
+    layer.norm = torch.nn.Identity()
+    out = layer(gr)["events"]
+    assert _uses_train(out) and torch.allclose(torch.nn.functional.layer_norm(out, (12,)), y, rtol=1e-4, atol=1e-4)
