@@ -754,6 +754,17 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
     return __shfl(x, 16 * (r >> 2) + r);
   };
   f32x4 rq[2] = {zero, zero}, rk[2] = {zero, zero};   // intra-chunk parts of dq, dk (no diagonal, no scale)
+  // The pair (i, j) enters dq_i and dk_j with the same three factors,
+  // 2^(G_i - S_I) 2^(S_I - E_J) 2^(E_J - G_j): what each adds to dG then cancels
+  // but for the products' rounding (dg 1.2e-6 -> 0.7e-6 off fp64 at strong
+  // gates against other splits of the exponent in dq and in dk).
+  f32x4 fi[2], fj[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int kc = 32 * P + 16 * c + 4 * gq;
+    fi[c] = exp4(Gr[c] - ref4(&L.sS[I][kc]));
+    fj[c] = exp4(ref4(&L.sE[I][kc]) - Gr[c]);
+  }
   for (int J = 0; J <= I; ++J) {                      // dq: earlier rows j
     if (J == I && !diag) break;
     f32x4 da = zero;                                  // dA[i = r][j = 4 gq + x]
@@ -776,9 +787,10 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
       for (int c = 0; c < 2; ++c)
         part[c] = mfma4(L.tK[tix(16 * J + 4 * gq + x, 32 * P + 16 * c + r)], da[x], part[c]);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {   // 2^(G_i - E_J)
+    for (int c = 0; c < 2; ++c) {   // 2^(G_i - S_I) 2^(S_I - E_J)
       const int kc = 32 * P + 16 * c + 4 * gq;
-      rq[c] += exp4(J == I ? Gr[c] - ref4(&L.sE[I][kc]) : Gr[c] + between(L.sE, J, I, kc)) * part[c];
+      const f32x4 S = ref4(&L.sS[I][kc]);
+      rq[c] += (fi[c] * exp4(J == I ? S - ref4(&L.sE[I][kc]) : S + between(L.sE, J, I, kc))) * part[c];
     }
   }
   for (int B = I; B < 4; ++B) {                       // dk, dv: later rows i of block B
@@ -810,10 +822,10 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
       }
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {   // 2^(S_B - G_j)
+    for (int c = 0; c < 2; ++c) {   // 2^(E_I - G_j) 2^(S_B - E_I)
       const int kc = 32 * P + 16 * c + 4 * gq;
       const f32x4 S = ref4(&L.sS[B][kc]);
-      rk[c] += exp4(B == I ? S - Gr[c] : (ref4(&L.sE[I][kc]) - Gr[c]) + (between(L.sE, I, B, kc) + S)) * part[c];
+      rk[c] += (fj[c] * exp4(B == I ? S - ref4(&L.sE[I][kc]) : S + between(L.sE, I, B, kc))) * part[c];
     }
   }
   if (!diag) {
