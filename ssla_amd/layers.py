@@ -93,11 +93,18 @@ def _grouped_linear(x: torch.Tensor, pos: torch.Tensor, weights: torch.Tensor) -
 
 
 # ---------------------------------------------------------------- attention --
+def _called_as_is(m) -> bool:
+    """Calling the module runs its class's forward and nothing else: no hooks
+    of its own, none registered for all modules, no forward put on the
+    instance."""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__ or nn.modules.module._has_any_global_hook())
+
+
 def _plain_linear(m) -> bool:
     """An nn.Linear without a bias, a parametrization or hooks: its map is
     its weight alone."""
-    return (type(m) is nn.Linear and m.bias is None and not m._forward_hooks and not m._forward_pre_hooks
-            and not m._backward_hooks and not m._backward_pre_hooks)
+    return type(m) is nn.Linear and m.bias is None and _called_as_is(m)
 
 
 def _plain_norm(m, H, dev) -> bool:
@@ -105,8 +112,7 @@ def _plain_norm(m, H, dev) -> bool:
     hooks: the map of RowNormFunction."""
     return (type(m) is nn.LayerNorm and tuple(m.normalized_shape) == (H,) and H <= 128
             and all(p is not None and p.dtype == torch.float32 and p.device == dev for p in (m.weight, m.bias))
-            and not m._forward_hooks and not m._forward_pre_hooks and not m._backward_hooks
-            and not m._backward_pre_hooks)
+            and _called_as_is(m))
 
 
 class RowNormFunction(torch.autograd.Function):
