@@ -92,14 +92,26 @@ __device__ __forceinline__ void seq_bounds(const int64_t *cu, int n, int64_t T, 
   eos = min(max(cu[n + 1], bos), T);
 }
 
-// Chunks per segment of the state passes.  At C2 (4096 chunk-heads) 16
-// measured the same state-pass time as 8 with half the fold work
-// (fold 7.9 vs 12.8 us); 4 was slower.
-constexpr int kSegC = 16;
+// Chunks per segment.  A segment is one workgroup of the state passes and of
+// the walk (one of those per CU), which go through its chunks one after another
+// (4 and 13 us a chunk), so batches of up to 16 chunks per CU are spread over
+// all CUs once; at 16 for every size, 2,048 rows of H = 4 ran on 8 CUs
+// (forward and backward 236 us a call, 74 at one chunk; 16 ragged sequences of
+// 12,000 rows, H = 3: 286 -> 103; fp16, 4,096 rows, H = 4: 141 -> 94).  The fold
+// is serial over a sequence's segments, so where few heads leave it exposed it
+// bounds their number, 128 in a sequence of T rows (24,576 rows, H = 1: 276 ->
+// 148, fp16 193 -> 171).  From 16 chunks on longer segments stay: 8 x 4096 rows
+// at H = 8 took as long in the state passes at 8 and 5 us more in the fold.
+constexpr int kSegMax = 16, kCus = 256, kFoldMax = 128;
+inline int seg_chunks(int64_t T, int H) {
+  const int64_t chunks = (T + BT - 1) / BT;
+  const int64_t spread = (chunks * H + kCus - 1) / kCus, fold = (chunks + kFoldMax - 1) / kFoldMax;
+  return static_cast<int>(std::min<int64_t>(kSegMax, std::max<int64_t>(1, std::max(spread, fold))));
+}
 
 // coff[n] = chunks of sequences 0..n-1 and sgoff[n] = their segments of
-// kSegC chunks (coff[n_seq], sgoff[n_seq]: the totals).  One workgroup.
-__global__ __launch_bounds__(256) void bwd_offsets_kernel(const int64_t *__restrict__ cu, int n_seq, int64_t T,
+// `per` chunks (coff[n_seq], sgoff[n_seq]: the totals).  One workgroup.
+__global__ __launch_bounds__(256) void bwd_offsets_kernel(const int64_t *__restrict__ cu, int n_seq, int64_t T, int per,
                                                           int64_t *__restrict__ coff, int64_t *__restrict__ sgoff) {
   __shared__ int64_t pc[256], ps[256];
   int64_t carry_c = 0, carry_s = 0;
@@ -111,7 +123,7 @@ __global__ __launch_bounds__(256) void bwd_offsets_kernel(const int64_t *__restr
       seq_bounds(cu, n, T, bos, eos);
       c = (eos - bos + BT - 1) / BT;
     }
-    const int64_t sgc = (c + kSegC - 1) / kSegC;
+    const int64_t sgc = (c + per - 1) / per;
     pc[threadIdx.x] = c;
     ps[threadIdx.x] = sgc;
     __syncthreads();
@@ -138,7 +150,7 @@ __global__ __launch_bounds__(256) void bwd_offsets_kernel(const int64_t *__restr
 }
 
 // --------------------------------------------------------- state passes --
-// Each sequence's chunks are cut into segments of kSegC chunks.  A local
+// Each sequence's chunks are cut into segments of `per` chunks.  A local
 // pass runs every segment from a zero state (one workgroup per (segment,
 // head); wavefront w owns value columns 16 w .. 16 w + 15, lane l holds
 // keys 16 Kb + 4 (l / 16) + i of tile Kb, column l % 16):
@@ -199,7 +211,7 @@ template <bool REV, int DT, bool GF32>
 __device__ __forceinline__ void seg_pass(SmemP &sm, const int64_t bid, const uint16_t *__restrict__ X,
                                          const uint16_t *__restrict__ Y, const void *__restrict__ g,
                                          const int64_t *__restrict__ cu, const int64_t *__restrict__ coff,
-                                         const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V,
+                                         const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V, int per,
                                          float xscale, float *__restrict__ loc, float *__restrict__ dec,
                                          float *__restrict__ eloc, float *__restrict__ dtot) {
   const int tid = threadIdx.x;
@@ -212,8 +224,8 @@ __device__ __forceinline__ void seg_pass(SmemP &sm, const int64_t bid, const uin
   int64_t bos, eos;
   seq_bounds(cu, n, T, bos, eos);
   const int64_t nc = (eos - bos + BT - 1) / BT;
-  const int64_t j0 = (sg - sgoff[n]) * kSegC;   // first chunk of the segment in the sequence
-  const int m = static_cast<int>(min(static_cast<int64_t>(kSegC), nc - j0));
+  const int64_t j0 = (sg - sgoff[n]) * per;   // first chunk of the segment in the sequence
+  const int m = static_cast<int>(min(static_cast<int64_t>(per), nc - j0));
   const int64_t c0 = coff[n] + j0;              // its global chunk index
   const int v0 = 16 * w;
   const bool active = v0 < V;
@@ -349,16 +361,16 @@ __global__ __launch_bounds__(256) void bwd_seg_passes(const uint16_t *__restrict
                                                       const void *__restrict__ g, const int64_t *__restrict__ cu,
                                                       const int64_t *__restrict__ coff,
                                                       const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H,
-                                                      int V, float scale, int64_t nb, float *__restrict__ hloc,
+                                                      int V, int per, float scale, int64_t nb, float *__restrict__ hloc,
                                                       float *__restrict__ dfw, float *__restrict__ eloc,
                                                       float *__restrict__ dtot, float *__restrict__ dloc,
                                                       float *__restrict__ drv) {
   __shared__ SmemP sm;
   const int64_t b = blockIdx.x;
   if (b < nb)
-    seg_pass<false, DT, GF32>(sm, b, k, v, g, cu, coff, sgoff, n_seq, T, H, V, 1.f, hloc, dfw, eloc, dtot);
+    seg_pass<false, DT, GF32>(sm, b, k, v, g, cu, coff, sgoff, n_seq, T, H, V, per, 1.f, hloc, dfw, eloc, dtot);
   else
-    seg_pass<true, DT, GF32>(sm, b - nb, q, dout, g, cu, coff, sgoff, n_seq, T, H, V, scale, dloc, drv, nullptr,
+    seg_pass<true, DT, GF32>(sm, b - nb, q, dout, g, cu, coff, sgoff, n_seq, T, H, V, per, scale, dloc, drv, nullptr,
                              nullptr);
 }
 
@@ -369,11 +381,14 @@ __global__ __launch_bounds__(256) void bwd_seg_passes(const uint16_t *__restrict
 // entries per sequence (index sgoff[n] + n + s).
 __global__ __launch_bounds__(256) void bwd_fold_kernel(const int64_t *__restrict__ coff,
                                                        const int64_t *__restrict__ sgoff, int n_seq, int H, int V,
-                                                       const float *__restrict__ h0, const float *__restrict__ dht,
+                                                       int per, const float *__restrict__ h0,
+                                                       const float *__restrict__ dht,
                                                        const float *__restrict__ eloc, const float *__restrict__ dtot,
                                                        const float *__restrict__ dloc, float *__restrict__ sin_,
                                                        float *__restrict__ dsend, float *__restrict__ dh0) {
-  // one thread per (sequence, head, state element)
+  // one thread per (sequence, head, state element), blockIdx.y 0 the states, 1
+  // the gradients; kFold segments' values in flight per round trip
+  constexpr int kFold = 16;
   const int64_t KV = static_cast<int64_t>(KD) * V;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int64_t idx = gid % KV;
@@ -381,19 +396,43 @@ __global__ __launch_bounds__(256) void bwd_fold_kernel(const int64_t *__restrict
   const int n = static_cast<int>(gid / (KV * H));
   if (n >= n_seq) return;
   const int key = static_cast<int>(idx / V);
-  const int64_t sg0 = sgoff[n], nseg = sgoff[n + 1] - sg0;
+  const int64_t sg0 = sgoff[n], nseg = sgoff[n + 1] - sg0, c0 = coff[n];
   const int64_t o = (static_cast<int64_t>(n) * H + h) * KV + idx;
-  float S = h0 ? h0[o] : 0.f;
-  for (int64_t s = 0; s < nseg; ++s) {
-    sin_[((sg0 + n + s) * H + h) * KV + idx] = S;
-    S = cexp2(dtot[((sg0 + s) * H + h) * KD + key]) * S + eloc[((sg0 + s) * H + h) * KV + idx];
+  if (blockIdx.y == 0) {
+    float S = h0 ? h0[o] : 0.f;
+    for (int64_t s0 = 0; s0 < nseg; s0 += kFold) {
+      float d[kFold], e[kFold];
+  #pragma unroll
+      for (int u = 0; u < kFold; ++u) {
+        const int64_t s = min(s0 + u, nseg - 1);
+        d[u] = dtot[((sg0 + s) * H + h) * KD + key];
+        e[u] = eloc[((sg0 + s) * H + h) * KV + idx];
+      }
+  #pragma unroll
+      for (int u = 0; u < kFold; ++u) {
+        if (s0 + u >= nseg) break;
+        sin_[((sg0 + n + s0 + u) * H + h) * KV + idx] = S;
+        S = cexp2(d[u]) * S + e[u];
+      }
+    }
+    sin_[((sg0 + n + nseg) * H + h) * KV + idx] = S;
+    return;
   }
-  sin_[((sg0 + n + nseg) * H + h) * KV + idx] = S;
   float dS = dht ? dht[o] : 0.f;
-  for (int64_t s = nseg - 1; s >= 0; --s) {
-    dsend[((sg0 + s) * H + h) * KV + idx] = dS;
-    const int64_t cf = coff[n] + s * kSegC;
-    dS = cexp2(dtot[((sg0 + s) * H + h) * KD + key]) * dS + dloc[(cf * H + h) * KV + idx];
+  for (int64_t s0 = nseg - 1; s0 >= 0; s0 -= kFold) {
+    float d[kFold], e[kFold];
+#pragma unroll
+    for (int u = 0; u < kFold; ++u) {
+      const int64_t s = max(s0 - u, (int64_t)0);
+      d[u] = dtot[((sg0 + s) * H + h) * KD + key];
+      e[u] = dloc[((c0 + s * per) * H + h) * KV + idx];
+    }
+#pragma unroll
+    for (int u = 0; u < kFold; ++u) {
+      if (s0 - u < 0) break;
+      dsend[((sg0 + s0 - u) * H + h) * KV + idx] = dS;
+      dS = cexp2(d[u]) * dS + e[u];
+    }
   }
   if (dh0) dh0[o] = dS;
 }
@@ -430,7 +469,7 @@ template <int DT, bool GF32>
 __global__ __launch_bounds__(64 * kCW) void bwd_chunk_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     const void *__restrict__ g, const uint16_t *__restrict__ dout, const int64_t *__restrict__ cu,
-    const int64_t *__restrict__ coff, const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V,
+    const int64_t *__restrict__ coff, const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V, int per,
     float scale, const float *__restrict__ hloc, const float *__restrict__ dfw, const float *__restrict__ dloc,
     const float *__restrict__ drv, const float *__restrict__ sin_, const float *__restrict__ dsend,
     uint16_t *__restrict__ dq, uint16_t *__restrict__ dk, uint16_t *__restrict__ dv, void *__restrict__ dg) {
@@ -454,8 +493,9 @@ __global__ __launch_bounds__(64 * kCW) void bwd_chunk_kernel(
   const int VP = (V + 31) & ~31;
   // states of this chunk: local part + 2^decay * carried part (per key)
   const int64_t nc = (eos - bos + BT - 1) / BT;
-  const int64_t sgi = sgoff[n] + j / kSegC;
-  const bool last_in_seg = (j % kSegC) == kSegC - 1 || j == nc - 1;
+  const uint32_t jseg = static_cast<uint32_t>(j) / static_cast<uint32_t>(per);   // j < 2^31
+  const int64_t sgi = sgoff[n] + jseg;
+  const bool last_in_seg = j - static_cast<int64_t>(jseg) * per == per - 1 || j == nc - 1;
   const float *sin_c = sin_ + ((sgi + n) * H + h) * KV;        // carried into this segment
   const float *sin_n = sin_ + ((sgi + n + 1) * H + h) * KV;    // carried into the next (or ht)
   const float *dsend_c = dsend + (sgi * H + h) * KV;           // gradient at this segment's end
@@ -895,7 +935,7 @@ template <bool REV, bool GF32>
 __device__ __forceinline__ void seg_pass_tiles(SmemT &sm, const int64_t bid, const uint16_t *__restrict__ X,
                                                const uint16_t *__restrict__ Y, const void *__restrict__ g,
                                                const int64_t *__restrict__ cu, const int64_t *__restrict__ coff,
-                                               const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V,
+                                               const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V, int per,
                                                float xscale, float *__restrict__ loc, float *__restrict__ dec,
                                                float *__restrict__ eloc, float *__restrict__ dtot) {
   const int tid = threadIdx.x;
@@ -907,8 +947,8 @@ __device__ __forceinline__ void seg_pass_tiles(SmemT &sm, const int64_t bid, con
   int64_t bos, eos;
   seq_bounds(cu, n, T, bos, eos);
   const int64_t nc = (eos - bos + BT - 1) / BT;
-  const int64_t j0 = (sg - sgoff[n]) * kSegC;
-  const int m = static_cast<int>(min(static_cast<int64_t>(kSegC), nc - j0));
+  const int64_t j0 = (sg - sgoff[n]) * per;
+  const int m = static_cast<int>(min(static_cast<int64_t>(per), nc - j0));
   const int64_t c0 = coff[n] + j0;
   const int v0 = 16 * w;
   const bool active = v0 < V;
@@ -1062,15 +1102,15 @@ __global__ __launch_bounds__(256) void bwd_seg_passes_tiles(const uint16_t *__re
                                                             const int64_t *__restrict__ cu,
                                                             const int64_t *__restrict__ coff,
                                                             const int64_t *__restrict__ sgoff, int n_seq, int64_t T,
-                                                            int H, int V, float scale, int64_t nb,
+                                                            int H, int V, int per, float scale, int64_t nb,
                                                             float *__restrict__ eloc, float *__restrict__ dtot,
                                                             float *__restrict__ dloc, float *__restrict__ drv) {
   __shared__ SmemT sm;
   const int64_t b = blockIdx.x;
   if (b < nb)
-    seg_pass_tiles<false, GF32>(sm, b, k, v, g, cu, coff, sgoff, n_seq, T, H, V, 1.f, nullptr, nullptr, eloc, dtot);
+    seg_pass_tiles<false, GF32>(sm, b, k, v, g, cu, coff, sgoff, n_seq, T, H, V, per, 1.f, nullptr, nullptr, eloc, dtot);
   else
-    seg_pass_tiles<true, GF32>(sm, b - nb, q, dout, g, cu, coff, sgoff, n_seq, T, H, V, scale, dloc, drv, nullptr,
+    seg_pass_tiles<true, GF32>(sm, b - nb, q, dout, g, cu, coff, sgoff, n_seq, T, H, V, per, scale, dloc, drv, nullptr,
                                nullptr);
 }
 
@@ -1334,7 +1374,7 @@ template <bool GF32>
 __global__ __launch_bounds__(64 * kWW) void bwd_walk_kernel(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
     const void *__restrict__ g, const uint16_t *__restrict__ dout, const int64_t *__restrict__ cu,
-    const int64_t *__restrict__ coff, const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V,
+    const int64_t *__restrict__ coff, const int64_t *__restrict__ sgoff, int n_seq, int64_t T, int H, int V, int per,
     float scale, const float *__restrict__ dloc, const float *__restrict__ drv, const float *__restrict__ sin_,
     const float *__restrict__ dsend, uint16_t *__restrict__ dq, uint16_t *__restrict__ dk, uint16_t *__restrict__ dv,
     void *__restrict__ dg) {
@@ -1350,8 +1390,8 @@ __global__ __launch_bounds__(64 * kWW) void bwd_walk_kernel(
   int64_t bos, eos;
   seq_bounds(cu, n, T, bos, eos);
   const int64_t nc = (eos - bos + BT - 1) / BT;
-  const int64_t j0 = (sg - sgoff[n]) * kSegC;   // first chunk of the segment in the sequence
-  const int m = static_cast<int>(min(static_cast<int64_t>(kSegC), nc - j0));
+  const int64_t j0 = (sg - sgoff[n]) * per;   // first chunk of the segment in the sequence
+  const int m = static_cast<int>(min(static_cast<int64_t>(per), nc - j0));
   const int64_t c0 = coff[n] + j0;              // its global chunk index
   const int64_t KV = static_cast<int64_t>(KD) * V;
 
@@ -1575,7 +1615,8 @@ struct BwdWs {
 inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 inline BwdWs bwd_ws(char *base, int n_seq, int64_t T, int H, int V) {
   const int64_t cmax = (T + BT - 1) / BT + n_seq;                  // chunks
-  const int64_t smax = (cmax + kSegC - 1) / kSegC + n_seq;         // segments
+  const int per = seg_chunks(T, H);
+  const int64_t smax = (cmax + per - 1) / per + n_seq;             // segments
   const size_t kv = static_cast<size_t>(H) * KD * V * sizeof(float), kk = static_cast<size_t>(H) * KD * sizeof(float);
   BwdWs w;
   size_t p = 0;
@@ -1606,30 +1647,31 @@ int launch_bwd(const void *q, const void *k, const void *v, const void *g, const
   const auto *Kp = static_cast<const uint16_t *>(k);
   const auto *Vp = static_cast<const uint16_t *>(v);
   const auto *DO = static_cast<const uint16_t *>(dout);
-  hipLaunchKernelGGL(bwd_offsets_kernel, dim3(1), dim3(256), 0, st, cu, n_seq, T, w.coff, w.sgoff);
+  const int per = seg_chunks(T, H);
+  hipLaunchKernelGGL(bwd_offsets_kernel, dim3(1), dim3(256), 0, st, cu, n_seq, T, per, w.coff, w.sgoff);
   const int64_t cmax = (T + BT - 1) / BT + n_seq;
-  const int64_t smax = (cmax + kSegC - 1) / kSegC + n_seq;
+  const int64_t smax = (cmax + per - 1) / per + n_seq;
   const int64_t nb = smax * H;
   // bf16: the walking chunk pass carries the forward state, so the forward
   // local pass keeps only its segment end states
   constexpr bool kWalk = DT == SSLA_BF16;
   if constexpr (kWalk)
     hipLaunchKernelGGL((bwd_seg_passes_tiles<GF32>), dim3(static_cast<unsigned>(2 * nb)), dim3(256), 0, st, Kp, Vp, Q,
-                       DO, g, cu, w.coff, w.sgoff, n_seq, T, H, V, scale, nb, w.eloc, w.dtot, w.dloc, w.drv);
+                       DO, g, cu, w.coff, w.sgoff, n_seq, T, H, V, per, scale, nb, w.eloc, w.dtot, w.dloc, w.drv);
   else
     hipLaunchKernelGGL((bwd_seg_passes<DT, GF32>), dim3(static_cast<unsigned>(2 * nb)), dim3(256), 0, st, Kp, Vp, Q,
-                       DO, g, cu, w.coff, w.sgoff, n_seq, T, H, V, scale, nb, w.hloc, w.dfw, w.eloc, w.dtot, w.dloc,
+                       DO, g, cu, w.coff, w.sgoff, n_seq, T, H, V, per, scale, nb, w.hloc, w.dfw, w.eloc, w.dtot, w.dloc,
                        w.drv);
   const int64_t fold_threads = static_cast<int64_t>(n_seq) * H * KD * V;
-  hipLaunchKernelGGL(bwd_fold_kernel, dim3(static_cast<unsigned>((fold_threads + 255) / 256)), dim3(256), 0, st,
-                     w.coff, w.sgoff, n_seq, H, V, h0, dht, w.eloc, w.dtot, w.dloc, w.sin_, w.dsend, dh0);
+  hipLaunchKernelGGL(bwd_fold_kernel, dim3(static_cast<unsigned>((fold_threads + 255) / 256), 2), dim3(256), 0, st,
+                     w.coff, w.sgoff, n_seq, H, V, per, h0, dht, w.eloc, w.dtot, w.dloc, w.sin_, w.dsend, dh0);
   if constexpr (kWalk) {
     hipLaunchKernelGGL((bwd_walk_kernel<GF32>), dim3(static_cast<unsigned>(nb)), dim3(64 * kWW), 0, st, Q, Kp, Vp, g,
-                       DO, cu, w.coff, w.sgoff, n_seq, T, H, V, scale, w.dloc, w.drv, w.sin_, w.dsend,
+                       DO, cu, w.coff, w.sgoff, n_seq, T, H, V, per, scale, w.dloc, w.drv, w.sin_, w.dsend,
                        static_cast<uint16_t *>(dq), static_cast<uint16_t *>(dk), static_cast<uint16_t *>(dv), dg);
   } else {
     hipLaunchKernelGGL((bwd_chunk_kernel<DT, GF32>), dim3(static_cast<unsigned>(cmax * H)), dim3(64 * kCW), 0, st, Q,
-                       Kp, Vp, g, DO, cu, w.coff, w.sgoff, n_seq, T, H, V, scale, w.hloc, w.dfw, w.dloc, w.drv,
+                       Kp, Vp, g, DO, cu, w.coff, w.sgoff, n_seq, T, H, V, per, scale, w.hloc, w.dfw, w.dloc, w.drv,
                        w.sin_, w.dsend, static_cast<uint16_t *>(dq), static_cast<uint16_t *>(dk),
                        static_cast<uint16_t *>(dv), dg);
   }

@@ -81,7 +81,7 @@ def _gpu_grads(dev, q, k, v, g, cu, s0, do, dht, scale):
     return out
 
 
-def _check(dev, lens, H, V, dtype, seed, gate="logsig", h0=True, scale=64 ** -0.5, tag="", case=None, K=64):
+def _check(dev, lens, H, V, dtype, seed, gate="logsig", h0=True, scale=64 ** -0.5, tag="", case=None, K=64, rtol=0.0):
     q, k, v, g, cu, s0, do, dht = _inputs(lens, H, V, dtype, seed, gate, h0, K=K)
     print(f"gla bwd {tag}: lens={lens} H={H} V={V} {dtype} gate={gate} h0={h0}", flush=True)
     got = _gpu_grads(dev, q, k, v, g, cu, s0, do, dht, scale)
@@ -94,7 +94,7 @@ def _check(dev, lens, H, V, dtype, seed, gate="logsig", h0=True, scale=64 ** -0.
             assert a is None
             continue
         band, ratio_max = bands[name]
-        assert_close(a, b, 0.0, f"{name}[{tag}]", band=band, ratio_max=ratio_max)
+        assert_close(a, b, rtol, f"{name}[{tag}]", band=band, ratio_max=ratio_max)
 
 
 @pytest.mark.parametrize("V", [16, 32, 48, 64])
@@ -114,6 +114,25 @@ def test_chunk_bwd_long_sequences(dev):
     """Two 4096-token sequences (64 chunks each), H = 4: the state passes
     carry 64 chunks."""
     _check(dev, [4096, 4096], 4, 64, torch.bfloat16, seed=5, tag="long", case="long")
+
+
+@pytest.mark.parametrize("lens,H,dtype", [
+    ([700, 0, 65, 1], 1, torch.bfloat16),          # a chunk per segment, more of them than one fold batch of 8
+    ([300, 129], 2, torch.float16),
+    ([8130, 190], 1, torch.bfloat16),              # bounded by the fold: 131 chunks, two per segment, odd counts
+    ([2500, 64 * 6 + 1, 1300], 13, torch.bfloat16),   # four chunks per segment, partial last ones
+    ([1100, 640], 33, torch.float16),
+])
+def test_chunk_bwd_segments(dev, lens, H, dtype):
+    """Segment lengths other than 16 chunks, in the bands of the tested gates
+    (logsig for bf16, fp16): the segments' states are fp32 whatever their
+    length.  The bands are of smaller cases; among a million elements larger
+    ones occur, whose rounding to 16 bits is up to 2^-9 (bf16) or 2^-11 (fp16)
+    of the element itself: dv of 13 to 16 is 2^-8 = 0.0039 off in fp16, one in
+    [16, 32) up to 0.0078."""
+    bf16 = dtype == torch.bfloat16
+    _check(dev, lens, H, 32, dtype, seed=H, tag=f"segments {lens} H={H}", case="logsig" if bf16 else "fp16",
+           rtol=2.0 ** -9 if bf16 else 2.0 ** -11)
 
 
 @pytest.mark.parametrize("K", [32, 128])
