@@ -34,6 +34,8 @@
 // Exponents are clamped to +-126.  Products run on v_mfma_f32_16x16x32_bf16
 // as split bf16 products (see mmax) with fp32 accumulation; states, A, dA
 // and dg are fp32.
+#include <type_traits>
+
 #include "lds_tile.h"
 
 namespace ssla {
@@ -97,10 +99,10 @@ __device__ __forceinline__ void seq_bounds(const int64_t *cu, int n, int64_t T, 
 // (4 and 13 us a chunk), so batches of up to 16 chunks per CU are spread over
 // all CUs once; at 16 for every size, 2,048 rows of H = 4 ran on 8 CUs
 // (forward and backward 236 us a call, 74 at one chunk; 16 ragged sequences of
-// 12,000 rows, H = 3: 286 -> 103; fp16, 4,096 rows, H = 4: 141 -> 94).  The fold
+// 12,000 rows, H = 3: 286 -> 100; fp16, 4,096 rows, H = 4: 141 -> 82).  The fold
 // is serial over a sequence's segments, so where few heads leave it exposed it
 // bounds their number, 128 in a sequence of T rows (24,576 rows, H = 1: 276 ->
-// 148, fp16 193 -> 171).  From 16 chunks on longer segments stay: 8 x 4096 rows
+// 123, fp16 193 -> 144).  From 16 chunks on longer segments stay: 8 x 4096 rows
 // at H = 8 took as long in the state passes at 8 and 5 us more in the fold.
 constexpr int kSegMax = 16, kCus = 256, kFoldMax = 128;
 inline int seg_chunks(int64_t T, int H) {
@@ -387,8 +389,8 @@ __global__ __launch_bounds__(256) void bwd_fold_kernel(const int64_t *__restrict
                                                        const float *__restrict__ dloc, float *__restrict__ sin_,
                                                        float *__restrict__ dsend, float *__restrict__ dh0) {
   // one thread per (sequence, head, state element), blockIdx.y 0 the states, 1
-  // the gradients; kFold segments' values in flight per round trip
-  constexpr int kFold = 16;
+  // the gradients; 16 segments' values in flight per round trip, 4 for the rest
+  // (16 throughout cost 3 us where sequences have 4 segments)
   const int64_t KV = static_cast<int64_t>(KD) * V;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int64_t idx = gid % KV;
@@ -398,43 +400,34 @@ __global__ __launch_bounds__(256) void bwd_fold_kernel(const int64_t *__restrict
   const int key = static_cast<int>(idx / V);
   const int64_t sg0 = sgoff[n], nseg = sgoff[n + 1] - sg0, c0 = coff[n];
   const int64_t o = (static_cast<int64_t>(n) * H + h) * KV + idx;
-  if (blockIdx.y == 0) {
-    float S = h0 ? h0[o] : 0.f;
-    for (int64_t s0 = 0; s0 < nseg; s0 += kFold) {
-      float d[kFold], e[kFold];
-  #pragma unroll
-      for (int u = 0; u < kFold; ++u) {
-        const int64_t s = min(s0 + u, nseg - 1);
-        d[u] = dtot[((sg0 + s) * H + h) * KD + key];
-        e[u] = eloc[((sg0 + s) * H + h) * KV + idx];
-      }
-  #pragma unroll
-      for (int u = 0; u < kFold; ++u) {
-        if (s0 + u >= nseg) break;
-        sin_[((sg0 + n + s0 + u) * H + h) * KV + idx] = S;
-        S = cexp2(d[u]) * S + e[u];
-      }
-    }
-    sin_[((sg0 + n + nseg) * H + h) * KV + idx] = S;
-    return;
-  }
-  float dS = dht ? dht[o] : 0.f;
-  for (int64_t s0 = nseg - 1; s0 >= 0; s0 -= kFold) {
-    float d[kFold], e[kFold];
+  const bool rev = blockIdx.y == 1;
+  const float *init = rev ? dht : h0;
+  float S = init ? init[o] : 0.f;
+  // segment of step i; its decay, its own contribution, and where its entering
+  // state (or the gradient at its end) goes
+  auto batch = [&](auto width, int64_t i0) __attribute__((always_inline)) {
+    constexpr int W = decltype(width)::value;
+    float d[W], e[W];
 #pragma unroll
-    for (int u = 0; u < kFold; ++u) {
-      const int64_t s = max(s0 - u, (int64_t)0);
+    for (int u = 0; u < W; ++u) {
+      const int64_t i = min(i0 + u, nseg - 1), s = rev ? nseg - 1 - i : i;
       d[u] = dtot[((sg0 + s) * H + h) * KD + key];
-      e[u] = dloc[((c0 + s * per) * H + h) * KV + idx];
+      e[u] = rev ? dloc[((c0 + s * per) * H + h) * KV + idx] : eloc[((sg0 + s) * H + h) * KV + idx];
     }
 #pragma unroll
-    for (int u = 0; u < kFold; ++u) {
-      if (s0 - u < 0) break;
-      dsend[((sg0 + s0 - u) * H + h) * KV + idx] = dS;
-      dS = cexp2(d[u]) * dS + e[u];
+    for (int u = 0; u < W; ++u) {
+      const int64_t i = i0 + u, s = rev ? nseg - 1 - i : i;
+      if (i >= nseg) break;
+      if (rev) dsend[((sg0 + s) * H + h) * KV + idx] = S;
+      else sin_[((sg0 + n + s) * H + h) * KV + idx] = S;
+      S = cexp2(d[u]) * S + e[u];
     }
-  }
-  if (dh0) dh0[o] = dS;
+  };
+  int64_t i0 = 0;
+  for (; i0 + 16 <= nseg; i0 += 16) batch(std::integral_constant<int, 16>{}, i0);
+  for (; i0 < nseg; i0 += 4) batch(std::integral_constant<int, 4>{}, i0);
+  if (!rev) sin_[((sg0 + n + nseg) * H + h) * KV + idx] = S;
+  else if (dh0) dh0[o] = S;
 }
 
 // ------------------------------------------------------------ chunk pass --
