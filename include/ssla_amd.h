@@ -88,9 +88,7 @@ int ssla_status_read(const int32_t *status, int *value_out, void *stream);
  * initialisation needed) holds one bf16 hi / lo state pair (as the
  * reference stores its per-chunk states, ops/gla/chunk.py:933) and one
  * fp32 decay row per segment.  A size of 0
- * means no workspace is needed for this shape (pass NULL, 0); a batch of so
- * many sequences that one segment each fills the GPU is cut only to balance
- * ragged lengths, and runs uncut when the workspace is not given. */
+ * means no workspace is needed for this shape (pass NULL, 0). */
 size_t ssla_gla_chunk_workspace_size(int n_seq, int64_t T, int H, int K, int V);
 
 int ssla_gla_chunk_fwd(const void *q, const void *k, const void *v,

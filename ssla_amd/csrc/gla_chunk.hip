@@ -1013,9 +1013,11 @@ inline int pick_nvt(int V) {
 // Segments: about two workgroups per CU (256 CUs), at least two chunks per
 // segment, at most 64 segments per average sequence, and for sequences of
 // equal length a count that leaves no segment empty.  `per` chunks each; a
-// batch whose average sequence is one segment of fewer than 16 chunks is not
-// cut at all (per = 0): the state pass's launch would cost about what its
-// longer sequences' walks do.
+// batch whose average sequence is one segment is not cut at all (per = 0): its
+// chains fill the GPU as they are, and a whole walk carries the state in fp32
+// where a cut hands it on in 16 bits.  (Cutting only the longer sequences of
+// such a batch would balance ragged lengths at that price, and make the
+// allocation-free entry, which has no scratch for them all, round otherwise.)
 struct Segments {
   int P, per;      // segments of an average sequence, chunks of a segment (0: uncut)
   int64_t stores;  // workspace slots per (head, key group)
@@ -1034,10 +1036,9 @@ inline Segments pick_segments(int n_seq, int64_t T, int H, int V) {
     per = (avg_chunks + p - 1) / p;
     p = (avg_chunks + per - 1) / per;
   }
-  // one sequence of T rows is exactly T / n_seq long: nothing to balance
-  if (p == 1 && (per < 16 || n_seq == 1)) return {1, 0, 0};
+  if (p == 1) return {1, 0, 0};
   // every stored segment is whole and has a successor: at most (T - 1) / unit
-  const int64_t stores = std::max<int64_t>(p > 1 ? n_seq * p : 0, (T - 1) / (BT * per));
+  const int64_t stores = std::max<int64_t>(n_seq * p, (T - 1) / (BT * per));
   return {static_cast<int>(p), static_cast<int>(per), stores};
 }
 
@@ -1137,11 +1138,7 @@ int chunk_fwd(const void *q, const void *k, const void *v, const void *g, int g_
   const int KG = K > KD ? 2 : 1;
   FwdArgs f = {q, k, v, g, cu_seqlens, n_seq, T, H, K, V, scale, h0, o, ht, pick_segments(n_seq, T, H, V), nullptr,
                nullptr, nullptr, static_cast<hipStream_t>(stream)};
-  size_t need = workspace_bytes_for(f.sg, H, KG, V);
-  if (f.sg.P == 1 && (workspace == nullptr || workspace_bytes < need)) {
-    f.sg = {1, 0, 0};   // cut only to balance a ragged batch: runs uncut without its workspace
-    need = 0;
-  }
+  const size_t need = workspace_bytes_for(f.sg, H, KG, V);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_error("gla_chunk_fwd: workspace of %zu bytes needed (ssla_gla_chunk_workspace_size), %zu given",
               need, workspace_bytes);
@@ -1264,8 +1261,7 @@ extern "C" int ssla_gla_chunk_fwd_noalloc(const void *q, const void *k, const vo
                                           float *ht, int dtype, void *stream) {
   using namespace ssla;
   clear_error();
-  size_t need = ssla_gla_chunk_workspace_size(n_seq, T, H, K, V);
-  if (need > kNoallocScratchBytes && pick_segments(n_seq, T, H, V).P == 1) need = 0;   // runs uncut
+  const size_t need = ssla_gla_chunk_workspace_size(n_seq, T, H, K, V);
   if (need > kNoallocScratchBytes) {
     set_error("gla_chunk_fwd_noalloc: this shape needs %zu bytes of workspace, the static scratch holds %zu "
               "(call ssla_gla_chunk_fwd with a workspace)", need, kNoallocScratchBytes);

@@ -82,6 +82,11 @@ def test_chunk_forward_workspace_layout():
     assert lib.ssla_gla_chunk_workspace_size(1, 64, 8, 64, 64) == 0
     assert lib.ssla_gla_chunk_workspace_size(1, 4096, 8, 32, 64) == 0
     assert lib.ssla_gla_chunk_workspace_size(1, 4096, 8, 64, 40) == 0
+    # sequences and heads that fill the GPU as they are stay whole
+    for n, T, H, K, V in ((64, 64 * 1024, 8, 64, 16), (512, 512 * 1024, 8, 64, 64), (3, 2800, 512, 64, 16),
+                          (64, 70000, 8, 128, 64)):
+        size = lib.ssla_gla_chunk_workspace_size if K == 64 else lib.ssla_gla_chunk_wide_workspace_size
+        assert size(n, T, H, K, V) == 0
 
 
 def test_python_wrappers_reject_cpu_tensors():

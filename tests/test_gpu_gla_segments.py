@@ -4,8 +4,8 @@ can go wrong, against the fp64 recurrence in the bands of test_gpu_gla.py
 among short and empty ones (many segments of one chain, whose states fold
 over more than one batch of 8), leading rows outside every sequence, more
 sequences than one probe round of the slot search takes, key widths of one
-partial group, two groups and two calls, the cut that only balances ragged
-lengths (and the same call without its workspace, uncut)."""
+partial group, two groups and two calls, and batches that fill the GPU with
+whole sequences."""
 import numpy as np
 import pytest
 import torch
@@ -47,27 +47,44 @@ def test_segments(dev, lens, H, K, V, dtype, g16):
 
 def test_many_ragged_sequences(dev):
     """64 sequences x 8 heads of 1,024 rows on average (one segment each
-    fills the GPU), one of them 9,000 rows: cut to balance, and uncut when
-    the caller has no workspace."""
-    from ssla_amd import _lib
+    fills the GPU), one of them 9,000 rows: every sequence in one walk."""
     from ssla_amd.gla import chunk_gla
     rng = np.random.default_rng(0)
     lens = rng.integers(600, 1150, 63).tolist()
     lens = lens + [64 * 1024 - sum(lens)]
     q, k, v, g, cu, s0 = _inputs(lens, 8, 64, 16, torch.bfloat16, seed=9)
-    T = sum(lens)
-    lib = _lib.load()
-    assert lib.ssla_gla_chunk_workspace_size(64, T, 8, 64, 16) > 0
     print("many ragged sequences", flush=True)
     o, ht = _run(chunk_gla, q, k, v, g, cu, s0, 0.125, dev)
     ro, rht = _oracle(q, k, v, g, cu, s0, 0.125)
     for nm, a, b, bands in (("o", o, ro, O_BANDS), ("ht", ht, rht, HT_BANDS)):
         assert_close(a, b, 0.0, nm, band=bands["logsig"][0], ratio_max=bands["logsig"][1])
-    d = [t.to(dev) for t in (q, k, v, g, cu, s0)]
-    o2, ht2 = torch.empty_like(d[2]), torch.empty_like(d[5])
-    P = _lib.ptr
-    _lib.check(lib.ssla_gla_chunk_fwd(P(d[0]), P(d[1]), P(d[2]), P(d[3]), _lib.SSLA_F32, P(d[4]), 64, T, 8, 64, 16, 0.125,
-                                      P(d[5]), P(o2), P(ht2), _lib.SSLA_BF16, None, 0, _lib.stream_of(o2)), "fwd")
-    assert_close(o2.float().cpu().numpy(), ro, 0.0, "o, uncut", band=O_BANDS["logsig"][0],
-                 ratio_max=O_BANDS["logsig"][1])
-    assert_close(ht2.cpu().numpy(), rht, 0.0, "ht, uncut", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_full_batches_carry_the_state_in_fp32(dev, dtype):
+    """A ragged batch whose sequences and heads fill the GPU uncut: each
+    sequence's bits are those of a call of its own, which is one walk with the
+    state in fp32 (a cut would enter its segments from 16-bit states), and
+    the allocation-free entry's are the same."""
+    from ssla_amd import _lib
+    from ssla_amd.gla import chunk_gla
+    lens, H, V = [2500, 0, 300], 512, 16
+    gen = torch.Generator(device=dev).manual_seed(3)
+    T = sum(lens)
+    q, k = (torch.randn(T, H, 64, generator=gen, device=dev).to(dtype) for _ in range(2))
+    v = torch.randn(T, H, V, generator=gen, device=dev).to(dtype)
+    g = torch.nn.functional.logsigmoid(torch.randn(T, H, 64, generator=gen, device=dev)) / 16
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int64, device=dev)
+    print(f"full batch {dtype}", flush=True)
+    with torch.no_grad():
+        o, ht = chunk_gla(q, k, v, g, cu, output_final_state=True)
+        for n, (a, b) in enumerate(zip(cu.tolist(), cu.tolist()[1:])):
+            if b > a:
+                on, hn = chunk_gla(q[a:b], k[a:b], v[a:b], g[a:b], torch.tensor([0, b - a], device=dev),
+                                   output_final_state=True)
+                assert torch.equal(o[a:b], on) and torch.equal(ht[n], hn[0]), f"sequence {n}"
+    lib, P = _lib.load(), _lib.ptr
+    o2, ht2 = torch.empty_like(o), torch.empty_like(ht)
+    _lib.check(lib.ssla_gla_chunk_fwd_noalloc(P(q), P(k), P(v), P(g), _lib.SSLA_F32, P(cu), 3, T, H, 64, V, 64 ** -0.5,
+                                              None, P(o2), P(ht2), _lib.DTYPE_CODE[dtype], _lib.stream_of(o2)), "noalloc")
+    assert torch.equal(o2, o) and torch.equal(ht2, ht)
