@@ -248,14 +248,18 @@ __global__ __launch_bounds__(kThreads) void f32_fwd_kernel(
 // and the totals of the blocks between.  q~_i = q_i 2^(G_i - S_I) and
 // k~_j = k_j 2^(E_J - G_j) are staged once; a block pair takes the per-key factor 2^(S_I - E_J) on one
 // operand, or 2^(G_i - E_J) / 2^(S_I - G_j) on its result, all <= 1 for J < I.
-// For J = I the factor undoes at most the block's own decay: while |G - S_I|
-// stays within 40 (a factor of 2^80 between the extremes) every intermediate
-// is a normal number for inputs above 2^-46, and the block runs on the matrix
-// cores like the others; a chunk with a stronger decay (`slow`, uniform over
-// the workgroup) adds its diagonal blocks term by term, exponentials of
-// non-positive arguments only.
+// For J = I the factor undoes at most the block's own decay, and the block runs
+// on the matrix cores like the others while |G - S_I| stays within 40 and q and
+// k are zero or within 2^-46 .. 2^47: then q~, k~ and either of them times the
+// factor are normal numbers (exponents of at most 80 and 40).  Any other chunk
+// (`slow`, uniform over the workgroup) adds its diagonal blocks term by term,
+// from raw q and k with exponentials of non-positive arguments only -- and so
+// does one with an infinity or NaN in its rows (of v and dO as well): the
+// matrix cores multiply a masked zero with every row of the block, which would
+// carry it to rows before its own (after, in dk and dv).
 
 constexpr float kDiagRange = 40.f;
+constexpr uint32_t kInputMin = (127u - 46) << 23, kInputMax = (127u + 47) << 23;   // the bits of 2^-46, 2^47
 
 __device__ __forceinline__ int tix(int r, int c) { return r * 64 + ((((c >> 2) ^ (r & 15)) << 2) | (c & 3)); }
 __device__ __forceinline__ f32x4 row4(const float *t, int r, int c) {
@@ -472,15 +476,38 @@ __global__ __launch_bounds__(256) void f32_prefix_kernel(F32Args a) {
   }
 }
 
-// q~ / k~ of the thread's rows into their tiles; sets *slow where a key's
-// decay over a 16-row block leaves the range of the matrix-core diagonal.
+// Largest magnitude, and smallest but zero less one, of the values, as bit
+// patterns (an infinity or NaN is past kHuge).
+constexpr uint32_t kHuge = 0x7f7fffffu;
+struct Magnitudes {
+  uint32_t most = 0, least = 0xffffffffu;
+  template <int RPT>
+  __device__ __forceinline__ void add(const f32x4 (&x)[RPT]) {
+#pragma unroll
+    for (int m = 0; m < RPT; ++m)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float f = x[m][e];   // (a bit cast of the element itself reads element 0)
+        const uint32_t u = __builtin_bit_cast(uint32_t, f) & 0x7fffffffu;
+        most = max(most, u);
+        least = min(least, u - 1);
+      }
+  }
+};
+
+// q~ / k~ of the thread's rows into their tiles; sets *slow where one of them
+// (`most`: or another operand's largest magnitude) leaves the range of the
+// matrix-core diagonal.
 template <int RPT>
 __device__ __forceinline__ void stage_tilde(const f32x4 (&q)[RPT], const f32x4 (&k)[RPT], const f32x4 (&g)[RPT],
                                             const float (*sS)[64], const float (*sE)[64], int r0, int quad, float *tq,
-                                            float *tk, int *slow) {
+                                            float *tk, uint32_t most, int *slow) {
   const int B = r0 >> 4;
   const f32x4 S = ref4(&sS[B][4 * quad]), E = ref4(&sE[B][4 * quad]);
-  bool out = false;
+  Magnitudes qk;
+  qk.add(q);
+  qk.add(k);
+  bool out = (most > kHuge) | (qk.most > kInputMax) | (qk.least < kInputMin - 1);
 #pragma unroll
   for (int m = 0; m < RPT; ++m) {
     f32x4 a, b;
@@ -565,6 +592,8 @@ __global__ __launch_bounds__(256, 2) void f32_out_kernel(F32Args a) {
     s[m] = ref4(st + (r0 + m) * 64 + 4 * quad);
   }
   if (tid == 0) slow = 0;
+  Magnitudes of;
+  of.add(v);
   cumsum_rows<4>(g, wtot);
   stage_refs<4>(g, r0, quad, sS, sE);
 #pragma unroll
@@ -573,7 +602,7 @@ __global__ __launch_bounds__(256, 2) void f32_out_kernel(F32Args a) {
     put4(tS, r0 + m, 4 * quad, s[m]);
   }
   __syncthreads();
-  stage_tilde<4>(q, k, g, sS, sE, r0, quad, tQ, tK, &slow);
+  stage_tilde<4>(q, k, g, sS, sE, r0, quad, tQ, tK, of.most, &slow);
   __syncthreads();
   const int lane = tid & 63, I = tid >> 6, r = lane & 15, gq = lane >> 4;
   const bool diag = !slow;
@@ -628,11 +657,16 @@ __global__ __launch_bounds__(256, 2) void f32_out_kernel(F32Args a) {
       put4(tS, r0 + m, 4 * quad, g[m]);
     }
     __syncthreads();
-    const f32x4 p = diag_terms<false>(tQ, tK, tS, I, gq, r, K);
+    const f32x4 p = diag_terms<false>(tQ, tK, tS, I, gq, r, K);   // A[i = r][j = 4 gq + x]
+#pragma unroll 1
+    for (int jg = 0; jg < 4; ++jg)
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < 4; ++x) {
+        const float aij = __shfl(p[x], 16 * jg + r);
+        if (4 * jg + x > r) continue;   // later rows are left out, not multiplied by zero
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c] = mfma4(tV[tix(16 * I + 4 * gq + x, 16 * c + r)], p[x], acc[c]);
+        for (int c = 0; c < 4; ++c) acc[c] += aij * row4(tV, 16 * I + 4 * jg + x, 16 * c + 4 * gq);
+      }
   }
   if (16 * I + r < at.nc) {
     float *o = a.o + ((at.t0 + 16 * I + r) * a.H + h) * V;
@@ -691,6 +725,9 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
       dh[m] = ref4(sd + (r0 + m) * 64 + 4 * quad);
     }
     if (tid == 0) L.slow = 0;
+    Magnitudes of;
+    of.add(v);
+    of.add(d);
     cumsum_rows<2>(g, L.wtot);
     stage_refs<2>(g, r0, quad, L.sS, L.sE);
 #pragma unroll
@@ -708,7 +745,7 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
       if (quad == 15) L.sDgH[r0 + m] = s;
     }
     __syncthreads();
-    stage_tilde<2>(q, k, g, L.sS, L.sE, r0, quad, L.tQ, L.tK, &L.slow);
+    stage_tilde<2>(q, k, g, L.sS, L.sE, r0, quad, L.tQ, L.tK, of.most, &L.slow);
   }
   const int lane = tid & 63, w = tid >> 6, I = w >> 1, P = w & 1, r = lane & 15, gq = lane >> 4;
   const int i0 = 16 * I + r;                       // this lane's row
@@ -846,12 +883,16 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
 #pragma unroll
     for (int x = 0; x < 4; ++x) L.sDA[I][P][4 * gq + x][r] = da[x];
     __syncthreads();
-    const f32x4 A = diag_terms<true>(L.tQ, L.tK, L.tG, I, gq, r, K);
+    const f32x4 A = diag_terms<true>(L.tQ, L.tK, L.tG, I, gq, r, K);   // A[i = 4 gq + x][j = r]
+#pragma unroll 1
+    for (int ig = 0; ig < 4; ++ig)
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < 4; ++x) {
+        const float aij = __shfl(A[x], 16 * ig + r) * a.scale;
+        if (4 * ig + x < r) continue;   // earlier rows are left out, not multiplied by zero
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-        ov[c] = mfma4(L.tO[tix(16 * I + 4 * gq + x, 32 * P + 16 * c + r)], A[x] * a.scale, ov[c]);
+        for (int c = 0; c < 2; ++c) ov[c] += aij * row4(L.tO, 16 * I + 4 * ig + x, 32 * P + 16 * c + 4 * gq);
+      }
 #pragma unroll 1
     for (int j = 0; j < 16; ++j) {
       const int row = 16 * I + j;

@@ -92,3 +92,53 @@ def test_f32_dg_cancellation(dev):
     err = np.sqrt(np.square(leaf[3].grad.cpu().double().numpy() - ref).mean() / np.square(ref).mean())
     print(f"dg error {err:.2e}", flush=True)
     assert err <= 16 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("name", ["q", "k", "v", "do"])
+def test_f32_nonfinite_row_stays_causal(dev, name, bad):
+    """An infinity or NaN in one row reaches no row that does not depend on
+    it: with it in row t of v or k, o before t is finite and as without it,
+    in q o at every other row; in dO, dv after t, and in q, k or v the
+    gradients that no product with that row enters."""
+    from ssla_amd.gla import chunk_gla
+    n, t = 150, 64 + 21                       # inside the second chunk's second 16-row block
+    q, k, v, g, cu, h0 = _case([n], 0, 0, 2, 64, 64, 0.2, seed=11)
+    do = torch.randn(v.shape, generator=torch.Generator().manual_seed(12))
+    print(f"f32 {bad} in {name}", flush=True)
+
+    def run(poison):
+        x = {"q": q.clone(), "k": k.clone(), "v": v.clone(), "do": do.clone()}
+        if poison:
+            x[name][t, :, 5] = bad
+        leaf = [y.to(dev).requires_grad_() for y in (x["q"], x["k"], x["v"], g)]
+        o, _ = chunk_gla(*leaf, cu.to(dev), scale=0.3, initial_state=h0.to(dev), output_final_state=True)
+        return [y.detach().cpu().numpy() for y in (o, *torch.autograd.grad(o, leaf, x["do"].to(dev)))]
+    clean, got = run(False), run(True)
+    # rows of (o, dq, dk, dv) that the poisoned row has no part in
+    rows = {"q": (np.r_[0:t, t + 1:n], np.r_[0:t, t + 1:n], np.r_[t + 1:n], np.r_[t + 1:n]),
+            "k": (np.r_[0:t], np.r_[0:t], np.r_[0:t, t + 1:n], np.r_[0:t, t + 1:n]),
+            "v": (np.r_[0:t], np.r_[0:t], np.r_[0:t, t + 1:n], np.r_[0:n]),
+            "do": (np.r_[0:n], np.r_[0:t, t + 1:n], np.r_[t + 1:n], np.r_[t + 1:n])}[name]
+    for nm, a, b, r in zip(("o", "dq", "dk", "dv"), got, clean, rows):
+        assert_close(a[r], b[r], 1e-4, nm)
+    assert not np.isfinite(got[0][t:] if name != "do" else got[3][:t + 1]).all()
+
+
+@pytest.mark.parametrize("e", [-112, 112])
+def test_f32_wide_exponents(dev, e):
+    """q scaled by 2^e and k by 2^-e: where q~ or k~ would leave the normal
+    range under the block's decay (some 30 bits here) the diagonal is summed
+    term by term."""
+    from ssla_amd.gla import chunk_gla
+    q, k, v, g, cu, h0 = _case([130], 0, 0, 2, 64, 64, 2.0, seed=13)
+    do = torch.randn(v.shape, generator=torch.Generator().manual_seed(14))
+    ref = oracle.gla_recurrent_bwd(q.numpy(), k.numpy(), v.numpy(), g.numpy(), cu.numpy(), do.numpy(), 0.3)
+    ro, _ = oracle.gla_recurrent(q.numpy(), k.numpy(), v.numpy(), g.numpy(), cu.numpy(), 0.3)
+    print(f"f32 exponents {e}", flush=True)
+    leaf = [y.to(dev).requires_grad_() for y in (q * 2.0 ** e, k * 2.0 ** -e, v, g)]
+    o, _ = chunk_gla(*leaf, cu.to(dev), scale=0.3)
+    o.backward(do.to(dev))
+    assert_close(o.detach().cpu().numpy(), ro, 1e-4, "o")
+    for nm, y, r, x in zip(("dq", "dk", "dv", "dg"), leaf, ref, (e, -e, 0, 0)):
+        assert_close((y.grad.cpu().double() * 2.0 ** x).numpy(), r, 1e-4, nm)
