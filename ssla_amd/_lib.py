@@ -208,37 +208,66 @@ def stream_of(t: torch.Tensor) -> int:
 
 class HostWords:
     """Two int64 words of pinned host memory that a kernel writes, and the
-    event recorded behind it.  ``take`` hands one out, ``read`` waits for the
-    event (not for work queued after it), returns the words and puts the
-    object back; at most 16 per device are kept.  One caller owns an object
-    between the two, so threads and streams never share one."""
-    __slots__ = ("words", "event", "dev", "ptr", "handle")
+    event recorded behind it.  ``with HostWords.take(t) as w`` hands one out for
+    the calls that queue the write; ``w.read()`` waits for the event (not for
+    work queued after it), returns the words and puts the object back, at most
+    16 per device.  One caller owns an object in between, so threads and
+    streams never share one.  A block left without a read (a call in it raised)
+    waits for the device first: the memory is given back only once nothing
+    queued can write to it, and never if that cannot be told."""
+    __slots__ = ("words", "event", "dev", "ptr", "handle", "pending")
     _free: dict = {}
+    _lost: list = []
 
     def __init__(self, dev: int):
         with torch.cuda.device(dev):
             self.words = torch.zeros(2, dtype=torch.int64, pin_memory=True).numpy()
             self.event = torch.cuda.Event()
             self.event.record()   # creates it on this device
+        self.pending = False
         self.dev, self.ptr, self.handle = dev, self.words.ctypes.data, self.event.cuda_event
 
     @classmethod
     def take(cls, t: torch.Tensor) -> "HostWords":
         dev = t.get_device()
+        if torch.cuda.is_current_stream_capturing():
+            raise SslaError("an answer the host waits for cannot be read under graph capture")
         try:
             w = cls._free[dev].pop()   # (one bytecode-level call: safe between threads)
         except (KeyError, IndexError):
             w = cls(dev)
         w.words[:] = 0
+        w.pending = True
         return w
+
+    def _give_back(self):
+        self.pending = False
+        free = self._free.setdefault(self.dev, [])
+        if len(free) < 16:
+            free.append(self)
 
     def read(self):
         self.event.synchronize()
         out = int(self.words[0]), int(self.words[1])
-        free = self._free.setdefault(self.dev, [])
-        if len(free) < 16:
-            free.append(self)
+        self._give_back()
         return out
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        if self.pending:
+            # (the event may not have been recorded: wait for the device)
+            try:
+                torch.cuda.synchronize(self.dev)
+            except RuntimeError:   # the error on its way out says more
+                self._lost.append(self)
+                return
+            self._give_back()
+
+    def __del__(self):
+        if self.pending:
+            self._lost.append(self)
 
 
 class ParamWatch:

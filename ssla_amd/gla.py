@@ -345,16 +345,15 @@ def fused_recurrent_gla(
                          f"got {tuple(h0.shape)}")
     o = torch.empty(T, H, V, device=q.device, dtype=q.dtype)
     ht = torch.empty(N, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
-    # the bounds are queued ahead of the recurrence and read while it runs
-    bounds = None
     if N > 0 and cu_seqlens.is_cuda:
-        bounds = _lib.HostWords.take(cu)
-        _lib.check(_lib.load().ssla_seq_bounds_async(_lib.ptr(cu), N, bounds.ptr, bounds.handle, _lib.stream_of(cu)),
-                   "ssla_seq_bounds_async")
-    o, ht = _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
-    if bounds is not None:
-        lo, hi = bounds.read()
+        # the bounds are queued ahead of the recurrence and read while it runs
+        with _lib.HostWords.take(cu) as bounds:
+            _lib.check(_lib.load().ssla_seq_bounds_async(_lib.ptr(cu), N, bounds.ptr, bounds.handle,
+                                                         _lib.stream_of(cu)), "ssla_seq_bounds_async")
+            o, ht = _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
+            lo, hi = bounds.read()
     else:
+        o, ht = _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
         lo, hi = (int(x) for x in cu_seqlens[[0, -1]].tolist()) if N > 0 else (0, 0)
     if (lo, hi) != (0, T):
         o = o[lo:hi]

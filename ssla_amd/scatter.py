@@ -74,9 +74,10 @@ def _run(name, src, index, n_out, sorted_index, out, argmax, check):
     # The index is checked ahead of the reduction: this waits for the answer
     # while the reduction runs (waiting for the whole call left the device
     # idle through the next call's host work).
-    bad = _lib.HostWords.take(src)
-    _lib.check(fn(*args, bad.ptr, bad.handle, _lib.stream_of(src)), name)
-    if bad.read()[0] != 0:
+    with _lib.HostWords.take(src) as bad:
+        _lib.check(fn(*args, bad.ptr, bad.handle, _lib.stream_of(src)), name)
+        found = bad.read()[0]
+    if found != 0:
         raise ValueError(f"{name}: index out of range [0, {n_out})"
                          + (" or not sorted" if sorted_index else ""))
 
