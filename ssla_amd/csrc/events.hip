@@ -332,10 +332,13 @@ __global__ void clear_and_fill(int64_t *counts, int32_t *bad, int64_t *a, int64_
   GRID_STRIDE(i, nd) d[i] = vb;
 }
 
-// Sorted-fill set-up in one launch: inv and dst to -1, and the field
-// index / length rows of the plan copied to the outputs.
+// Sorted-fill set-up in one launch: inv and dst to -1, the counts of the piece
+// lists to 0 (n_lists of them, 16 words apart), and the field index / length
+// rows of the plan copied to the outputs.
 __global__ void rf_sorted_setup(int32_t *inv, int64_t n_inv, int32_t *dst, int64_t n_dst, int64_t *f_index,
-                                const int64_t *plan_index, int64_t *f_len, const int64_t *plan_len, int64_t n_act) {
+                                const int64_t *plan_index, int64_t *f_len, const int64_t *plan_len, int64_t n_act,
+                                uint64_t *counts, int n_lists) {
+  if (blockIdx.x == 0 && threadIdx.x < static_cast<unsigned>(n_lists)) counts[16 * threadIdx.x] = 0;
   GRID_STRIDE(i, n_inv) inv[i] = -1;
   GRID_STRIDE(i, n_dst) dst[i] = -1;
   GRID_STRIDE(i, n_act) {
@@ -1633,6 +1636,51 @@ __global__ void rf_merge(const int32_t *__restrict__ ev2g, const int64_t *__rest
   }
 }
 
+constexpr int kPiece = 64;
+struct MergeArgs {
+  const int64_t *f_index;   // the active fields
+  int64_t n_act;
+  const int32_t *pixmap;
+  const int64_t *gstart, *glen, *lut;
+  int64_t n_rf;
+  int A;
+  int64_t n_f, HW;
+  const int64_t *ev_pre, *time;
+  int64_t E_in, E_out;
+  int64_t *o_src, *o_time, *o_pos;
+  int32_t *dst_map;
+  // The large fields' pieces of kPiece rows, active index << 32 | piece, in
+  // n_lists (1 or 4) lists of cap words each, one per row, so any of them holds
+  // all; their counts lie 16 words apart.
+  uint64_t *pieces[4], *counts;
+  int n_lists;
+  int64_t cap;
+};
+// The run of position j in the field (of n events from event s); lanes past
+// the positions hold none.  Returns the field's first row.
+__device__ __forceinline__ int64_t field_run(const MergeArgs &m, int64_t i, int j, int &s, int &n) {
+  const int64_t f = i < m.n_act ? m.f_index[i] : -1;
+  const bool valid = f >= 0 && f < m.n_f;
+  s = n = 0;   // E_in < 2^28
+  if (valid && j < m.A) {
+    const uint32_t b = static_cast<uint32_t>(f) / static_cast<uint32_t>(m.n_rf);
+    const int64_t p = m.lut[(f - static_cast<int64_t>(b) * m.n_rf) * m.A + j];
+    const int32_t g = p >= 0 ? m.pixmap[b * m.HW + p] : -1;
+    if (g >= 0) {
+      s = static_cast<int>(min(max(m.gstart[g], (int64_t)0), m.E_in));
+      n = static_cast<int>(min(max(m.glen[g], (int64_t)0), m.E_in - s));
+    }
+  }
+  return valid ? m.ev_pre[f] : 0;
+}
+__device__ __forceinline__ void emit_row(const MergeArgs &m, int64_t row, int64_t e, int64_t t, int a) {
+  if (row < 0 || row >= m.E_out) return;   // inconsistent inputs: drop, never write out of range
+  m.o_src[row] = e;
+  if (m.o_time) m.o_time[row] = t;
+  m.o_pos[row] = a;
+  if (m.dst_map) m.dst_map[e * m.A + a] = static_cast<int32_t>(row);
+}
+
 // The same fill with 16 lanes per active field (at most 16 positions): lane
 // a looks up position a's run once, the field's rows (event, position, time)
 // are laid side by side in LDS, position by position, and a row's place is
@@ -1640,7 +1688,7 @@ __global__ void rf_merge(const int32_t *__restrict__ ev2g, const int64_t *__rest
 // them, where rf_merge makes every (event, position) pair look the other
 // positions' runs up again and search each.  A 3 x 3 field holds 7 rows on
 // average (400,000 events, 3.6 M rows): rf_merge 212 us, here 124.  Fields of
-// more than kFieldRows rows search the runs.
+// more than kFieldRows rows go to rf_merge_rows.
 // Bound by its instructions (some 300 per wavefront of four fields), so a row
 // carries one 64-bit key (time << 7 | place) and a place is one compare per
 // other row.
@@ -1656,30 +1704,14 @@ __device__ __forceinline__ void field_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__global__ __launch_bounds__(256) void rf_merge_fields(
-    const int64_t *__restrict__ f_index, int64_t n_act, const int32_t *__restrict__ pixmap,
-    const int64_t *__restrict__ gstart, const int64_t *__restrict__ glen, const int64_t *__restrict__ lut, int64_t n_rf,
-    int A, int64_t n_f, int64_t HW, const int64_t *__restrict__ ev_pre, const int64_t *__restrict__ time, int64_t E_in,
-    int64_t E_out, int64_t *__restrict__ o_src, int64_t *__restrict__ o_time, int64_t *__restrict__ o_pos,
-    int32_t *__restrict__ dst_map) {
+__global__ __launch_bounds__(256) void rf_merge_fields(MergeArgs m) {
   // (odd pitches: the four fields of a wavefront read different banks)
   __shared__ uint64_t s_t[16][kFieldRows + 1];   // time (clamped at 0) << 7 | row
   __shared__ uint32_t s_e[16][kFieldRows + 1];   // event << 4 | position
   const int j = threadIdx.x & 15, fl = threadIdx.x >> 4;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 16 + fl;
-  const int64_t f = i < n_act ? f_index[i] : -1;
-  const bool valid = f >= 0 && f < n_f;
-  const int64_t base = valid ? ev_pre[f] : 0;
-  int s = 0, n = 0;   // E_in < 2^28
-  if (valid && j < A) {
-    const uint32_t b = static_cast<uint32_t>(f) / static_cast<uint32_t>(n_rf);
-    const int64_t p = lut[(f - static_cast<int64_t>(b) * n_rf) * A + j];
-    const int32_t g = p >= 0 ? pixmap[b * HW + p] : -1;
-    if (g >= 0) {
-      s = static_cast<int>(min(max(gstart[g], (int64_t)0), E_in));
-      n = static_cast<int>(min(max(glen[g], (int64_t)0), E_in - s));
-    }
-  }
+  int s, n;
+  const int64_t base = field_run(m, i, j, s, n);
   const int nc = min(n, kFieldRows + 1);   // (no sum of a field's runs overflows)
   int off = nc;   // inclusive, then exclusive over the field's positions
   off += row_shr_i<1>(off);
@@ -1688,60 +1720,123 @@ __global__ __launch_bounds__(256) void rf_merge_fields(
   off += row_shr_i<8>(off);
   const int total = __shfl(off, 15, 16);
   off -= nc;
-  auto emit = [&](int64_t e, int64_t t, int a, int rank) {
-    const int64_t row = base + rank;
-    if (row < 0 || row >= E_out) return;   // inconsistent inputs: drop, never write out of range
-    o_src[row] = e;
-    if (o_time) o_time[row] = t;
-    o_pos[row] = a;
-    if (dst_map) dst_map[e * A + a] = static_cast<int32_t>(row);
-  };
-  bool late = total > kFieldRows;
+  bool late = total > kFieldRows;   // or, in this lane's rows, too late a time
   if (!late) {
     for (int k = 0; k < n; ++k) s_e[fl][off + k] = static_cast<uint32_t>(s + k) << 4 | static_cast<uint32_t>(j);
     field_sync();
     for (int r = j; r < total; r += 16) {
-      const int64_t t = time[s_e[fl][r] >> 4];
+      const int64_t t = m.time[s_e[fl][r] >> 4];
       late |= t >= kFieldTime;
       s_t[fl][r] = static_cast<uint64_t>(min(max(t, (int64_t)0), kFieldTime)) << 7 | static_cast<uint64_t>(r);
     }
     field_sync();
   }
-  // A field with more rows, or later times, than its keys hold goes by search.
-  if ((__builtin_amdgcn_ballot_w64(late) >> (threadIdx.x & 48) & 0xffff) == 0) {
+  // (more rows, or later times, than the keys hold: listed for rf_merge_rows)
+  const uint64_t any = __builtin_amdgcn_ballot_w64(late);
+  const bool large = any >> (threadIdx.x & 48) & 0xffff;
+  if (!large) {
     for (int r = j; r < total; r += 16) {
       const uint64_t key = s_t[fl][r];
       int rank = 0;
 #pragma unroll 4
       for (int q = 0; q < total; ++q) rank += s_t[fl][q] < key ? 1 : 0;
       const int64_t e = s_e[fl][r] >> 4, t = static_cast<int64_t>(key >> 7);
-      emit(e, o_time && t == 0 ? time[e] : t, static_cast<int>(s_e[fl][r] & 15), rank);
+      emit_row(m, base + rank, e, m.o_time && t == 0 ? m.time[e] : t, static_cast<int>(s_e[fl][r] & 15));
     }
-    return;
   }
-  for (int a = 0; a < A; ++a) {
-    const int sa = __shfl(s, a, 16), na = __shfl(n, a, 16);
-    for (int k0 = 0; k0 < na; k0 += 16) {
-      const bool in = k0 + j < na;
-      const int64_t e = sa + k0 + j;
-      const int64_t t = in ? time[e] : 0, tc = max(t, (int64_t)0);
-      int rank = k0 + j;
-      for (int a2 = 0; a2 < A; ++a2) {
-        const int s2 = __shfl(s, a2, 16);
-        int lo = 0, hi = __shfl(n, a2, 16);
-        if (a2 == a || !in) continue;
-        while (lo < hi) {   // elements < tc (<= tc for earlier positions)
-          const int mid = (lo + hi) >> 1;
-          const int64_t v = max(time[s2 + mid], (int64_t)0);
-          if (a2 < a ? v <= tc : v < tc)
-            lo = mid + 1;
-          else
-            hi = mid;
-        }
-        rank += lo;
+  if (any == 0) return;
+  // The large fields' pieces, one addition to a list's count per wavefront of
+  // four fields.  (One list for all: 11 us more for 4,225 such fields.)
+  long long rows = large ? n : 0;
+#pragma unroll
+  for (int d = 1; d < 16; d *= 2) rows += __shfl_xor(rows, d, 16);
+  const long long pieces = (rows + kPiece - 1) / kPiece;
+  long long before = 0, all = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const long long pq = __shfl(pieces, 16 * q);
+    if (q < (fl & 3)) before += pq;
+    all += pq;
+  }
+  const int list = static_cast<int>((threadIdx.x >> 6) & (m.n_lists - 1));
+  long long at = 0;
+  if ((threadIdx.x & 63) == 0)
+    at = static_cast<long long>(atomicAdd(reinterpret_cast<unsigned long long *>(m.counts + 16 * list),
+                                          static_cast<unsigned long long>(all)));
+  at = __shfl(at, 0) + before;
+  uint64_t *to = m.pieces[list];
+  for (long long u = j; u < pieces && at + u < m.cap; u += 16)
+    to[at + u] = static_cast<uint64_t>(i) << 32 | static_cast<uint64_t>(u);
+}
+
+// The rows of the large fields, a wavefront per piece: a lane finds its row's
+// run among the field's and its place by binary searches in the others, MB
+// positions at a time in lockstep as rf_merge does, but without its lookups.  A
+// hot pixel makes every field over it large, and walking such a field with its
+// own 16 lanes left its searches one after another: 3 x 3 fields over 506
+// neighbouring pixels of 50 events (50,000 events in all) took 321 us, here 35
+// (rf_merge 46); one pixel of 20,000 events 6.8 ms, here 24 us (rf_merge 45).
+// Without large fields the launch finds nothing to do: 2.5 of 17 us.
+constexpr int64_t kRowBlocks = 2048;
+template <int MB>
+__global__ __launch_bounds__(256) void rf_merge_rows(MergeArgs m) {
+  const int lane = threadIdx.x & 63, j = lane & 15;
+  const int64_t w = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), nw = static_cast<int64_t>(gridDim.x) * 4;
+  int64_t upto[4], n_pieces = 0;   // pieces of the lists up to each
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    if (l < m.n_lists) n_pieces += min(static_cast<int64_t>(m.counts[16 * l]), m.cap);
+    upto[l] = n_pieces;
+  }
+  for (int64_t it = w; it < n_pieces; it += nw) {
+    const uint64_t piece = it < upto[0]   ? m.pieces[0][it]
+                           : it < upto[1] ? m.pieces[1][it - upto[0]]
+                           : it < upto[2] ? m.pieces[2][it - upto[1]]
+                                          : m.pieces[3][it - upto[2]];
+    const int64_t r = static_cast<int64_t>(piece & 0xffffffffu) * kPiece + lane;
+    int s, n;
+    const int64_t base = field_run(m, static_cast<int64_t>(piece >> 32), j, s, n);
+    // the lane's row: event k of position a
+    int64_t off = 0, e = 0, rank = 0;
+    int a = -1;
+    for (int p = 0; p < m.A; ++p) {
+      const int np = __shfl(n, p), sp = __shfl(s, p);
+      if (r >= off && r < off + np) {
+        a = p;
+        rank = r - off;
+        e = sp + rank;
       }
-      if (in) emit(e, t, a, rank);
+      off += np;
     }
+    const int64_t t = a >= 0 ? m.time[e] : 0, tc = max(t, (int64_t)0);
+    for (int p0 = 0; p0 < m.A; p0 += MB) {
+      int s2[MB], lo[MB], hi[MB];
+#pragma unroll
+      for (int v = 0; v < MB; ++v) {
+        const int p = p0 + v, np = __shfl(n, p);   // (below 16: lanes past the positions hold empty runs)
+        s2[v] = __shfl(s, p);
+        lo[v] = 0;
+        hi[v] = p == a || a < 0 ? 0 : np;
+      }
+      bool more = true;
+      while (more) {
+        more = false;
+#pragma unroll
+        for (int v = 0; v < MB; ++v) {
+          if (lo[v] < hi[v]) {   // elements < tc (<= tc for earlier positions)
+            const int mid = (lo[v] + hi[v]) >> 1;
+            const int64_t x = max(m.time[s2[v] + mid], (int64_t)0);
+            const bool le = p0 + v < a ? x <= tc : x < tc;
+            lo[v] = le ? mid + 1 : lo[v];
+            hi[v] = le ? hi[v] : mid;
+            more = true;
+          }
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < MB; ++v) rank += lo[v];
+    }
+    if (a >= 0) emit_row(m, base + rank, e, t, a);
   }
 }
 }  // namespace
@@ -1976,14 +2071,25 @@ extern "C" int ssla_rf_scatter_fill_sorted(const int64_t *gr_batch, const int64_
   // one position has nothing to merge; past 16 a field's lanes would take several lookups each
   // (rf_merge needs the inverse table, rf_merge_fields none)
   const bool fields = A > 1 && A <= 16 && n_f < 0x7fffffff && E_in < (int64_t{1} << 28);
+  // (free here, E_cap words each: the sort fill's buffers)
+  const int n_lists = E_cap >= 256 ? 4 : 1;
+  uint64_t *counts = n_lists == 4 ? reinterpret_cast<uint64_t *>(L.perm) : reinterpret_cast<uint64_t *>(L.tmax);
+  const MergeArgs m = {L.f_index, n_act, L.pixmap, L.gstart, gr_len, lut, n_rf, A, n_f, HW, L.ev_pre, time, E_in, E_out,
+                       out_src, out_time, out_pos, dst_map,
+                       {L.key, L.skey, reinterpret_cast<uint64_t *>(L.pre_src), reinterpret_cast<uint64_t *>(L.pre_pos)},
+                       counts, n_lists, E_cap};
   hipLaunchKernelGGL(rf_sorted_setup, dim3(grid_for(std::max(std::max(fields ? 0 : HW * A, n_dst), n_act))),
                      dim3(kThreads), 0, st, inv, fields ? 0 : HW * A, dst_map, n_dst, f_index, L.f_index, f_len, L.f_len,
-                     n_act);
+                     n_act, counts, n_lists);
   if (fields) {
-    if (n_act > 0 && E_out > 0)
-      hipLaunchKernelGGL(rf_merge_fields, dim3(static_cast<unsigned>((n_act + 15) / 16)), dim3(256), 0, st, L.f_index,
-                         n_act, L.pixmap, L.gstart, gr_len, lut, n_rf, A, n_f, HW, L.ev_pre, time, E_in, E_out, out_src,
-                         out_time, out_pos, dst_map);
+    if (n_act > 0 && E_out > 0) {
+      hipLaunchKernelGGL(rf_merge_fields, dim3(static_cast<unsigned>((n_act + 15) / 16)), dim3(256), 0, st, m);
+      const dim3 rows(static_cast<unsigned>(std::min<int64_t>(kRowBlocks, (E_out + 255) / 256)));
+      if (A <= 4)
+        hipLaunchKernelGGL(rf_merge_rows<4>, rows, dim3(256), 0, st, m);
+      else
+        hipLaunchKernelGGL(rf_merge_rows<8>, rows, dim3(256), 0, st, m);
+    }
     return launch_status("rf_scatter_fill_sorted");
   }
   hipLaunchKernelGGL(rf_inv_lut, dim3(grid_for(n_rf * A)), dim3(kThreads), 0, st, lut, n_rf, A, HW, inv);

@@ -50,3 +50,43 @@ def test_field_fill_late_times(dev):
         assert rows == sorted(rows) and torch.equal(tim[at:at + m], gr["time"][src[at:at + m]])
         at += m
     assert at == src.numel() > 2 * n
+
+
+@pytest.mark.parametrize("kh,kw", [(1, 2), (2, 2), (1, 5), (3, 3), (4, 4)])
+@pytest.mark.parametrize("late", [0, 1 << 57])
+def test_large_fields(dev, kh, kw, late):
+    """Pixels of 1 to 5,000 events without a cap: fields of one to hundreds
+    of 64-row pieces, about the edges of a piece, beside small ones, two runs
+    of the same workspace; also with timestamps past a key's 56 bits."""
+    from ssla_amd import events as E
+    H, W = 12, 17
+    gen = torch.Generator().manual_seed(kh * 10 + kw)
+    cnt = torch.randint(0, 3, (H * W,), generator=gen)
+    for p, n in ((20, 97), (40, 128), (60, 129), (80, 191), (100, 192), (120, 193), (140, 5000), (141, 700), (158, 64)):
+        cnt[p] = n
+    pix = torch.nonzero(cnt).flatten()
+    ln = cnt[pix]
+    t = torch.randint(0, 300, (int(ln.sum()),), generator=gen)
+    gid = torch.repeat_interleave(torch.arange(pix.numel()), ln)
+    t = t[torch.argsort(gid * 300 + t, stable=True)] + late
+    gr = {"time": t.to(dev), "batch_id": torch.zeros_like(pix).to(dev), "h": (pix // W).to(dev), "w": (pix % W).to(dev),
+          "lengths": ln.to(dev), "batch_size": 1}
+    lut, _ = E.compute_rf2pixels((H, W), (kh, kw), (1, 1), device=dev)
+    print(f"large fields {kh}x{kw} late={late}", flush=True)
+    a = E._rf_scatter(gr, (H, W), lut, dst_map=True)
+    if late == 0:
+        b = E._rf_scatter(gr, (H, W), lut, force_sort=True)
+        for name, x, y in zip(("src", "time", "pos", "f_index", "f_len"), a[:5], b[:5]):
+            assert torch.equal(x, y), name
+        return
+    # (the radix keys do not hold such times with the field beside them)
+    src, tim, pos, f_len = (x.cpu() for x in (a[0], a[1], a[2], a[4]))
+    assert torch.equal(tim, t[src])
+    field = torch.repeat_interleave(torch.arange(f_len.numel()), f_len)
+    key = torch.stack([field, tim - late, pos, src])   # strictly increasing
+    d = key[:, 1:] - key[:, :-1]
+    first = (d != 0).int().argmax(0)
+    assert (d.gather(0, first[None]) > 0).all()
+    dst = a[6].cpu()
+    assert torch.equal(dst[src * kh * kw + pos], torch.arange(src.numel(), dtype=torch.int32))
+    assert int((dst >= 0).sum()) == src.numel()
