@@ -420,13 +420,14 @@ struct ChunkArgs {
 // Where a workgroup works.  Blocks go to the 8 XCDs in turn: the `inner` blocks
 // that read the same rows (V groups, key groups of the state pass) are placed
 // 8 apart, so they run on one XCD close in time and share its L2.  Beyond that
-// heads vary fastest, so every XCD runs every segment index of a sequence in
-// equal shares (with a fixed segment index per XCD the one holding the last
-// segments, the longest folds, set the end: 54.8 against 48.1 us at 8 x 4096
-// rows, H = 8).  The state pass (STORES) runs over the storing segments' own
-// slots: over the segment pass's a quarter of its workgroups found nothing to
-// do, but had been dealt to CUs like the rest, and some CUs got three that
-// did and some one (37.1 against 29.5 us).
+// heads vary fastest in the segment pass, so every XCD runs every segment index
+// of a sequence in equal shares (with a fixed segment index per XCD the one
+// holding the last segments, the longest folds, set the end: 54.8 against 48.1
+// us at 8 x 4096 rows, H = 8).  The state pass (STORES) runs over the storing
+// segments' own slots: over the segment pass's a quarter of its workgroups
+// found nothing to do, but had been dealt to CUs like the rest, and some CUs
+// got three that did and some one (37.1 against 29.5 us).  It folds nothing
+// and takes segments fastest, which spreads the heads' rows over all XCDs.
 struct SegPlace {
   int n, seg, nseg, h, in;
   int64_t bos, len, first;
@@ -436,9 +437,9 @@ __device__ __forceinline__ bool segment_place(const int64_t *cu, int n_seq, int6
                                               int slots, int even, SegPlace &p) {
   const unsigned t = blockIdx.x >> 3, item = t / inner * 8 + (blockIdx.x & 7);
   p.in = static_cast<int>(t % inner);
-  p.h = static_cast<int>(item % H);
-  const int slot = static_cast<int>(item / H);
-  if (slot >= slots) return false;   // (the grid is rounded up)
+  if (item >= static_cast<unsigned>(slots) * H) return false;   // (the grid is rounded up)
+  int slot = static_cast<int>(STORES ? item % slots : item / H);
+  p.h = static_cast<int>(STORES ? item / slots : item % H);
   const int64_t unit = static_cast<int64_t>(BT) * per;
   int64_t eos;
   if (even) {
@@ -446,8 +447,21 @@ __device__ __forceinline__ bool segment_place(const int64_t *cu, int n_seq, int6
     // one whose slot this would be is, its place is known without a search
     // (a call of 8 x 4096 rows takes 77.5 us so, 79.1 with the search)
     const int own = STORES ? even : even + 1;
-    p.n = static_cast<int>(static_cast<unsigned>(slot) / static_cast<unsigned>(own));
-    p.seg = slot - p.n * own;
+    if (STORES) {
+      // each sequence's last slot is then an empty one: dealt after the others
+      // (as above, 56 of 504: a call 79.1 -> 78.4 us; a reordering of the slots,
+      // whatever the lengths)
+      const unsigned full = even - 1, n_full = n_seq * full * H;
+      const unsigned at = item < n_full ? item / full : item - n_full;
+      p.seg = static_cast<int>(item < n_full ? item % full : full);
+      p.h = static_cast<int>(at % H);
+      p.n = static_cast<int>(at / H);
+      slot = p.n * own + p.seg;
+      if (slot >= slots) return false;   // past the last slot that a segment can own
+    } else {
+      p.n = static_cast<int>(static_cast<unsigned>(slot) / static_cast<unsigned>(own));
+      p.seg = slot - p.n * own;
+    }
     if (p.n < n_seq) {
       p.bos = cu[p.n];
       eos = cu[p.n + 1];
@@ -1072,7 +1086,9 @@ int launch_kg(const FwdArgs &f) {
   const int64_t items = (slots * f.H + 7) / 8 * 8;   // (segment_place deals them in eights)
   const int64_t stores = f.sg.per ? (f.T - 1) / (static_cast<int64_t>(BT) * per) : 0;
   const int64_t unit = static_cast<int64_t>(BT) * per;
-  const int even = f.sg.per && f.T % (f.n_seq * unit) == 0 ? static_cast<int>(f.T / (f.n_seq * unit)) : 0;
+  // (segment_place; 2 and up: an average sequence has more than one segment)
+  const int64_t each = f.sg.per && f.T % (f.n_seq * unit) == 0 ? f.T / (f.n_seq * unit) : 0;
+  const int even = each >= 2 ? static_cast<int>(each) : 0;
   if (items * nvg * KG > 0x7fffffff) {
     set_error("gla_chunk_fwd: too many workgroups");
     return SSLA_ERR_UNSUPPORTED;

@@ -45,6 +45,26 @@ def test_segments(dev, lens, H, K, V, dtype, g16):
     assert_close(ht2, rht, 0.0, "ht, led", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
 
 
+@pytest.mark.parametrize("lens,H,K", [
+    ([256, 256, 100, 412], 2, 64),             # two sequences where equal lengths would put them, two not
+    ([0, 512, 256, 256], 3, 64),
+    ([100, 668, 256], 1, 64),
+    ([256] * 5, 3, 128),
+    ([2048, 1, 2047, 4096], 1, 64),
+    ([384, 384, 1, 767, 384], 9, 48),
+])
+def test_totals_of_equal_lengths(dev, lens, H, K):
+    """Batches whose total is a whole number of segments per sequence, so that
+    workgroups are dealt as for equal lengths, with equal and other lengths."""
+    from ssla_amd.gla import chunk_gla
+    print(f"even totals lens={lens} H={H} K={K}", flush=True)
+    q, k, v, g, cu, s0 = _inputs(lens, H, K, 32, torch.bfloat16, seed=K + H)
+    o, ht = _run(chunk_gla, q, k, v, g, cu, s0, K ** -0.5, dev)
+    ro, rht = _oracle(q, k, v, g, cu, s0, K ** -0.5)
+    assert_close(o, ro, 0.0, "o", band=O_BANDS["logsig"][0], ratio_max=O_BANDS["logsig"][1])
+    assert_close(ht, rht, 0.0, "ht", band=HT_BANDS["logsig"][0], ratio_max=HT_BANDS["logsig"][1])
+
+
 def test_many_ragged_sequences(dev):
     """64 sequences x 8 heads of 1,024 rows on average (one segment each
     fills the GPU), one of them 9,000 rows: every sequence in one walk."""
