@@ -179,7 +179,7 @@ def _chunk_fwd(q, k, v, g, cu, scale, h0, output_final_state):
 def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
     """One ssla_gla_chunk_fwd (K == 64) or ssla_gla_chunk_fwd_wide call (other
     K up to 128), or one ssla_gla_chunk_f32_fwd_ws call for fp32 inputs (K up
-    to 64)."""
+    to 64; ssla_gla_chunk_f32_fwd where its workspace does not fit)."""
     T, H, K = q.shape
     V = v.shape[-1]
     N = cu.numel() - 1
@@ -188,7 +188,14 @@ def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
     lib = _lib.load()
     if q.dtype == torch.float32:
         ws_bytes = lib.ssla_gla_chunk_f32_fwd_workspace_size(N, T, H, K, V)
-        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+        try:
+            ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError:   # no room for the chunks' states: the walk needs none
+            st = lib.ssla_gla_chunk_f32_fwd(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.ptr(cu), N, T, H,
+                                            K, V, float(scale), _lib.ptr(h0), _lib.ptr(o), _lib.ptr(ht),
+                                            _lib.stream_of(q))
+            _lib.check(st, "ssla_gla_chunk_f32_fwd")
+            return o, ht
         st = lib.ssla_gla_chunk_f32_fwd_ws(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(g), _lib.ptr(cu), N, T, H,
                                            K, V, float(scale), _lib.ptr(h0), _lib.ptr(o), _lib.ptr(ht), _lib.ptr(ws),
                                            ws_bytes, _lib.stream_of(q))

@@ -142,3 +142,23 @@ def test_f32_wide_exponents(dev, e):
     assert_close(o.detach().cpu().numpy(), ro, 1e-4, "o")
     for nm, y, r, x in zip(("dq", "dk", "dv", "dg"), leaf, ref, (e, -e, 0, 0)):
         assert_close((y.grad.cpu().double() * 2.0 ** x).numpy(), r, 1e-4, nm)
+
+
+def test_f32_forward_where_the_workspace_does_not_fit(dev, monkeypatch):
+    """chunk_gla on a device without room for the chunks' states (16 KB per
+    64 rows or sequence, and head) takes the entry that needs none."""
+    from ssla_amd.gla import chunk_gla
+    q, k, v, g, cu, h0 = _case([70, 64, 1], 0, 0, 2, 80, 40, 0.3, seed=6)
+    ro, rht = oracle.gla_recurrent(q.numpy(), k.numpy(), v.numpy(), g.numpy(), cu.numpy(), 0.3, h0.numpy(), True)
+    empty = torch.empty
+
+    def full(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*a, **kw)
+    monkeypatch.setattr(torch, "empty", full)
+    with torch.no_grad():
+        o, ht = chunk_gla(*(t.to(dev) for t in (q, k, v, g, cu)), scale=0.3, initial_state=h0.to(dev),
+                          output_final_state=True)
+    assert_close(o.cpu().numpy(), ro, 1e-4, "o")
+    assert_close(ht.cpu().numpy(), rht, 1e-4, "ht")
