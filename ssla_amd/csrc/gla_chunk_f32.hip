@@ -52,10 +52,9 @@ __device__ __forceinline__ void seq_bounds(const int64_t *cu, int n, int64_t T, 
 }
 
 // Per-key references of a chunk (64 threads, one key each, after the
-// cumsum): E[J] = G at row 16 J + 15, S[I] = G at row 16 I, PE[J] =
-// 2^(gamma - E[J]), DL = 2^gamma, GAM = gamma.
+// cumsum): E[J] = G at row 16 J + 15, PE[J] = 2^(gamma - E[J]), DL = 2^gamma.
 struct ChunkRefs {
-  float E[4][64], S[4][64], PE[4][64], DL[64], GAM[64];
+  float E[4][64], PE[4][64], DL[64];
 };
 
 // Chunk-local cumsum of the gates (log2-scaled, in place) and the
@@ -71,21 +70,17 @@ __device__ __forceinline__ void chunk_cumsum(float (*sG)[kP], ChunkRefs &R) {
 #pragma unroll
   for (int I = 0; I < 4; ++I) {
     R.E[I][kk] = sG[16 * I + 15][kk];
-    R.S[I][kk] = sG[16 * I][kk];
     R.PE[I][kk] = ex2c(acc - sG[16 * I + 15][kk]);
   }
   R.DL[kk] = ex2c(acc);
-  R.GAM[kk] = acc;
 }
 
-// k~_j = k_j 2^(E_J - G_j) (into sKt) and, when sQt is given,
-// q~_i = q_i 2^(G_i - S_I) (into sQt).
-__device__ __forceinline__ void chunk_tilde(const float (*sQ)[kP], const float (*sK)[kP], const float (*sG)[kP],
-                                            const ChunkRefs &R, float (*sKt)[kP], float (*sQt)[kP]) {
+// k~_j = k_j 2^(E_J - G_j) (into sKt).
+__device__ __forceinline__ void chunk_tilde(const float (*sK)[kP], const float (*sG)[kP], const ChunkRefs &R,
+                                            float (*sKt)[kP]) {
   for (int e = threadIdx.x; e < kC * 64; e += kThreads) {
     const int r = e >> 6, kk = e & 63, B = r >> 4;
     sKt[r][kk] = sK[r][kk] * ex2c(R.E[B][kk] - sG[r][kk]);
-    if (sQt) sQt[r][kk] = sQ[r][kk] * ex2c(sG[r][kk] - R.S[B][kk]);
   }
 }
 
@@ -159,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void f32_fwd_kernel(
     __syncthreads();
     chunk_cumsum(sG, R);
     __syncthreads();
-    chunk_tilde(sQ, sK, sG, R, sKt, nullptr);
+    chunk_tilde(sK, sG, R, sKt);
     __syncthreads();
     {   // A, thread (row ri, block q4)
       float a[16];
