@@ -201,8 +201,12 @@ def _chunk_call(q, k, v, g, cu, scale, h0, output_final_state):
                                            ws_bytes, _lib.stream_of(q))
         _lib.check(st, "ssla_gla_chunk_f32_fwd_ws")
         return o, ht
-    size, fwd = ((lib.ssla_gla_chunk_workspace_size, lib.ssla_gla_chunk_fwd) if K == KD else
-                 (lib.ssla_gla_chunk_wide_workspace_size, lib.ssla_gla_chunk_fwd_wide))
+    if K == KD:
+        size, fwd = lib.ssla_gla_chunk_workspace_size, lib.ssla_gla_chunk_fwd
+    else:
+        size, fwd = lib.ssla_gla_chunk_wide_workspace_size, lib.ssla_gla_chunk_fwd_wide
+        # (views that start off 16 bytes, which the kernels' wide loads need)
+        q, k, g = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, g))
     ws_bytes = size(N, T, H, K, V)
     ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
     st = fwd(

@@ -108,3 +108,19 @@ def test_full_batches_carry_the_state_in_fp32(dev, dtype):
     _lib.check(lib.ssla_gla_chunk_fwd_noalloc(P(q), P(k), P(v), P(g), _lib.SSLA_F32, P(cu), 3, T, H, 64, V, 64 ** -0.5,
                                               None, P(o2), P(ht2), _lib.DTYPE_CODE[dtype], _lib.stream_of(o2)), "noalloc")
     assert torch.equal(o2, o) and torch.equal(ht2, ht)
+
+
+@pytest.mark.parametrize("K", [16, 32, 48, 80, 128, 144])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_unaligned_views(dev, K, dtype):
+    """q, k and g that start one element off a 16-byte boundary (slices of a
+    flat buffer) give the aligned tensors' bits at key widths other than 64."""
+    from ssla_amd.gla import chunk_gla
+    q, k, v, g, cu, s0 = (t.to(dev) for t in _inputs([130, 7], 1, K, 16, dtype, seed=K))
+    off = lambda t: torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)   # noqa: E731
+    print(f"unaligned K={K} {dtype}", flush=True)
+    with torch.no_grad():
+        for gg in (g, g.to(dtype)):
+            a = chunk_gla(q, k, v, gg, cu, initial_state=s0, output_final_state=True)
+            b = chunk_gla(off(q), off(k), v, off(gg), cu, initial_state=off(s0), output_final_state=True)
+            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
