@@ -158,7 +158,20 @@ def _chunk_fwd(q, k, v, g, cu, scale, h0, output_final_state):
         o = torch.empty_like(v)
         ht = torch.empty(N, H, K, V, device=q.device, dtype=torch.float32) if output_final_state else None
         return _recurrent(q, k, v, g, cu, float(scale), h0, o, ht, None, 0)
-    step = KD if q.dtype == torch.float32 else KF
+    if q.dtype == torch.float32:
+        return _chunk_groups(q, k, v, g, cu, scale, h0, output_final_state, KD)
+    try:
+        return _chunk_groups(q, k, v, g, cu, scale, h0, output_final_state, KF)
+    except NotImplementedError:
+        if K <= KD:
+            raise
+        # a sequence of 2^31 bytes or more at 128 keys: half as many a call
+        return _chunk_groups(q, k, v, g, cu, scale, h0, output_final_state, KD)
+
+
+def _chunk_groups(q, k, v, g, cu, scale, h0, output_final_state, step):
+    """The forward in calls of up to ``step`` keys."""
+    K = q.shape[-1]
     if K <= step:
         return _chunk_call(q, k, v, g, cu, scale, h0, output_final_state)
     # key groups: o adds up over the groups (in fp32, rounded once more for

@@ -124,3 +124,21 @@ def test_unaligned_views(dev, K, dtype):
             a = chunk_gla(q, k, v, gg, cu, initial_state=s0, output_final_state=True)
             b = chunk_gla(off(q), off(k), v, off(gg), cu, initial_state=off(s0), output_final_state=True)
             assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+def test_long_sequence_of_wide_keys(dev):
+    """One sequence past 2^31 bytes of 128 fp32 gates, which 64 keys a call still take."""
+    from ssla_amd.gla import chunk_gla
+    T, K, V = (1 << 22) + 70, 128, 16
+    gen = torch.Generator(device=dev).manual_seed(2)
+    q, k, v = (torch.randn(T, 1, d, generator=gen, device=dev, dtype=torch.bfloat16) for d in (K, K, V))
+    g = torch.randn(T, 1, K, generator=gen, device=dev).abs_().mul_(-0.1)
+    print("long sequence of 128 keys", flush=True)
+    with torch.no_grad():
+        o, ht = chunk_gla(q, k, v, g, torch.tensor([0, T], device=dev), output_final_state=True)
+        t0 = T - 2000   # gates of 0.1 a step on average: the state forgets within a few hundred rows
+        last = [x[t0:].contiguous() for x in (q, k, v, g)]
+        on, hn = chunk_gla(*last, torch.tensor([0, T - t0], device=dev), output_final_state=True)
+    err = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())   # noqa: E731
+    assert err(o[-1000:], on[-1000:]) < 6e-3 and err(ht, hn) < 6e-3   # two bf16 roundings of o, and the state's
+    assert bool(torch.isfinite(o).all())
