@@ -46,7 +46,7 @@ __device__ __forceinline__ bool seq_of_slot(const int64_t *cu, int n_seq, int64_
     first = readlane64(f, from);
   } while (hi - lo > 1);
   n = lo;
-  return true;
+  return first <= slot;   // (always, unless the starts decrease: then no row before the sequence's is touched)
 }
 
 }  // namespace ssla

@@ -162,3 +162,23 @@ def test_f32_forward_where_the_workspace_does_not_fit(dev, monkeypatch):
                           output_final_state=True)
     assert_close(o.cpu().numpy(), ro, 1e-4, "o")
     assert_close(ht.cpu().numpy(), rht, 1e-4, "ht")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_decreasing_offsets_stay_in_bounds(dev, dtype):
+    """cu_seqlens that decrease break the contract, and what the overlapping
+    sequences give is unspecified; but no chunk may start before its
+    sequence (the slot search assumes increasing starts).  A correct call
+    behind it is right."""
+    from ssla_amd.gla import chunk_gla
+    T, H, K = 640, 1, 64
+    q, k, v, g, _cu, _h0 = _case([T], 0, 0, H, K, K, 0.2, seed=17)
+    d = [x.to(dev) for x in (q.to(dtype), k.to(dtype), v.to(dtype), g)]
+    cu = torch.tensor([0, 600] + [2 * i for i in range(150)] + [T], device=dev)
+    print(f"decreasing offsets {dtype}", flush=True)
+    with torch.no_grad():
+        chunk_gla(*d, cu, scale=0.3, output_final_state=True)
+        torch.cuda.synchronize()
+        o, _ = chunk_gla(*d, torch.tensor([0, T], device=dev), scale=0.3)
+    ro, _ = oracle.gla_recurrent(*(x.float().cpu().numpy() for x in d), np.array([0, T]), 0.3)
+    assert_close(o.float().cpu().numpy(), ro, 1e-4 if dtype == torch.float32 else 2e-2, "o")
