@@ -134,9 +134,9 @@ int ssla_gla_chunk_fwd_noalloc(const void *q, const void *k, const void *v,
  * use TF32 operands, here every product is fp32).  q, k, g fp32 [T, H, K],
  * v fp32 [T, H, V], states fp32 [N, H, K, V] (h0 / ht / dht may be NULL),
  * o, dq, dk, dv, dg fp32 in the input layouts; rows outside
- * [cu_seqlens[0], cu_seqlens[n_seq]) are not written.  Chunks of 64 rows,
- * walked in order per (sequence, head): no serial walk over time steps.
- * Forward: K <= 64, V <= 256 per call (wider K: groups of 64 keys whose o
+ * [cu_seqlens[0], cu_seqlens[n_seq]) are not written.  Chunks of 64 rows: no
+ * serial walk over time steps.  An infinity or NaN reaches only the rows whose
+ * sums it enters.  Forward: K <= 64, V <= 256 per call (wider K: groups of 64 keys whose o
  * add up).  Backward: K, V <= 64 per call (wider K or V: groups of 64 keys
  * or value columns, as for the bf16 backward); dh0 is required with h0.
  * ssla_gla_chunk_f32_fwd_ws is the forward with a workspace of
@@ -210,11 +210,6 @@ int ssla_gla_chunk_bwd(const void *q, const void *k, const void *v,
  * walking the whole sequence.  The size query returns 0 for shapes where
  * the single pass is faster (sequences shorter than 64 steps on average)
  * or not available (K not a multiple of 16 up to 64); then pass NULL, 0. */
-/* cu_seqlens[0] and cu_seqlens[n_seq] into host_out[0..1] (pinned host
- * memory) in stream order, then `event` (hipEvent_t) recorded: the rows the
- * sequences cover, known without waiting for work queued after. */
-int ssla_seq_bounds_async(const int64_t *cu_seqlens, int n_seq, int64_t *host_out, void *event, void *stream);
-
 size_t ssla_gla_recurrent_workspace_size(int n_seq, int64_t T, int H, int K, int V);
 int ssla_gla_recurrent_fwd(const void *q, const void *k, const void *v,
                            const void *g, int g_dtype,
@@ -224,6 +219,13 @@ int ssla_gla_recurrent_fwd(const void *q, const void *k, const void *v,
                            const int32_t *state_idx, int n_state_rows,
                            int32_t *status, int dtype, void *workspace,
                            size_t workspace_bytes, void *stream);
+
+/* cu_seqlens[0] and cu_seqlens[n_seq] into host_out[0..1] (pinned host
+ * memory) in stream order, then `event` (hipEvent_t) recorded: the rows the
+ * sequences cover, known without waiting for work queued after.
+ * The memory must stay the caller's until the event has passed, also where a
+ * later call fails. */
+int ssla_seq_bounds_async(const int64_t *cu_seqlens, int n_seq, int64_t *host_out, void *event, void *stream);
 
 /* ------------------------------------------------------------------------
  * G2 -- sparse sequential scans.
@@ -378,20 +380,21 @@ int ssla_scatter_mean(const float *src, const int64_t *index, int64_t E,
 /* Copies the device status word written by the last scatter call that used
  * `workspace` into *status_out (host), synchronising `stream`.  Returns
  * SSLA_OK; *status_out is SSLA_ERR_ARG if any index was out of range. */
+int ssla_scatter_check(const void *workspace, int *status_out, void *stream);
+
 /* ssla_scatter_max / _mean that settle the index's validity first: *host_bad
  * (pinned host memory, set to SSLA_OK by the caller) receives SSLA_ERR_ARG
  * for an index out of [0, n_out) or, with index_sorted, below the one before
  * it, and `event` (hipEvent_t) is recorded on the stream after that and
  * before the reduction, so a caller can wait for the answer while the
- * reduction runs. */
+ * reduction runs.  The word must stay the caller's until the stream has passed
+ * the check, also where the call fails after launching it. */
 int ssla_scatter_max_checked(const float *src, const int64_t *index, int64_t E, int C, int64_t n_out,
                              int index_sorted, float *out, int64_t *argmax, void *workspace,
                              size_t workspace_bytes, int32_t *host_bad, void *event, void *stream);
 int ssla_scatter_mean_checked(const float *src, const int64_t *index, int64_t E, int C, int64_t n_out,
                               int index_sorted, float *out, void *workspace, size_t workspace_bytes,
                               int32_t *host_bad, void *event, void *stream);
-int ssla_scatter_check(const void *workspace, int *status_out, void *stream);
-
 
 /* ------------------------------------------------------------------------
  * G4 -- event-stream glue (grouping, receptive fields / patches, ordered
@@ -475,7 +478,8 @@ int ssla_rf_scatter_fill(const int64_t *gr_len, int64_t G, const int64_t *time, 
  * non-decreasing in time, as group_events and the field outputs leave them,
  * and E_in <= E_cap): the same outputs as ssla_rf_scatter_fill, each row
  * placed by counting the earlier events of the field's other runs.  inv
- * (H * W * A int32) is caller scratch; dst_map (E_in * A int32, may be NULL)
+ * (H * W * A int32) is caller scratch (needed, but not touched for 2 to 16
+ * positions); dst_map (E_in * A int32, may be NULL)
  * receives the row of every (event, kernel position) pair or -1. */
 int ssla_rf_scatter_fill_sorted(const int64_t *gr_batch, const int64_t *gr_h, const int64_t *gr_w,
                                 const int64_t *gr_len, int64_t G, const int64_t *time, int64_t E_in, int B, int H,

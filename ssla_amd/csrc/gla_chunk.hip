@@ -35,8 +35,8 @@
 // past K read zeros), 64 < K <= 128 two groups side by side in a workgroup of
 // 8 wavefronts: the groups are independent GLAs (each key decays its own
 // state row) whose o tiles add up in fp32 through LDS before the one rounding.
-// 21 ragged sequences of 16,411 rows in all at H = 4, K = V = 128: 91 us a call
-// (state pass 23, segment pass 75 us under the profiler), against 288-333 us
+// 21 ragged sequences of 16,411 rows in all at H = 4, K = V = 128: 92-93 us a
+// call (under the profiler: state pass 22 + segment pass 71), against 288-333 us
 // as one call per 64 zero-padded keys, cut into equal counts of segments, with
 // the copies and the sum around them.  What bounds it is the segment pass's
 // chunk loop at two wavefronts per SIMD, as at K = 64.

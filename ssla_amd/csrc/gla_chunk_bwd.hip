@@ -102,7 +102,8 @@ __device__ __forceinline__ void seq_bounds(const int64_t *cu, int n, int64_t T, 
 // 12,000 rows, H = 3: 286 -> 100; fp16, 4,096 rows, H = 4: 141 -> 82).  The fold
 // is serial over a sequence's segments, so where few heads leave it exposed it
 // bounds their number, 128 in a sequence of T rows (24,576 rows, H = 1: 276 ->
-// 123, fp16 193 -> 144).  From 16 chunks on longer segments stay: 8 x 4096 rows
+// 123, fp16 193 -> 144) as long as that takes no more than kSegMax chunks each,
+// up to 131,072 rows.  From 16 chunks on longer segments stay: 8 x 4096 rows
 // at H = 8 took as long in the state passes at 8 and 5 us more in the fold.
 constexpr int kSegMax = 16, kCus = 256, kFoldMax = 128;
 inline int seg_chunks(int64_t T, int H) {

@@ -221,9 +221,9 @@ __global__ __launch_bounds__(kThreads) void f32_fwd_kernel(
 //                       its entering state (and leaving gradient)
 // The walks they replace ran one workgroup per (sequence, head), 48 of them
 // on 256 CUs at 12 ragged sequences of 8,209 rows in all, H = 4, K = V = 64:
-// 14.4 ms for forward and backward against 0.159 ms here (grad 74, states 37
-// in two launches, out 31, prefix 30 us of kernels under the profiler).  What
-// bounds them now is latency: each workgroup's load, cumsum, stage and product
+// 14.4 ms for forward and backward against 0.159 ms here.  (Under the profiler,
+// which drains the device between kernels, grad 73, states 35 and prefix 38 in
+// two launches each, out 32 us: 179 in all.)  What bounds them now is latency: each workgroup's load, cumsum, stage and product
 // phases follow one another with one or two workgroups per CU, and the prefix
 // is a serial chain over the longest sequence's chunks.
 //

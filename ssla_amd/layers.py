@@ -306,7 +306,9 @@ class MosAttention(nn.Module):
         """fused: None picks the fused forward whenever it applies, else the
         training kernels whenever they do; False forces the composed
         (differentiable) path; True requires the fused one (SslaError if it
-        does not apply)."""
+        does not apply).  A second derivative (create_graph=True) through the
+        training kernels raises; the composed path's leaves out what passes
+        through the scan."""
         events = inputs["events"]
         lengths = inputs["lengths"]
         dev = _lib.require_cuda(events, lengths)
