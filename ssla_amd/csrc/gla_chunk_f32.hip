@@ -254,7 +254,8 @@ __global__ __launch_bounds__(kThreads) void f32_fwd_kernel(
 // carry it to rows before its own (after, in dk and dv).
 
 constexpr float kDiagRange = 40.f;
-constexpr uint32_t kInputMin = (127u - 46) << 23, kInputMax = (127u + 47) << 23;   // the bits of 2^-46, 2^47
+constexpr uint32_t kInputMin = (127u - 46) << 23;   // the bits of 2^-46
+constexpr float kInputMax = 0x1p47f;
 
 __device__ __forceinline__ int tix(int r, int c) { return r * 64 + ((((c >> 2) ^ (r & 15)) << 2) | (c & 3)); }
 __device__ __forceinline__ f32x4 row4(const float *t, int r, int c) {
@@ -471,21 +472,20 @@ __global__ __launch_bounds__(256) void f32_prefix_kernel(F32Args a) {
   }
 }
 
-// Largest magnitude, and smallest but zero less one, of the values, as bit
-// patterns (an infinity or NaN is past kHuge).
-constexpr uint32_t kHuge = 0x7f7fffffu;
+// Largest magnitude of the values (NaN if one is), and the smallest but zero
+// as twice its bits less one (a zero gives the largest number).
 struct Magnitudes {
-  uint32_t most = 0, least = 0xffffffffu;
-  template <int RPT>
+  float most = 0.f;
+  uint32_t least = 0xffffffffu;
+  template <int RPT, bool LEAST>
   __device__ __forceinline__ void add(const f32x4 (&x)[RPT]) {
 #pragma unroll
     for (int m = 0; m < RPT; ++m)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float f = x[m][e];   // (a bit cast of the element itself reads element 0)
-        const uint32_t u = __builtin_bit_cast(uint32_t, f) & 0x7fffffffu;
-        most = max(most, u);
-        least = min(least, u - 1);
+        most = __builtin_elementwise_maximum(most, fabsf(f));
+        if (LEAST) least = min(least, (__builtin_bit_cast(uint32_t, f) << 1) - 1);
       }
   }
 };
@@ -496,13 +496,14 @@ struct Magnitudes {
 template <int RPT>
 __device__ __forceinline__ void stage_tilde(const f32x4 (&q)[RPT], const f32x4 (&k)[RPT], const f32x4 (&g)[RPT],
                                             const float (*sS)[64], const float (*sE)[64], int r0, int quad, float *tq,
-                                            float *tk, uint32_t most, int *slow) {
+                                            float *tk, float most, int *slow) {
   const int B = r0 >> 4;
   const f32x4 S = ref4(&sS[B][4 * quad]), E = ref4(&sE[B][4 * quad]);
   Magnitudes qk;
-  qk.add(q);
-  qk.add(k);
-  bool out = (most > kHuge) | (qk.most > kInputMax) | (qk.least < kInputMin - 1);
+  qk.add<RPT, true>(q);
+  qk.add<RPT, true>(k);
+  // (a NaN fails either comparison)
+  bool out = !(most < __builtin_inff()) | !(qk.most <= kInputMax) | (qk.least < 2 * kInputMin - 1);
 #pragma unroll
   for (int m = 0; m < RPT; ++m) {
     f32x4 a, b;
@@ -588,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void f32_out_kernel(F32Args a) {
   }
   if (tid == 0) slow = 0;
   Magnitudes of;
-  of.add(v);
+  of.add<4, false>(v);
   cumsum_rows<4>(g, wtot);
   stage_refs<4>(g, r0, quad, sS, sE);
 #pragma unroll
@@ -721,8 +722,8 @@ __global__ __launch_bounds__(kGradThreads) void f32_grad_kernel(F32Args a) {
     }
     if (tid == 0) L.slow = 0;
     Magnitudes of;
-    of.add(v);
-    of.add(d);
+    of.add<2, false>(v);
+    of.add<2, false>(d);
     cumsum_rows<2>(g, L.wtot);
     stage_refs<2>(g, r0, quad, L.sS, L.sE);
 #pragma unroll
