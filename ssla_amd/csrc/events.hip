@@ -1121,10 +1121,6 @@ __global__ void seg_ends(const int64_t *__restrict__ start, const int64_t *__res
   GRID_STRIDE(i, n) end[i] = start[i] + len[i];
 }
 
-__global__ void store_u64_as_i64(const unsigned long long *__restrict__ src, int64_t *__restrict__ dst) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *dst = static_cast<int64_t>(*src);
-}
-
 // ---------------------------------------------------------------- delays --
 // column 0 of feat [E, C] holds timestamps; replace them by the per-pixel
 // delay (t_i - t_{i-1}) / 1e5 clamped at 1, with 1 for the first event of
@@ -1847,7 +1843,7 @@ struct RfWs {
   int64_t *counts, *gstart, *nev, *act, *act_pre, *ev_pre, *f_index, *f_len, *pre_src, *pre_pos, *pk, *pk_pre;
   int32_t *bad, *pixmap, *val, *perm;
   uint64_t *key, *skey;
-  unsigned long long *tmax;
+  unsigned long long *n_large;   // pieces of large fields, where one list holds them
   // look-back scan states (zeroed by the plan's set-up kernel): the group
   // starts' scan (lb_state_words(G)) and the segment heads' scan of the
   // pooling plan (lb_state_words(E_cap)), contiguous
@@ -1861,7 +1857,7 @@ RfWs rf_layout(void *ws, int64_t G, int64_t n_pix, int64_t n_f, int64_t E_cap) {
   RfWs L;
   L.counts = c.take<int64_t>(8);
   L.bad = c.take<int32_t>(8);
-  L.tmax = c.take<unsigned long long>(1);
+  L.n_large = c.take<unsigned long long>(1);
   L.gstart = c.take<int64_t>(G + 1);
   L.pixmap = c.take<int32_t>(n_pix);
   L.nev = c.take<int64_t>(n_f);
@@ -1929,7 +1925,7 @@ int rf_plan_impl(const int64_t *gr_batch, const int64_t *gr_h, const int64_t *gr
   hipLaunchKernelGGL(clear_and_fill,
                      dim3(grid_for(std::max(std::max(std::max<int64_t>(8, n_pix), std::max(n_inv, n_ev2g)),
                                             L.lb_words))),
-                     dim3(kThreads), 0, st, L.counts, L.bad, reinterpret_cast<int64_t *>(L.tmax), (int64_t)1,
+                     dim3(kThreads), 0, st, L.counts, L.bad, reinterpret_cast<int64_t *>(L.n_large), (int64_t)1,
                      (int64_t)0, L.pixmap, n_pix, -1, inv, n_inv, L.lb_g, L.lb_words, L.val, n_ev2g);
   if (G > 0 || inv)
     hipLaunchKernelGGL(rf_pixmap, dim3(grid_for(std::max(G, inv ? n_rf * A : 0))), dim3(kThreads), 0, st, gr_batch,
@@ -1973,11 +1969,10 @@ int rf_plan_impl(const int64_t *gr_batch, const int64_t *gr_h, const int64_t *gr
   }
   if (E_in > 0 && with_tmax)
     hipLaunchKernelGGL(max_i64, dim3(grid_for(std::min<int64_t>(E_in, 1 << 16))), dim3(kThreads), 0, st, time, E_in,
-                       L.tmax);
+                       reinterpret_cast<unsigned long long *>(L.counts + 2));
   if (!packed)
     hipLaunchKernelGGL(rf_fields, dim3(grid_for(n_f)), dim3(kThreads), 0, st, L.act, L.act_pre, L.nev, n_f, L.f_index,
                        L.f_len);
-  if (with_tmax) hipLaunchKernelGGL(store_u64_as_i64, dim3(1), dim3(64), 0, st, L.tmax, L.counts + 2);
   // the event -> group table and the count of unsorted runs
   if (G > 0 || !store)
     hipLaunchKernelGGL(rf_groups_scan, dim3(grid_for(std::max<int64_t>(std::max(G, E_in), 1))), dim3(kThreads), 0,
@@ -2073,7 +2068,7 @@ extern "C" int ssla_rf_scatter_fill_sorted(const int64_t *gr_batch, const int64_
   const bool fields = A > 1 && A <= 16 && n_f < 0x7fffffff && E_in < (int64_t{1} << 28);
   // (free here, E_cap words each: the sort fill's buffers)
   const int n_lists = E_cap >= 256 ? 4 : 1;
-  uint64_t *counts = n_lists == 4 ? reinterpret_cast<uint64_t *>(L.perm) : reinterpret_cast<uint64_t *>(L.tmax);
+  uint64_t *counts = n_lists == 4 ? reinterpret_cast<uint64_t *>(L.perm) : reinterpret_cast<uint64_t *>(L.n_large);
   const MergeArgs m = {L.f_index, n_act, L.pixmap, L.gstart, gr_len, lut, n_rf, A, n_f, HW, L.ev_pre, time, E_in, E_out,
                        out_src, out_time, out_pos, dst_map,
                        {L.key, L.skey, reinterpret_cast<uint64_t *>(L.pre_src), reinterpret_cast<uint64_t *>(L.pre_pos)},
@@ -2367,8 +2362,7 @@ extern "C" int ssla_sparse_pool_plan_finish(const int64_t *gr_len, int64_t G, co
   int s = SSLA_OK;
   if (c[3] != 0 && E_out > 0) {   // a pixel run not sorted by time: the sort fill
     hipLaunchKernelGGL(max_i64, dim3(grid_for(std::min<int64_t>(E_in, 1 << 16))), dim3(kThreads), 0, st, time, E_in,
-                       L.rf.tmax);
-    hipLaunchKernelGGL(store_u64_as_i64, dim3(1), dim3(64), 0, st, L.rf.tmax, L.rf.counts + 2);
+                       reinterpret_cast<unsigned long long *>(L.rf.counts + 2));
     s = ssla_events_counts(workspace, c, 5, nullptr, stream);
     if (s) return s;
     const int64_t t_max = c[2];
